@@ -894,8 +894,10 @@ static int range_common(hm_tree* t, const uint64_t* start, const uint64_t* hi, c
     dl = b;
   }
   uint64_t* doff = nullptr;
-  if (out_offsets) {
-    doff = ho ? (uint64_t*)take(k8p) : out_offsets;
+  // lengths in mapped host memory are read once, by the scan kernel, not by every range
+  const bool scan = out_offsets && !mapped && n <= kRangeScanMax;
+  if (out_offsets) doff = ho ? (uint64_t*)take(k8p) : out_offsets;
+  if (out_offsets && !scan) {
     void* scan_tmp = take(align256(scan_tmp_bytes(n + 1)));
     HM_TRY(exclusive_scan_u32_to_u64(dl, doff, n, scan_tmp, s));
     HM_TRY(range_offsets_tail(dl, doff, n, s));
@@ -903,7 +905,7 @@ static int range_common(hm_tree* t, const uint64_t* start, const uint64_t* hi, c
   uint64_t* dk = hk ? (uint64_t*)take(cap_bytes) : out_keys;
   uint64_t* dv = hv ? (uint64_t*)take(cap_bytes) : out_vals;
   uint32_t* dc = hc ? (uint32_t*)take(k4) : out_counts;
-  HM_TRY(launch_range(t->view(), ds, dh, dl, cap_const, n, doff, cap_const, dk, dv, dc, capacity, s));
+  HM_TRY(launch_range(t->view(), ds, dh, dl, cap_const, n, doff, scan, cap_const, dk, dv, dc, capacity, s));
   if (ho) HM_TRY(hipMemcpyAsync(out_offsets, doff, (n + 1) * 8, hipMemcpyDeviceToHost, s));
   if (hk) HM_TRY(hipMemcpyAsync(out_keys, dk, capacity * 8, hipMemcpyDeviceToHost, s));
   if (hv) HM_TRY(hipMemcpyAsync(out_vals, dv, capacity * 8, hipMemcpyDeviceToHost, s));
