@@ -965,8 +965,10 @@ struct UpdBufs {
   uint32_t *leaf, *slot;
   uint32_t* nlist;  // nodes to re-spread: (node, first batch entry) pairs
   uint8_t* found;
-  uint32_t* summary;  // [0] overflow, [1] new keys, [2] unique count, [3] validation flags, [4] nodes listed
+  uint32_t* summary;  // [0] overflow, [2] unique count, [4] nodes listed, [6] new keys, [7] plan blocks done
 };
+// Words of hm_tree::upd_host: the plan summary in 0..4, its edge keys as two u64 at 8, the staging flag.
+constexpr int kHostEdge = 8, kHostFlag = 16;
 
 static size_t upd_need(size_t n) {
   const size_t k8 = align256(n * 8), k4 = align256((n + 1) * 4);
@@ -1086,19 +1088,19 @@ int stage_updates(hm_tree* t, const uint64_t* keys, const uint64_t* vals, uint64
   }
   // chain the staging streams, so stage_ev covers every batch staged so far
   if (t->stage_valid) HM_TRY(hipStreamWaitEvent(s, t->stage_ev, 0));
-  HM_TRY(copy_words(t->pend_k + t->pend_n, keys, n, s));
-  HM_TRY(copy_words(t->pend_v + t->pend_n, vals, n, s));
-  HM_TRY(hipEventRecord(t->stage_ev, s));
-  t->stage_valid = true;
-  if (dk) {  // device keys: check on the device (validate_sorted sets bit 0 for KEY_MAX; bit 1 is ignored)
+  uint32_t* flag = nullptr;
+  if (dk) {  // device keys are checked by the staging kernel
     int rc = ensure_upd(t, t->pend_n + n, s);
     if (rc) return rc;
-    UpdBufs b = carve_upd(t->upd_buf, t->pend_n + n);
-    HM_TRY(hipMemsetAsync(b.summary + 3, 0, 4, s));
-    HM_TRY(validate_sorted(t->pend_k + t->pend_n, n, b.summary + 3, s));
-    HM_TRY(copy_u32s(t->upd_host + 3, b.summary + 3, 1, s));
+    flag = t->upd_host + kHostFlag;
+    *flag = 0;  // every kernel that writes it was waited for below
+  }
+  HM_TRY(stage_pairs(keys, vals, t->pend_k + t->pend_n, t->pend_v + t->pend_n, n, flag, s));
+  HM_TRY(hipEventRecord(t->stage_ev, s));
+  t->stage_valid = true;
+  if (dk) {
     HM_TRY(hipStreamSynchronize(s));
-    if (t->upd_host[3] & 1u) return set_err(HM_EINVAL, "key 0xFFFFFFFFFFFFFFFF is reserved for padding");
+    if (*(volatile uint32_t*)flag) return set_err(HM_EINVAL, "key 0xFFFFFFFFFFFFFFFF is reserved for padding");
   }
   t->pend_n += n;
   return HM_OK;
@@ -1141,11 +1143,13 @@ int publish_prepare(hm_tree* t, hipStream_t s, PublishPlan* plan) {
   if (t->stage_valid) HM_TRY(hipStreamWaitEvent(s, t->stage_ev, 0));       // staging on other streams
   const UpdBufs b = carve_upd(t->upd_buf, n);
   uint32_t* dm = b.summary + 2;
-  HM_TRY(hipMemsetAsync(b.summary, 0, 32, s));
-  // sort by key (stable: a later write of a key follows the earlier one), keep the last write
+  const TreeView tv = t->view();
+  // sort by key (stable: a later write of a key follows the earlier one), keep the last write, locate
   if (n <= kSmallUpdate) {
-    HM_TRY(small_sort_dedupe(t->pend_k, t->pend_v, (uint32_t)n, b.uk, b.uv, dm, s));
+    HM_TRY(small_sort_locate(tv, t->pend_k, t->pend_v, (uint32_t)n, b.k0, b.keep, b.uk, b.uv, b.leaf, b.slot, b.found,
+                             b.summary, dm, s));
   } else {
+    HM_TRY(hipMemsetAsync(b.summary, 0, 32, s));
     const uint64_t* sk;
     const uint64_t* sv;
     if (n <= kMergeUpdate) {  // the index ping-pong uses keep / keep_scan before they are needed
@@ -1161,14 +1165,12 @@ int publish_prepare(hm_tree* t, hipStream_t s, PublishPlan* plan) {
     HM_TRY(exclusive_scan_u32(b.keep, b.keep_scan, n, 0u, b.stmp, s));
     HM_TRY(compact_pairs(sk, sv, b.keep, b.keep_scan, n, b.uk, b.uv, s));
     HM_TRY(unique_count(b.keep, b.keep_scan, n, dm, s));
+    HM_TRY(launch_locate(tv, b.uk, n, b.leaf, b.slot, b.found, s, dm));
   }
-  const TreeView tv = t->view();
-  HM_TRY(launch_locate(tv, b.uk, n, b.leaf, b.slot, b.found, s, dm));
-  HM_TRY(plan_runs(t->d_leaves, (uint32_t)t->n_leaves, t->F, b.leaf, b.found, n, dm, b.summary, b.nlist, s));
-  HM_TRY(copy_u32s(t->upd_host, b.summary, 5, s));
-  uint64_t* edge = reinterpret_cast<uint64_t*>(t->upd_host + 8);  // bytes 32..47 of the pinned summary
-  HM_TRY(edge_keys(b.uk, dm, edge, s));
+  HM_TRY(plan_runs(t->d_leaves, (uint32_t)t->n_leaves, t->F, b.leaf, b.slot, b.found, b.uk, n, dm, b.summary, b.nlist,
+                   t->upd_host, s));
   HM_TRY(hipStreamSynchronize(s));
+  const uint64_t* edge = reinterpret_cast<const uint64_t*>(t->upd_host + kHostEdge);
   plan->key_lo = edge[0];
   plan->key_hi = edge[1];
   plan->n_new = t->upd_host[1];

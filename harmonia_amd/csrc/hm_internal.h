@@ -203,11 +203,16 @@ hipError_t compact_pairs(const uint64_t* k, const uint64_t* v, const uint32_t* k
 // Per-leaf insert counts for the not-found keys (keys sorted => leaf ids nondecreasing).
 hipError_t count_inserts(const uint32_t* leaf, const uint8_t* found, size_t n, uint32_t* ins_per_leaf,
                          hipStream_t s);
-// Small batches (n <= kSmallUpdate): one block sorts the staged (key, value) pairs by key in LDS,
-// keeps the last write of each key and writes the m unique pairs to (uk, uv), m to *dm.
+// Copy a batch into the staging arrays; *flag (mapped pinned memory, may be null) = 1 if a key is KEY_MAX.
+hipError_t stage_pairs(const uint64_t* k, const uint64_t* v, uint64_t* dk, uint64_t* dv, size_t n, uint32_t* flag,
+                       hipStream_t s);
+// Small batches (n <= kSmallUpdate): the staged pairs sorted by key (through sk, si), the last write of
+// each key kept in (uk, uv), its count in *dm, and each kept key located as launch_locate does.  Zeroes
+// the 8 words of summary.
 constexpr uint32_t kSmallUpdate = 4096;
-hipError_t small_sort_dedupe(const uint64_t* pk, const uint64_t* pv, uint32_t n, uint64_t* uk, uint64_t* uv,
-                             uint32_t* dm, hipStream_t s);
+hipError_t small_sort_locate(const TreeView& tv, const uint64_t* pk, const uint64_t* pv, uint32_t n, uint64_t* sk,
+                             uint32_t* si, uint64_t* uk, uint64_t* uv, uint32_t* leaf, uint32_t* slot, uint8_t* found,
+                             uint32_t* summary, uint32_t* dm, hipStream_t s);
 // Mid-size batches (kSmallUpdate < n <= kMergeUpdate): stable sort of the staged pairs by key, as a
 // merge sort -- chunks of kSmallUpdate sorted in LDS, then log2(n / kSmallUpdate) merge passes over
 // (key, staging index) in (k0, i0) / (k1, i1), then the values gathered into vout.  *sorted_keys is
@@ -218,15 +223,15 @@ hipError_t merge_sort_pairs(const uint64_t* pk, const uint64_t* pv, uint32_t n, 
 // *dm = keep_scan[n - 1] + keep[n - 1] (unique count after compact_pairs).
 hipError_t unique_count(const uint32_t* keep, const uint32_t* keep_scan, size_t n, uint32_t* dm, hipStream_t s);
 // Over the m located unique keys (sorted, so each leaf's keys form one run and each last-level
-// node's keys one range): summary[1] += number of new keys; summary[0] |= 1 if some leaf would exceed
+// node's keys one range): counts the new keys; summary[0] |= 1 if some leaf would exceed
 // 8 keys.  Such a node goes on the re-spread list (nlist: pairs of node index within the last level and
 // first batch entry; summary[4] = their count) when its leaves can hold all its keys, else
-// summary[0] |= 2 (a full re-layout is needed).  n sizes the grid; nlist holds 2 n entries.
-hipError_t plan_runs(const Leaf* leaves, uint32_t n_leaves, int F, const uint32_t* leaf, const uint8_t* found, size_t n,
-                     const uint32_t* dm, uint32_t* summary, uint32_t* nlist, hipStream_t s);
-// edge[0] = uk[0] and edge[1] = uk[*dm - 1], the smallest and largest of the *dm sorted unique keys
-// (edge = {KEY_MAX, 0} when *dm == 0).  edge may be mapped pinned host memory.
-hipError_t edge_keys(const uint64_t* uk, const uint32_t* dm, uint64_t* edge, hipStream_t s);
+// summary[0] |= 2 (a full re-layout is needed).  n sizes the grid; nlist holds 2 n entries; summary (8
+// words, zeroed) counts new keys in [6] and finished blocks in [7].  host (mapped pinned memory) receives
+// summary[0], the new keys, summary[2..4] and, as two u64 at word 8, the smallest and largest of the *dm sorted unique keys (KEY_MAX, 0 if none).
+hipError_t plan_runs(const Leaf* leaves, uint32_t n_leaves, int F, const uint32_t* leaf, const uint32_t* slot,
+                     const uint8_t* found, const uint64_t* uk, size_t n, const uint32_t* dm, uint32_t* summary,
+                     uint32_t* nlist, uint32_t* host, hipStream_t s);
 // found[j] |= 2 for the batch entries of the listed nodes (the in-place merge then skips them).
 hipError_t mark_nodes(const uint32_t* nlist, uint32_t n_nodes, int F, const uint32_t* leaf, uint8_t* found,
                       const uint32_t* dm, hipStream_t s);

@@ -648,7 +648,8 @@ hipError_t launch_window(const TreeView& tv, const SearchLaunch& sl, const uint6
   return hipGetLastError();
 }
 
-// Locate for the update path: leaf id, lower_bound slot and found flag per key (input order).
+// Locate for the update path: leaf id, lower_bound slot (low byte) with the leaf's free slots (next byte),
+// and found flag per key (input order).
 template <int F, int G>
 __global__ __launch_bounds__(kThreads) void locate_kernel(TreeView tv, const uint64_t* __restrict__ keys, uint32_t n,
                                                           uint32_t* __restrict__ leaf_out,
@@ -672,9 +673,10 @@ __global__ __launch_bounds__(kThreads) void locate_kernel(TreeView tv, const uin
     load_keys<W>(tv.leaves[leaf].key + gl * W, k);
     const int lt = group_count_lt<G, W>(k, t, gbase);
     const bool eq = group_any_eq<G, W>(k, t, gbase) && t != KEY_MAX;
+    const uint32_t room = LEAF_KEYS - (uint32_t)group_count_lt<G, W>(k, KEY_MAX, gbase);
     if (valid && gl == 0) {
       leaf_out[qi] = leaf;
-      slot_out[qi] = (uint32_t)lt;
+      slot_out[qi] = (uint32_t)lt | room << 8;
       found_out[qi] = eq ? 1 : 0;
     }
   }

@@ -9,13 +9,15 @@
 // out (overflowing leaves split evenly into ceil(total / fill) leaves) at offsets given by a device
 // scan, and the caller rebuilds the inner levels and re-scans the prefix array on the device.
 //
-// The common serving case (a few thousand keys, no leaf overflows) stays O(batch): one block sorts
-// and de-duplicates the batch in LDS, the keys are located, each leaf's keys form one run of the
-// sorted batch, and one thread per run plans (overflow? how many new keys?) and then applies it.
+// The common serving case (a few thousand keys, no leaf overflows) stays O(batch) and is bound by its
+// launches: the keys are placed in order by counting, de-duplicated and located in one launch, each
+// leaf's keys form one run of the sorted batch, and one thread per run plans (overflow? how many new
+// keys?) and then applies it.  An epoch of 4001 keys (2^24 stored) with the read of its keys: 115 us in
+// 17 launches, now 60 us in six.
+#include <algorithm>
 #include <utility>
 
-#include "hm_block.h"
-#include "hm_internal.h"
+#include "hm_device.h"
 
 namespace hm {
 namespace {
@@ -199,7 +201,7 @@ __global__ void relayout_touched_kernel(const Leaf* __restrict__ old_leaves, con
     const uint32_t a = ins[L];
     LeafRegs l = load_leaf(old_leaves + L);
     for (size_t j = h; j < m && bleaf[j] == L; ++j)
-      if (found[j]) put(l.val, (int)bslot[j], bv[j]);
+      if (found[j]) put(l.val, (int)(bslot[j] & 255u), bv[j]);
     Leaf* dst = new_leaves + new_start[L];
     uint64_t* dmin = new_mins + new_start[L];
     if (!a) {
@@ -235,33 +237,6 @@ __global__ void relayout_touched_kernel(const Leaf* __restrict__ old_leaves, con
 }
 
 constexpr int kSortThreads = 1024;
-
-// Bitonic network over N (a power of two, <= kSmallUpdate) (key, index) pairs in LDS, ascending by
-// key, then index.  Pair q (elements i, i + j) is handled by thread q % kSortThreads, so every lane
-// has work in every step.  Each step moves every pair through LDS (about 98 KB at N = 4096), and that
-// bounds it: wave-level syncs for the steps whose pairs stay inside one wave measured the same as block
-// barriers.  Ends with a block barrier.
-__device__ __forceinline__ void bitonic_pairs(uint64_t* sk, uint32_t* si, uint32_t N) {
-  for (uint32_t k = 2; k <= N; k <<= 1) {
-    for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-      // pair q: i = q with a zero bit inserted at j's position, partner i + j (every lane busy)
-      for (uint32_t q = threadIdx.x; q < N / 2; q += kSortThreads) {
-        const uint32_t i = ((q & ~(j - 1)) << 1) | (q & (j - 1));
-        const uint32_t p = i + j;
-        const uint64_t a = sk[i], b = sk[p];
-        const uint32_t ia = si[i], ib = si[p];
-        const bool gt = a > b || (a == b && ia > ib);
-        if (gt == ((i & k) == 0)) {
-          sk[i] = b;
-          sk[p] = a;
-          si[i] = ib;
-          si[p] = ia;
-        }
-      }
-      __syncthreads();
-    }
-  }
-}
 
 // LSD radix sort, in LDS, of kSmallUpdate (key, index) pairs held in (sk[0], si[0]), over the 8 key
 // bytes; stable, so equal keys keep their index order.  8 passes that each move the pairs through LDS
@@ -389,55 +364,91 @@ __global__ void gather_by_index_kernel(const uint64_t* __restrict__ v, const uin
   if (i < n) out[i] = v[ix[i]];
 }
 
-// Sort of (key, staging index) in LDS, stable in the index, so the last write of a key ends its run
-// of equal keys; then the last of each run is kept.  Padding (KEY_MAX, ~0) sorts after every real key
-// (KEY_MAX is never staged).
-__global__ __launch_bounds__(kSortThreads) void small_sort_dedupe_kernel(const uint64_t* __restrict__ pk,
-                                                                         const uint64_t* __restrict__ pv, uint32_t n,
-                                                                         uint64_t* __restrict__ uk,
-                                                                         uint64_t* __restrict__ uv,
-                                                                         uint32_t* __restrict__ dm) {
-  __shared__ RadixLds L;
-  __shared__ uint32_t scan_sh[kSortThreads / 64 + 1];
-  // up to 1024 keys: the bitonic network over the next power of two; above: the radix sort (8 passes
-  // over all kSmallUpdate slots, padding included), which is cheaper there
-  const bool radix = n > 1024;
-  uint32_t N = 1;
-  while (N < n) N <<= 1;
-  if (radix) N = kSmallUpdate;
-  for (uint32_t i = threadIdx.x; i < N; i += kSortThreads) {
-    L.sk[0][i] = i < n ? pk[i] : KEY_MAX;
-    L.si[0][i] = i < n ? i : 0xFFFFFFFFu;
+// Small batches (n <= kSmallUpdate), first kernel: every staged key's place in the order by (key, staging
+// index), counted against all n keys held in LDS.  A block places 16 keys, 32 slices of the batch each, so
+// 4096 keys take 256 blocks and 128 steps of two compares per thread.  One block sorting 4096 keys (LSD
+// radix in LDS, eight passes) took 37.6 us on one CU with the others idle.
+constexpr int kRankThreads = 512;
+constexpr int kRankKeys = 16;
+constexpr int kRankSlices = kRankThreads / kRankKeys;
+__global__ __launch_bounds__(kRankThreads) void rank_keys_kernel(const uint64_t* __restrict__ pk, uint32_t n,
+                                                                 uint64_t* __restrict__ sk, uint32_t* __restrict__ si,
+                                                                 uint32_t* __restrict__ summary) {
+  __shared__ ulonglong2 lk[kSmallUpdate / 2];
+  __shared__ uint32_t place[kRankKeys];
+  if (blockIdx.x == 0 && threadIdx.x < 8) summary[threadIdx.x] = 0;
+  if (threadIdx.x < kRankKeys) place[threadIdx.x] = 0;
+  const uint32_t pairs = (n + 1) / 2;
+  for (uint32_t p = threadIdx.x; p < pairs; p += kRankThreads)
+    lk[p] = make_ulonglong2(pk[2 * p], 2 * p + 1 < n ? pk[2 * p + 1] : KEY_MAX);
+  __syncthreads();
+  const uint32_t ki = blockIdx.x * kRankKeys + threadIdx.x % kRankKeys;
+  // staged keys are below KEY_MAX, so an earlier equal key counts as smaller through key + 1
+  const uint64_t key = ki < n ? pk[ki] : 0ull;
+  uint32_t c = 0;
+#pragma unroll 8
+  for (uint32_t p = threadIdx.x / kRankKeys; p < pairs; p += kRankSlices) {
+    const ulonglong2 v = lk[p];
+    c += v.x < key + (2 * p < ki ? 1u : 0u) ? 1u : 0u;
+    c += v.y < key + (2 * p + 1 < ki ? 1u : 0u) ? 1u : 0u;
   }
-  int cur = 0;
-  if (radix) {  // block-uniform
-    cur = radix_sort_lds(L);
-  } else {
-    __syncthreads();
-    bitonic_pairs(L.sk[0], L.si[0], N);
+  c += __shfl_xor(c, 16);
+  c += __shfl_xor(c, 32);
+  if ((threadIdx.x & 63) < kRankKeys) atomicAdd(&place[threadIdx.x % kRankKeys], c);
+  __syncthreads();
+  if (threadIdx.x < kRankKeys && ki < n) {
+    sk[place[threadIdx.x]] = key;
+    si[place[threadIdx.x]] = ki;
   }
-  const uint64_t* sk = L.sk[cur];
-  const uint32_t* si = L.si[cur];
-  constexpr int kPer = kSmallUpdate / kSortThreads;  // consecutive elements per thread
-  const uint32_t b0 = threadIdx.x * kPer;
-  bool keep[kPer];
-  uint32_t cnt = 0;
+}
+
+// Number of keys of a leaf's 8 (one per lane of an 8-lane group): its free slots.
+__device__ __forceinline__ uint32_t group_room(uint64_t k, int gbase) {
+  return (uint32_t)LEAF_KEYS - (uint32_t)__popcll((__ballot(k != KEY_MAX) >> gbase) & 0xFFull);
+}
+
+// Second kernel: the last write of each key kept (32 sorted entries per block, which counts the kept
+// entries before its own: at most 32 KiB of keys, all in L2), and located, 8 lanes per key.
+template <int F>
+__global__ __launch_bounds__(256) void dedupe_locate_kernel(TreeView tv, const uint64_t* __restrict__ sk,
+                                                            const uint32_t* __restrict__ si,
+                                                            const uint64_t* __restrict__ pv, uint32_t n,
+                                                            uint64_t* __restrict__ uk, uint64_t* __restrict__ uv,
+                                                            uint32_t* __restrict__ leaf_out,
+                                                            uint32_t* __restrict__ slot_out,
+                                                            uint8_t* __restrict__ found_out, uint32_t* __restrict__ dm) {
+  constexpr uint32_t kPer = 32;
+  __shared__ uint32_t before_w[4];
+  __shared__ uint32_t kept_s[kPer];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const uint32_t base = blockIdx.x * kPer;
+  uint32_t c = 0;
+  for (uint32_t p = threadIdx.x; p < base; p += 256) c += sk[p] != sk[p + 1] ? 1u : 0u;  // base < n
 #pragma unroll
-  for (int r = 0; r < kPer; ++r) {
-    const uint32_t i = b0 + r;
-    keep[r] = i < n && (i + 1 == n || sk[i] != sk[i + 1]);
-    cnt += keep[r] ? 1u : 0u;
+  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+  if (lane == 0) before_w[w] = c;
+  const int gl = lane & 7, gbase = lane - gl;
+  const uint32_t g = threadIdx.x / 8, p = base + g;
+  const uint64_t t = p < n ? sk[p] : 0ull;
+  const bool kept = p < n && (p + 1 == n || sk[p + 1] != t);
+  if (gl == 0) kept_s[g] = kept ? 1u : 0u;
+  const uint32_t leaf = descend<F, 8>(tv, 0, nullptr, t, gl, gbase);
+  const uint64_t k[1] = {tv.leaves[leaf].key[gl]};
+  const int lt = group_count_lt<8, 1>(k, t, gbase);
+  const bool eq = group_any_eq<8, 1>(k, t, gbase);
+  const uint32_t room = group_room(k[0], gbase);
+  __syncthreads();
+  const uint32_t before = before_w[0] + before_w[1] + before_w[2] + before_w[3];
+  const uint32_t km = (uint32_t)__ballot(lane < (int)kPer && kept_s[lane & (kPer - 1)] != 0u);
+  if (kept && gl == 0) {
+    const uint32_t o = before + (uint32_t)__popc(km & ((1u << g) - 1u));
+    uk[o] = t;
+    uv[o] = pv[si[p]];
+    leaf_out[o] = leaf;
+    slot_out[o] = (uint32_t)lt | room << 8;
+    found_out[o] = eq ? 1 : 0;
   }
-  uint32_t total = 0;
-  uint32_t off = block_exclusive_scan<uint32_t, kSortThreads>(cnt, scan_sh, total);
-#pragma unroll
-  for (int r = 0; r < kPer; ++r)
-    if (keep[r]) {
-      uk[off] = sk[b0 + r];
-      uv[off] = pv[si[b0 + r]];
-      ++off;
-    }
-  if (threadIdx.x == 0) *dm = total;
+  if (threadIdx.x == 0 && base + kPer >= n) *dm = before + (uint32_t)__popc(km);
 }
 
 __global__ void unique_count_kernel(const uint32_t* __restrict__ keep, const uint32_t* __restrict__ scan, size_t n,
@@ -449,18 +460,25 @@ __device__ __forceinline__ bool run_head(const uint32_t* __restrict__ leaf, uint
   return i == 0 || leaf[i] != leaf[i - 1];
 }
 
-// Plan an epoch, one thread per last-level node the batch touches (its first batch entry: the batch
-// is sorted, so a node's entries are contiguous).  Last-level node j holds leaves
+// Plan an epoch, one thread per leaf the batch touches (its first batch entry: the batch is sorted, so a
+// leaf's and a node's entries are contiguous).  Last-level node j holds leaves
 // [j F, min((j + 1) F, n_leaves)): the bulk build and re-layouts fill every node but the last, and
 // an in-node re-spread keeps each node's leaf count.  summary[1] += new keys; if a leaf of the node
 // would overflow, summary[0] |= 1 and the node either goes on the re-spread list (nlist: node, first
 // batch entry; count in summary[4]) when its leaves can hold all its keys, or summary[0] |= 2 (the
 // epoch needs a full re-layout).
+// The locate step left each entry's leaf's free slots beside its slot, so the plan reads leaves only for
+// nodes that overflow, and a thread walks one leaf's entries, not a node's: 2^20 entries took 61 us with
+// one thread per node reading its leaves, now 22.  The block that
+// finishes last writes the summary and the smallest and largest key to `host` (mapped pinned memory:
+// words 0..4 and the two u64 at word 8), in place of two more launches.
 __global__ void plan_runs_kernel(const Leaf* __restrict__ leaves, uint32_t n_leaves, int F,
-                                 const uint32_t* __restrict__ leaf, const uint8_t* __restrict__ found, size_t n_max,
+                                 const uint32_t* __restrict__ leaf, const uint32_t* __restrict__ slot,
+                                 const uint8_t* __restrict__ found, const uint64_t* __restrict__ uk, size_t n_max,
                                  const uint32_t* __restrict__ dm, uint32_t* __restrict__ summary,
-                                 uint32_t* __restrict__ nlist) {
+                                 uint32_t* __restrict__ nlist, uint32_t* __restrict__ host) {
   __shared__ uint32_t block_new;
+  __shared__ bool last_block;
   if (threadIdx.x == 0) block_new = 0;
   __syncthreads();
   const uint32_t m = dm ? *dm : (uint32_t)n_max;
@@ -468,20 +486,26 @@ __global__ void plan_runs_kernel(const Leaf* __restrict__ leaves, uint32_t n_lea
   const uint32_t uF = (uint32_t)F;
   uint32_t my_new = 0;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += stride) {
+    const uint32_t L = leaf[i];
     my_new += found[i] ? 0u : 1u;
-    const uint32_t node = leaf[i] / uF;
-    if (i > 0 && leaf[i - 1] / uF == node) continue;  // not the node's first entry
-    bool over = false;
+    if (i > 0 && leaf[i - 1] == L) continue;  // not the leaf's first entry
+    uint32_t ins = 0;
+    for (uint32_t j = i; j < m && leaf[j] == L; ++j) ins += found[j] ? 0u : 1u;
+    if (ins <= slot[i] >> 8) continue;
+    // the leaf overflows: the first such leaf of a node plans the node, from its first entry i0 on
+    const uint32_t node = L / uF;
+    uint32_t i0 = i;
+    while (i0 > 0 && leaf[i0 - 1] / uF == node) --i0;
     uint32_t node_ins = 0;
-    for (uint32_t j = i; j < m && leaf[j] / uF == node;) {
-      const uint32_t L = leaf[j];
-      const uint32_t room = (uint32_t)(LEAF_KEYS - leaf_count(leaves[L]));
-      uint32_t ins = 0;
-      for (; j < m && leaf[j] == L; ++j) ins += found[j] ? 0u : 1u;
-      over |= ins > room;
-      node_ins += ins;
+    bool first = true;
+    for (uint32_t j = i0; first && j < m && leaf[j] / uF == node;) {
+      const uint32_t x = leaf[j], room = slot[j] >> 8;
+      uint32_t c = 0;
+      for (; j < m && leaf[j] == x; ++j) c += found[j] ? 0u : 1u;
+      first = c <= room || x >= L;
+      node_ins += c;
     }
-    if (!over) continue;
+    if (!first) continue;
     atomicOr(&summary[0], 1u);
     const uint32_t x0 = node * uF, x1 = x0 + uF < n_leaves ? x0 + uF : n_leaves;
     uint32_t total = node_ins;
@@ -489,18 +513,35 @@ __global__ void plan_runs_kernel(const Leaf* __restrict__ leaves, uint32_t n_lea
     if (total <= (x1 - x0) * (uint32_t)LEAF_KEYS) {
       const uint32_t k = atomicAdd(&summary[4], 1u);
       nlist[2 * k] = node;
-      nlist[2 * k + 1] = i;
+      nlist[2 * k + 1] = i0;
     } else {
       atomicOr(&summary[0], 2u);
     }
   }
-  // new-key count: wave sum, then one LDS atomic per wave and one global atomic per block (a
-  // global atomic per wave on one address serializes)
+  // new-key count: wave sum, then one LDS atomic per wave and one global atomic per block
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) my_new += __shfl_xor(my_new, o);
   if ((threadIdx.x & 63) == 0 && my_new) atomicAdd(&block_new, my_new);
+  __syncthreads();  // waits for every thread's summary atomics, so they come before the block's count
+  if (threadIdx.x == 0) {
+    // new keys in the low word, finished blocks in the high one: one atomic per block.  (A device-scope
+    // fence instead of the barrier above would write the L2 back, in every block: 0.25 ms for 2^20 entries.)
+    const uint64_t mine = (1ull << 32) | block_new;
+    const uint64_t old = atomicAdd(reinterpret_cast<unsigned long long*>(summary + 6), (unsigned long long)mine);
+    last_block = (uint32_t)(old >> 32) == gridDim.x - 1;
+    block_new += (uint32_t)old;  // in the last block: every new key
+  }
   __syncthreads();
-  if (threadIdx.x == 0 && block_new) atomicAdd(&summary[1], block_new);
+  if (!last_block) return;  // every block's atomics are done
+  if (threadIdx.x < 5)
+    host[threadIdx.x] = threadIdx.x == 1 ? block_new
+                                         : __hip_atomic_load(&summary[threadIdx.x], __ATOMIC_RELAXED,
+                                                             __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 64) {
+    uint64_t* edge = reinterpret_cast<uint64_t*>(host + 8);
+    edge[0] = m ? uk[0] : KEY_MAX;
+    edge[1] = m ? uk[m - 1] : 0ull;
+  }
 }
 
 // Mark the batch entries of the listed nodes (found |= 2) so the in-place merge leaves them to the
@@ -573,7 +614,7 @@ __global__ __launch_bounds__(64) void node_respread_kernel(Leaf* __restrict__ le
       const uint32_t j = j0 + lane;
       const bool in = j < m && leaf[j] / (uint32_t)F == node;
       const uint8_t f = in ? (found[j] & 1u) : 0u;
-      if (in && f) ev[off[leaf[j] - x0] + slot[j]] = uv[j];
+      if (in && f) ev[off[leaf[j] - x0] + (slot[j] & 255u)] = uv[j];
       const uint32_t isnew = in && !f ? 1u : 0u;
       const uint32_t inc = wave_inclusive_scan(isnew);
       if (isnew) {
@@ -640,7 +681,7 @@ __global__ void apply_runs_kernel(Leaf* __restrict__ leaves, const uint32_t* __r
     uint32_t ins = 0;
     for (uint32_t j = i; j < m && leaf[j] == L; ++j) {
       if (found[j])
-        leaves[L].val[slot[j]] = uv[j];
+        leaves[L].val[slot[j] & 255u] = uv[j];
       else
         ++ins;
     }
@@ -661,27 +702,71 @@ __global__ void apply_runs_kernel(Leaf* __restrict__ leaves, const uint32_t* __r
   }
 }
 
-__global__ void edge_keys_kernel(const uint64_t* __restrict__ uk, const uint32_t* __restrict__ dm,
-                                 uint64_t* __restrict__ edge) {
-  if (threadIdx.x == 0) {
-    const uint32_t m = *dm;
-    edge[0] = m ? uk[0] : KEY_MAX;
-    edge[1] = m ? uk[m - 1] : 0ull;
+// Staging of an upsert batch: keys and values copied, and *flag (mapped pinned memory, may be null) set
+// if a key is the reserved one.  One launch and no reduction: the flag is only ever written by a bad key.
+// (Two copies, a memset, a validation that ended in 4096 atomics on one word and a copy of that word
+// took 70 us for 2^20 pairs, 48 of them in the validation.)
+constexpr int kStageUnroll = 4;
+__global__ __launch_bounds__(256) void stage_pairs_kernel(const uint64_t* __restrict__ k, const uint64_t* __restrict__ v,
+                                                          uint64_t* __restrict__ dk, uint64_t* __restrict__ dv,
+                                                          size_t n, uint32_t* __restrict__ flag) {
+  const size_t stride = (size_t)gridDim.x * 256;
+  bool bad = false;
+  for (size_t b = (size_t)blockIdx.x * 256 + threadIdx.x; b < n; b += kStageUnroll * stride) {
+    uint64_t x[kStageUnroll], y[kStageUnroll];
+#pragma unroll
+    for (int u = 0; u < kStageUnroll; ++u) {
+      const size_t i = b + u * stride;
+      x[u] = i < n ? k[i] : 0ull;
+      y[u] = i < n ? v[i] : 0ull;
+    }
+#pragma unroll
+    for (int u = 0; u < kStageUnroll; ++u) {
+      const size_t i = b + u * stride;
+      if (i < n) {
+        dk[i] = x[u];
+        dv[i] = y[u];
+        bad |= x[u] == KEY_MAX;
+      }
+    }
   }
+  if (bad && flag) *flag = 1u;
 }
 
 }  // namespace
 
-hipError_t edge_keys(const uint64_t* uk, const uint32_t* dm, uint64_t* edge, hipStream_t s) {
-  hipLaunchKernelGGL(edge_keys_kernel, dim3(1), dim3(64), 0, s, uk, dm, edge);
+hipError_t stage_pairs(const uint64_t* k, const uint64_t* v, uint64_t* dk, uint64_t* dv, size_t n, uint32_t* flag,
+                       hipStream_t s) {
+  if (!n) return hipSuccess;
+  ProfScope prof("update", s);
+  size_t nb = (n + 256 * kStageUnroll - 1) / (256 * kStageUnroll);
+  if (nb > 2048) nb = 2048;
+  hipLaunchKernelGGL(stage_pairs_kernel, dim3((unsigned)nb), dim3(256), 0, s, k, v, dk, dv, n, flag);
   return hipGetLastError();
 }
 
-hipError_t small_sort_dedupe(const uint64_t* pk, const uint64_t* pv, uint32_t n, uint64_t* uk, uint64_t* uv,
-                             uint32_t* dm, hipStream_t s) {
+hipError_t small_sort_locate(const TreeView& tv, const uint64_t* pk, const uint64_t* pv, uint32_t n, uint64_t* sk,
+                             uint32_t* si, uint64_t* uk, uint64_t* uv, uint32_t* leaf, uint32_t* slot, uint8_t* found,
+                             uint32_t* summary, uint32_t* dm, hipStream_t s) {
   if (n == 0 || n > kSmallUpdate) return hipErrorInvalidValue;
   ProfScope prof("update", s);
-  hipLaunchKernelGGL(small_sort_dedupe_kernel, dim3(1), dim3(kSortThreads), 0, s, pk, pv, n, uk, uv, dm);
+  hipLaunchKernelGGL(rank_keys_kernel, dim3((n + kRankKeys - 1) / kRankKeys), dim3(kRankThreads), 0, s, pk, n, sk, si,
+                     summary);
+  const dim3 grid((n + 31) / 32);
+  switch (tv.fanout) {
+    case 32:
+      hipLaunchKernelGGL(dedupe_locate_kernel<32>, grid, dim3(256), 0, s, tv, sk, si, pv, n, uk, uv, leaf, slot, found, dm);
+      break;
+    case 64:
+      hipLaunchKernelGGL(dedupe_locate_kernel<64>, grid, dim3(256), 0, s, tv, sk, si, pv, n, uk, uv, leaf, slot, found, dm);
+      break;
+    case 128:
+      hipLaunchKernelGGL(dedupe_locate_kernel<128>, grid, dim3(256), 0, s, tv, sk, si, pv, n, uk, uv, leaf, slot, found,
+                         dm);
+      break;
+    default:
+      return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 
@@ -710,12 +795,14 @@ hipError_t unique_count(const uint32_t* keep, const uint32_t* keep_scan, size_t 
   return hipGetLastError();
 }
 
-hipError_t plan_runs(const Leaf* leaves, uint32_t n_leaves, int F, const uint32_t* leaf, const uint8_t* found, size_t n,
-                     const uint32_t* dm, uint32_t* summary, uint32_t* nlist, hipStream_t s) {
+hipError_t plan_runs(const Leaf* leaves, uint32_t n_leaves, int F, const uint32_t* leaf, const uint32_t* slot,
+                     const uint8_t* found, const uint64_t* uk, size_t n, const uint32_t* dm, uint32_t* summary,
+                     uint32_t* nlist, uint32_t* host, hipStream_t s) {
   if (!n) return hipSuccess;
   ProfScope prof("update", s);
-  hipLaunchKernelGGL(plan_runs_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, leaves, n_leaves, F, leaf, found, n,
-                     dm, summary, nlist);
+  // at most 1024 blocks: each ends in an atomic on one word (~10 ns, one after the other)
+  hipLaunchKernelGGL(plan_runs_kernel, dim3(std::min(grid_for(n, 256), 1024)), dim3(256), 0, s, leaves, n_leaves, F, leaf, slot,
+                     found, uk, n, dm, summary, nlist, host);
   return hipGetLastError();
 }
 
