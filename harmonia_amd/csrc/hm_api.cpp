@@ -960,8 +960,8 @@ struct UpdBufs {
   uint64_t *uk, *uv;          // sorted unique batch
   uint64_t *k0, *v0, *k1, *v1;  // radix ping-pong (large batches)
   void* rtmp;
-  uint32_t *keep, *keep_scan;
-  void* stmp;
+  uint32_t *i0, *i1;            // staging indices of the merge sort
+  void* stmp;                   // kept keys per tile (dedupe_tmp_bytes)
   uint32_t *leaf, *slot;
   uint32_t* nlist;  // nodes to re-spread: (node, first batch entry) pairs
   uint8_t* found;
@@ -988,8 +988,8 @@ static UpdBufs carve_upd(void* base, size_t n) {
   b.k1 = (uint64_t*)cur, cur += k8;
   b.v1 = (uint64_t*)cur, cur += k8;
   b.rtmp = cur, cur += align256(radix_tmp_bytes(n));
-  b.keep = (uint32_t*)cur, cur += k4;
-  b.keep_scan = (uint32_t*)cur, cur += k4;
+  b.i0 = (uint32_t*)cur, cur += k4;
+  b.i1 = (uint32_t*)cur, cur += k4;
   b.stmp = cur, cur += align256(scan_tmp_bytes(n + 1));
   b.leaf = (uint32_t*)cur, cur += k4;
   b.slot = (uint32_t*)cur, cur += k4;
@@ -1146,25 +1146,25 @@ int publish_prepare(hm_tree* t, hipStream_t s, PublishPlan* plan) {
   const TreeView tv = t->view();
   // sort by key (stable: a later write of a key follows the earlier one), keep the last write, locate
   if (n <= kSmallUpdate) {
-    HM_TRY(small_sort_locate(tv, t->pend_k, t->pend_v, (uint32_t)n, b.k0, b.keep, b.uk, b.uv, b.leaf, b.slot, b.found,
+    HM_TRY(small_sort_locate(tv, t->pend_k, t->pend_v, (uint32_t)n, b.k0, b.i0, b.uk, b.uv, b.leaf, b.slot, b.found,
                              b.summary, dm, s));
   } else {
-    HM_TRY(hipMemsetAsync(b.summary, 0, 32, s));
     const uint64_t* sk;
-    const uint64_t* sv;
-    if (n <= kMergeUpdate) {  // the index ping-pong uses keep / keep_scan before they are needed
-      HM_TRY(merge_sort_pairs(t->pend_k, t->pend_v, (uint32_t)n, b.k0, b.k1, b.keep, b.keep_scan, b.v0, s, &sk));
-      sv = b.v0;
+    const uint64_t* sv = t->pend_v;
+    const uint32_t* si = nullptr;
+    uint32_t* tile_kept = (uint32_t*)b.stmp;
+    if (n <= kMergeUpdate) {
+      HM_TRY(merge_sort_index(t->pend_k, (uint32_t)n, b.k0, b.k1, b.i0, b.i1, tile_kept, b.summary, s, &sk,
+                              &si));
     } else {
+      HM_TRY(hipMemsetAsync(b.summary, 0, 32, s));
       int which = 0;
       HM_TRY(radix_sort_u64pay(t->pend_k, t->pend_v, n, 0, 64, b.k0, b.v0, b.k1, b.v1, b.rtmp, s, &which));
       sk = which ? b.k1 : b.k0;
       sv = which ? b.v1 : b.v0;
+      HM_TRY(count_kept(sk, n, tile_kept, s));
     }
-    HM_TRY(mark_last_of_runs(sk, n, b.keep, s));
-    HM_TRY(exclusive_scan_u32(b.keep, b.keep_scan, n, 0u, b.stmp, s));
-    HM_TRY(compact_pairs(sk, sv, b.keep, b.keep_scan, n, b.uk, b.uv, s));
-    HM_TRY(unique_count(b.keep, b.keep_scan, n, dm, s));
+    HM_TRY(compact_last(sk, si, sv, n, tile_kept, b.uk, b.uv, dm, s));
     HM_TRY(launch_locate(tv, b.uk, n, b.leaf, b.slot, b.found, s, dm));
   }
   HM_TRY(plan_runs(t->d_leaves, (uint32_t)t->n_leaves, t->F, b.leaf, b.slot, b.found, b.uk, n, dm, b.summary, b.nlist,

@@ -181,8 +181,8 @@ hipError_t copy_u32s(uint32_t* dst, const uint32_t* src, size_t n, hipStream_t s
 hipError_t build_child_array(const uint32_t* prefix, uint32_t n_inner, int F, uint32_t* child, hipStream_t s);
 hipError_t launch_search_baseline(const TreeView& tv, const uint32_t* child, const uint64_t* q, uint64_t* out_vals,
                                   uint8_t* out_found, uint32_t n, int group, int kind, hipStream_t s);
-// Locate (leaf, slot, found) per key (update path); n sizes the grid, dn (device) may hold the
-// actual count.
+// Locate (update path): leaf, lower_bound slot (low byte) with the leaf's free slots (next byte)
+// and found flag per key; n sizes the grid, dn (device) may hold the actual count.
 hipError_t launch_locate(const TreeView& tv, const uint64_t* keys, size_t n, uint32_t* leaf_out, uint32_t* slot_out,
                          uint8_t* found_out, hipStream_t s, const uint32_t* dn = nullptr);
 
@@ -196,10 +196,6 @@ hipError_t launch_range(const TreeView& tv, const uint64_t* start, const uint64_
                         uint64_t* out_keys, uint64_t* out_vals, uint32_t* out_counts, uint64_t capacity, hipStream_t s);
 
 // ---- update (hm_update.hip) ------------------------------------------------------------
-// Marks run ends of a sorted key array (keep the last of equal keys): keep[i] = 1 if last.
-hipError_t mark_last_of_runs(const uint64_t* sorted_keys, size_t n, uint32_t* keep, hipStream_t s);
-hipError_t compact_pairs(const uint64_t* k, const uint64_t* v, const uint32_t* keep, const uint32_t* keep_scan,
-                         size_t n, uint64_t* ko, uint64_t* vo, hipStream_t s);
 // Per-leaf insert counts for the not-found keys (keys sorted => leaf ids nondecreasing).
 hipError_t count_inserts(const uint32_t* leaf, const uint8_t* found, size_t n, uint32_t* ins_per_leaf,
                          hipStream_t s);
@@ -213,15 +209,21 @@ constexpr uint32_t kSmallUpdate = 4096;
 hipError_t small_sort_locate(const TreeView& tv, const uint64_t* pk, const uint64_t* pv, uint32_t n, uint64_t* sk,
                              uint32_t* si, uint64_t* uk, uint64_t* uv, uint32_t* leaf, uint32_t* slot, uint8_t* found,
                              uint32_t* summary, uint32_t* dm, hipStream_t s);
-// Mid-size batches (kSmallUpdate < n <= kMergeUpdate): stable sort of the staged pairs by key, as a
-// merge sort -- chunks of kSmallUpdate sorted in LDS, then log2(n / kSmallUpdate) merge passes over
-// (key, staging index) in (k0, i0) / (k1, i1), then the values gathered into vout.  *sorted_keys is
-// k0 or k1.  1 + log2(n / 4096) + 1 launches in place of the radix sort's 24.
+// Mid-size batches (kSmallUpdate < n <= kMergeUpdate, hm_merge.hip): the staged keys sorted with their
+// staging indices, stable, through (k0, i0) and (k1, i1), as a merge sort: chunks of kSmallUpdate in LDS,
+// then a pass per doubling.  tile_kept (dedupe_tmp_bytes) receives what compact_last needs; the 8 words of
+// summary are zeroed.
 constexpr uint32_t kMergeUpdate = 1u << 22;
-hipError_t merge_sort_pairs(const uint64_t* pk, const uint64_t* pv, uint32_t n, uint64_t* k0, uint64_t* k1,
-                            uint32_t* i0, uint32_t* i1, uint64_t* vout, hipStream_t s, const uint64_t** sorted_keys);
-// *dm = keep_scan[n - 1] + keep[n - 1] (unique count after compact_pairs).
-hipError_t unique_count(const uint32_t* keep, const uint32_t* keep_scan, size_t n, uint32_t* dm, hipStream_t s);
+size_t dedupe_tmp_bytes(size_t n);
+hipError_t merge_sort_index(const uint64_t* pk, uint32_t n, uint64_t* k0, uint64_t* k1, uint32_t* i0, uint32_t* i1,
+                            uint32_t* tile_kept, uint32_t* summary, hipStream_t s, const uint64_t** sorted_keys,
+                            const uint32_t** sorted_index);
+// tile_kept for keys sorted by other means.
+hipError_t count_kept(const uint64_t* sorted_keys, size_t n, uint32_t* tile_kept, hipStream_t s);
+// The last of each run of equal sorted keys to uk, its value vals[index[i]] (vals[i] without an index) to
+// uv, the number of them to *dm.
+hipError_t compact_last(const uint64_t* sorted_keys, const uint32_t* index, const uint64_t* vals, size_t n,
+                        const uint32_t* tile_kept, uint64_t* uk, uint64_t* uv, uint32_t* dm, hipStream_t s);
 // Over the m located unique keys (sorted, so each leaf's keys form one run and each last-level
 // node's keys one range): counts the new keys; summary[0] |= 1 if some leaf would exceed
 // 8 keys.  Such a node goes on the re-spread list (nlist: pairs of node index within the last level and

@@ -1,0 +1,329 @@
+// Stable merge sort of (key, staging index) for upsert batches, and the removal of all but the last write
+// of each key.
+//
+// Chunks of 4096 keys are sorted in LDS, then every pass merges pairs of runs.  Both steps are merges of
+// two sorted runs by tiles: a diagonal search splits the runs for each tile (merge path), the tile's keys
+// go to LDS, and each thread finds its own diagonal there and merges eight keys in registers.  Equal keys
+// of the left run go first, so the order of equal keys is the staging order.
+//
+// What bounds it: latency, not bytes (a pass over 2^20 keys moves 25 MB, 5 us at the copy rate).  A pass
+// in which every key searched the other run in global memory (20 dependent reads) took 17 us, now 12;
+// the chunks, sorted before by eight LSD radix passes in LDS (36 us for 2^20 keys, one block per CU, a block
+// barrier every few hundred cycles), take 30.
+#include <utility>
+
+#include "hm_block.h"
+#include "hm_internal.h"
+
+namespace hm {
+namespace {
+
+constexpr int kPer = 8;             // keys per thread
+constexpr int kChunkThreads = 512;  // 4096 keys per chunk
+constexpr int kTileThreads = 256;   // 2048 keys per merge tile
+constexpr uint32_t kTile = kTileThreads * kPer;
+static_assert(kChunkThreads * kPer == (int)kSmallUpdate, "batches of one chunk take the small path");
+
+// Element i sits at slot i + i / 8: threads that each touch eight consecutive elements hit all banks.
+__device__ __forceinline__ uint32_t slot_of(uint32_t i) { return i + (i >> 3); }
+
+template <int NT>
+struct MergeLds {
+  uint64_t k[NT * (kPer + 1)];
+  uint32_t ix[NT * (kPer + 1)];
+};
+
+// Elements diag .. diag + 7 of the merge of the runs [a0, a0 + na) and [b0, b0 + nb) in LDS; past the end
+// of both (KEY_MAX, ~0).
+template <int NT>
+__device__ __forceinline__ void merge_eight(const MergeLds<NT>& m, uint32_t a0, uint32_t na, uint32_t b0, uint32_t nb,
+                                            uint32_t diag, uint64_t (&k)[kPer], uint32_t (&ix)[kPer]) {
+  uint32_t lo = diag > nb ? diag - nb : 0u, hi = diag < na ? diag : na;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (m.k[slot_of(a0 + mid)] <= m.k[slot_of(b0 + diag - 1 - mid)])
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  uint32_t a = a0 + lo, b = b0 + diag - lo;
+  const uint32_t ae = a0 + na, be = b0 + nb;
+  uint64_t ka = a < ae ? m.k[slot_of(a)] : KEY_MAX, kb = b < be ? m.k[slot_of(b)] : KEY_MAX;
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const bool left = a < ae && (b >= be || ka <= kb);
+    const uint32_t src = left ? a : b;
+    k[r] = left ? ka : kb;
+    ix[r] = src < (left ? ae : be) ? m.ix[slot_of(src)] : 0xFFFFFFFFu;
+    if (left) {
+      ++a;
+      ka = a < ae ? m.k[slot_of(a)] : KEY_MAX;
+    } else if (b < be) {
+      ++b;
+      kb = b < be ? m.k[slot_of(b)] : KEY_MAX;
+    }
+  }
+}
+
+template <int NT>
+__device__ __forceinline__ void put_eight(MergeLds<NT>& m, const uint64_t (&k)[kPer], const uint32_t (&ix)[kPer]) {
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    m.k[threadIdx.x * (kPer + 1) + r] = k[r];
+    m.ix[threadIdx.x * (kPer + 1) + r] = ix[r];
+  }
+}
+
+// Chunk c of 4096 staged keys sorted by (key, index); block 0 zeroes the epoch's 8 summary words.
+__global__ __launch_bounds__(kChunkThreads) void chunk_sort_kernel(const uint64_t* __restrict__ pk, uint32_t n,
+                                                                   uint64_t* __restrict__ ko,
+                                                                   uint32_t* __restrict__ io,
+                                                                   uint32_t* __restrict__ summary) {
+  __shared__ MergeLds<kChunkThreads> m;
+  constexpr uint32_t kChunk = kChunkThreads * kPer;
+  if (blockIdx.x == 0 && threadIdx.x < 8) summary[threadIdx.x] = 0;
+  const uint32_t c0 = blockIdx.x * kChunk, e0 = c0 + threadIdx.x * kPer;
+  uint64_t k[kPer];
+  uint32_t ix[kPer];
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    k[r] = e0 + r < n ? pk[e0 + r] : KEY_MAX;
+    ix[r] = e0 + r;
+  }
+  // the thread's eight keys: odd-even transposition, which moves no key past an equal one
+#pragma unroll
+  for (int p = 0; p < kPer; ++p)
+#pragma unroll
+    for (int r = p & 1; r + 1 < kPer; r += 2)
+      if (k[r] > k[r + 1]) {
+        const uint64_t x = k[r];
+        const uint32_t y = ix[r];
+        k[r] = k[r + 1], ix[r] = ix[r + 1];
+        k[r + 1] = x, ix[r + 1] = y;
+      }
+  for (uint32_t w = kPer; w < kChunk; w <<= 1) {  // uniform across the block
+    put_eight(m, k, ix);
+    __syncthreads();
+    const uint32_t t0 = threadIdx.x * kPer, base = t0 & ~(2 * w - 1);
+    merge_eight(m, base, w, base + w, w, t0 - base, k, ix);
+    __syncthreads();
+  }
+  put_eight(m, k, ix);
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint32_t i = r * kChunkThreads + threadIdx.x;
+    if (c0 + i < n) {
+      ko[c0 + i] = m.k[slot_of(i)];
+      io[c0 + i] = m.ix[slot_of(i)];
+    }
+  }
+}
+
+// Where diagonal `diag` splits the merge of A (na keys) and B (nb keys): how many come from A.  One wave,
+// 64 probes per step (four steps for runs of 2^19).
+__device__ __forceinline__ uint32_t wave_split(const uint64_t* __restrict__ A, uint32_t na,
+                                               const uint64_t* __restrict__ B, uint32_t nb, uint32_t diag, int lane) {
+  uint32_t lo = diag > nb ? diag - nb : 0u, hi = diag < na ? diag : na;
+  while (lo < hi) {  // wave-uniform
+    const uint32_t step = (hi - lo + 63) / 64;
+    const uint32_t p = lo + (uint32_t)lane * step;
+    const bool left = p < hi && A[p] <= B[diag - 1 - p];
+    const uint32_t c = (uint32_t)__popcll(__ballot(left));  // the probes that hold are the first c
+    if (c == 0) break;
+    const uint32_t top = lo + c * step;
+    lo = lo + (c - 1) * step + 1;
+    hi = top < hi ? top : hi;
+  }
+  return lo;
+}
+
+// One pass over runs of length L: tile t writes elements [t kTile, (t + 1) kTile) of the merged pairs.
+// LAST: also the tile's number of keys that differ from the next one, for the de-duplication.
+template <bool LAST>
+__global__ __launch_bounds__(kTileThreads) void merge_tile_kernel(const uint64_t* __restrict__ kin,
+                                                                  const uint32_t* __restrict__ iin,
+                                                                  uint64_t* __restrict__ kout,
+                                                                  uint32_t* __restrict__ iout, uint32_t n, uint32_t L,
+                                                                  uint32_t* __restrict__ tile_kept) {
+  __shared__ MergeLds<kTileThreads> m;
+  __shared__ uint32_t split[2], kept_w[kTileThreads / 64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const uint32_t t0 = blockIdx.x * kTile;
+  const uint32_t base = t0 / (2 * L) * (2 * L);  // 2 L is a multiple of kTile: a tile lies in one pair
+  const uint32_t mid = base + L < n ? base + L : n;
+  const uint32_t end = mid + L < n ? mid + L : n;
+  const uint32_t na = mid - base, nb = end - mid;
+  const uint32_t d0 = t0 - base, d1 = d0 + kTile < na + nb ? d0 + kTile : na + nb;
+  if (w < 2) {
+    const uint32_t s = wave_split(kin + base, na, kin + mid, nb, w == 0 ? d0 : d1, lane);
+    if (lane == 0) split[w] = s;
+  }
+  __syncthreads();
+  const uint32_t a0 = split[0], a1 = split[1], b0 = d0 - a0, b1 = d1 - a1;
+  const uint32_t ca = a1 - a0, cb = b1 - b0, cnt = d1 - d0;
+  uint64_t k[kPer];
+  uint32_t ix[kPer];
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {  // every load before the first LDS store
+    const uint32_t i = r * kTileThreads + threadIdx.x;
+    if (i < cnt) {
+      const uint32_t src = i < ca ? base + a0 + i : mid + b0 + (i - ca);
+      k[r] = kin[src];
+      ix[r] = iin[src];
+    }
+  }
+  // the key after the tile, for its last element
+  uint64_t next = KEY_MAX;
+  if (LAST && threadIdx.x == 0) {
+    const uint64_t xa = a1 < na ? kin[base + a1] : KEY_MAX, xb = b1 < nb ? kin[mid + b1] : KEY_MAX;
+    next = xa < xb ? xa : xb;
+  }
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint32_t i = r * kTileThreads + threadIdx.x;
+    if (i < cnt) {
+      m.k[slot_of(i)] = k[r];
+      m.ix[slot_of(i)] = ix[r];
+    }
+  }
+  __syncthreads();
+  const uint32_t diag = threadIdx.x * kPer < cnt ? threadIdx.x * kPer : cnt;
+  merge_eight(m, 0, ca, ca, cb, diag, k, ix);
+  __syncthreads();
+  put_eight(m, k, ix);
+  __syncthreads();
+  uint32_t kept = 0;
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint32_t i = r * kTileThreads + threadIdx.x;
+    if (i < cnt) {
+      const uint64_t x = m.k[slot_of(i)];
+      kout[t0 + i] = x;
+      iout[t0 + i] = m.ix[slot_of(i)];
+      if (LAST && i + 1 < cnt) kept += x != m.k[slot_of(i + 1)] ? 1u : 0u;
+    }
+  }
+  if constexpr (LAST) {
+    if (threadIdx.x == 0 && cnt) kept += m.k[slot_of(cnt - 1)] != next ? 1u : 0u;  // staged keys are below KEY_MAX
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) kept += __shfl_xor(kept, o);
+    if (lane == 0) kept_w[w] = kept;
+    __syncthreads();
+    if (threadIdx.x == 0) tile_kept[blockIdx.x] = kept_w[0] + kept_w[1] + kept_w[2] + kept_w[3];
+  }
+}
+
+// The same count for keys sorted elsewhere (the radix sort of the largest batches).
+__global__ __launch_bounds__(kTileThreads) void count_kept_kernel(const uint64_t* __restrict__ sk, uint32_t n,
+                                                                  uint32_t* __restrict__ tile_kept) {
+  __shared__ uint32_t kept_w[kTileThreads / 64];
+  uint32_t kept = 0;
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint32_t i = blockIdx.x * kTile + r * kTileThreads + threadIdx.x;
+    if (i < n) kept += i + 1 == n || sk[i] != sk[i + 1] ? 1u : 0u;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) kept += __shfl_xor(kept, o);
+  if ((threadIdx.x & 63) == 0) kept_w[threadIdx.x >> 6] = kept;
+  __syncthreads();
+  if (threadIdx.x == 0) tile_kept[blockIdx.x] = kept_w[0] + kept_w[1] + kept_w[2] + kept_w[3];
+}
+
+// The last write of each key to (uk, uv), its value read at the staging index (si) or from the sorted
+// values (si null); *dm = how many.  Each block adds up the tiles before its own (2048 words for 2^22 keys).
+__global__ __launch_bounds__(kTileThreads) void compact_last_kernel(const uint64_t* __restrict__ sk,
+                                                                    const uint32_t* __restrict__ si,
+                                                                    const uint64_t* __restrict__ v, uint32_t n,
+                                                                    const uint32_t* __restrict__ tile_kept,
+                                                                    uint64_t* __restrict__ uk,
+                                                                    uint64_t* __restrict__ uv,
+                                                                    uint32_t* __restrict__ dm) {
+  constexpr int kW = kTileThreads / 64;
+  __shared__ uint32_t scan_sh[kW + 1];
+  __shared__ uint32_t cnt[kPer * kW];  // kept keys per 64 consecutive ones, in order
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint64_t k[kPer], x[kPer];
+  uint32_t at[kPer];
+  bool last[kPer];
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint32_t i = blockIdx.x * kTile + r * kTileThreads + threadIdx.x;
+    k[r] = i < n ? sk[i] : KEY_MAX;
+    last[r] = i < n && (i + 1 == n || sk[i + 1] != k[r]);
+    at[r] = i < n ? (si ? si[i] : i) : 0u;
+  }
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) x[r] = v[at[r]];
+  uint32_t part = 0, before;
+  for (uint32_t t = threadIdx.x; t < blockIdx.x; t += kTileThreads) part += tile_kept[t];
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint64_t b = __ballot(last[r]);
+    at[r] = (uint32_t)__popcll(b & ((1ull << lane) - 1ull));
+    if (lane == 0) cnt[r * kW + w] = (uint32_t)__popcll(b);
+  }
+  (void)block_exclusive_scan<uint32_t, kTileThreads>(part, scan_sh, before);  // its barriers cover cnt too
+  uint32_t total = 0;
+#pragma unroll
+  for (int r = 0; r < kPer; ++r)
+#pragma unroll
+    for (int ww = 0; ww < kW; ++ww) {
+      if (ww == w) at[r] += before + total;
+      total += cnt[r * kW + ww];
+    }
+#pragma unroll
+  for (int r = 0; r < kPer; ++r)
+    if (last[r]) {
+      uk[at[r]] = k[r];
+      uv[at[r]] = x[r];
+    }
+  if (threadIdx.x == 0 && (blockIdx.x + 1) * (uint64_t)kTile >= n) *dm = before + total;
+}
+
+}  // namespace
+
+size_t dedupe_tmp_bytes(size_t n) { return ((n + kTile - 1) / kTile) * sizeof(uint32_t); }
+
+hipError_t merge_sort_index(const uint64_t* pk, uint32_t n, uint64_t* k0, uint64_t* k1, uint32_t* i0, uint32_t* i1,
+                            uint32_t* tile_kept, uint32_t* summary, hipStream_t s, const uint64_t** sorted_keys,
+                            const uint32_t** sorted_index) {
+  if (n <= kSmallUpdate || n > kMergeUpdate) return hipErrorInvalidValue;
+  ProfScope prof("update", s);
+  hipLaunchKernelGGL(chunk_sort_kernel, dim3((n + kSmallUpdate - 1) / kSmallUpdate), dim3(kChunkThreads), 0, s, pk, n,
+                     k0, i0, summary);
+  uint64_t *ka = k0, *kb = k1;
+  uint32_t *ia = i0, *ib = i1;
+  const dim3 grid((n + kTile - 1) / kTile);
+  for (uint32_t L = kSmallUpdate; L < n; L *= 2) {
+    if (2 * (uint64_t)L >= n)
+      hipLaunchKernelGGL(merge_tile_kernel<true>, grid, dim3(kTileThreads), 0, s, ka, ia, kb, ib, n, L, tile_kept);
+    else
+      hipLaunchKernelGGL(merge_tile_kernel<false>, grid, dim3(kTileThreads), 0, s, ka, ia, kb, ib, n, L, tile_kept);
+    std::swap(ka, kb);
+    std::swap(ia, ib);
+  }
+  *sorted_keys = ka;
+  *sorted_index = ia;
+  return hipGetLastError();
+}
+
+hipError_t count_kept(const uint64_t* sorted_keys, size_t n, uint32_t* tile_kept, hipStream_t s) {
+  if (!n) return hipErrorInvalidValue;
+  ProfScope prof("update", s);
+  hipLaunchKernelGGL(count_kept_kernel, dim3((unsigned)((n + kTile - 1) / kTile)), dim3(kTileThreads), 0, s,
+                     sorted_keys, (uint32_t)n, tile_kept);
+  return hipGetLastError();
+}
+
+hipError_t compact_last(const uint64_t* sorted_keys, const uint32_t* index, const uint64_t* vals, size_t n,
+                        const uint32_t* tile_kept, uint64_t* uk, uint64_t* uv, uint32_t* dm, hipStream_t s) {
+  if (!n) return hipErrorInvalidValue;
+  ProfScope prof("update", s);
+  hipLaunchKernelGGL(compact_last_kernel, dim3((unsigned)((n + kTile - 1) / kTile)), dim3(kTileThreads), 0, s,
+                     sorted_keys, index, vals, (uint32_t)n, tile_kept, uk, uv, dm);
+  return hipGetLastError();
+}
+
+}  // namespace hm

@@ -15,7 +15,6 @@
 // keys?) and then applies it.  An epoch of 4001 keys (2^24 stored) with the read of its keys: 115 us in
 // 17 launches, now 60 us in six.
 #include <algorithm>
-#include <utility>
 
 #include "hm_device.h"
 
@@ -88,23 +87,6 @@ __device__ __forceinline__ int leaf_count(const Leaf& l) {
 #pragma unroll
   for (int i = 0; i < LEAF_KEYS; ++i) c += l.key[i] != KEY_MAX ? 1 : 0;
   return c;
-}
-
-__global__ void mark_last_kernel(const uint64_t* __restrict__ k, size_t n, uint32_t* __restrict__ keep) {
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-    keep[i] = (i + 1 == n || k[i] != k[i + 1]) ? 1u : 0u;
-}
-
-__global__ void compact_kernel(const uint64_t* __restrict__ k, const uint64_t* __restrict__ v,
-                               const uint32_t* __restrict__ keep, const uint32_t* __restrict__ scan, size_t n,
-                               uint64_t* __restrict__ ko, uint64_t* __restrict__ vo) {
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-    if (keep[i]) {
-      ko[scan[i]] = k[i];
-      vo[scan[i]] = v[i];
-    }
 }
 
 __global__ void count_inserts_kernel(const uint32_t* __restrict__ leaf, const uint8_t* __restrict__ found, size_t n,
@@ -236,134 +218,6 @@ __global__ void relayout_touched_kernel(const Leaf* __restrict__ old_leaves, con
   }
 }
 
-constexpr int kSortThreads = 1024;
-
-// LSD radix sort, in LDS, of kSmallUpdate (key, index) pairs held in (sk[0], si[0]), over the 8 key
-// bytes; stable, so equal keys keep their index order.  8 passes that each move the pairs through LDS
-// once (a bitonic network over the same pairs takes 78 steps).  Wave w owns positions
-// [256 w, 256 w + 256), element r of lane l being 256 w + 64 r + l; ranks within a wave come from the
-// digit ballots (match_digit), in that order.  Returns the buffer (0 or 1) holding the result; ends
-// with a block barrier.
-constexpr int kChunkWaves = kSortThreads / 64;
-constexpr int kChunkItems = kSmallUpdate / kSortThreads;
-static_assert(kChunkItems * 64 * kChunkWaves == (int)kSmallUpdate, "each wave owns 64 x kChunkItems positions");
-struct RadixLds {
-  uint64_t sk[2][kSmallUpdate];
-  uint32_t si[2][kSmallUpdate];
-  uint32_t wcnt[kChunkWaves][256];
-  uint32_t boff[256];
-  uint32_t scan_sh[kChunkWaves + 1];
-};
-__device__ __forceinline__ int radix_sort_lds(RadixLds& L) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const uint64_t lt = (1ull << lane) - 1ull;
-  const uint32_t base = (uint32_t)w * 64 * kChunkItems;
-  int cur = 0;
-  for (int shift = 0; shift < 64; shift += 8) {  // uniform across the block
-    for (int i = threadIdx.x; i < kChunkWaves * 256; i += kSortThreads) (&L.wcnt[0][0])[i] = 0;
-    __syncthreads();  // the pairs (first pass) and the cleared counters
-    uint64_t k[kChunkItems];
-    uint32_t ix[kChunkItems], pkd[kChunkItems];
-#pragma unroll
-    for (int r = 0; r < kChunkItems; ++r) {
-      k[r] = L.sk[cur][base + r * 64 + lane];
-      ix[r] = L.si[cur][base + r * 64 + lane];
-    }
-#pragma unroll
-    for (int r = 0; r < kChunkItems; ++r) {
-      const uint32_t d = (uint32_t)(k[r] >> shift) & 255u;
-      const uint64_t peers = match_digit(d, ~0ull);
-      const uint32_t prior = L.wcnt[w][d];
-      if ((peers & lt) == 0) L.wcnt[w][d] = prior + (uint32_t)__popcll(peers);
-      pkd[r] = ((prior + (uint32_t)__popcll(peers & lt)) << 8) | d;
-    }
-    __syncthreads();
-    {
-      // per digit: each wave's start inside the digit, then the digit's start
-      const int d = threadIdx.x;
-      uint32_t run = 0;
-      if (d < 256) {
-#pragma unroll
-        for (int ww = 0; ww < kChunkWaves; ++ww) {
-          const uint32_t t = L.wcnt[ww][d];
-          L.wcnt[ww][d] = run;
-          run += t;
-        }
-      }
-      uint32_t total;
-      const uint32_t e = block_exclusive_scan<uint32_t, kSortThreads>(run, L.scan_sh, total);
-      if (d < 256) L.boff[d] = e;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kChunkItems; ++r) {
-      const uint32_t d = pkd[r] & 255u;
-      const uint32_t np = L.boff[d] + L.wcnt[w][d] + (pkd[r] >> 8);
-      L.sk[cur ^ 1][np] = k[r];
-      L.si[cur ^ 1][np] = ix[r];
-    }
-    cur ^= 1;
-    __syncthreads();  // every thread has read wcnt / boff before the next pass clears them
-  }
-  return cur;
-}
-
-// First stage of the merge sort of mid-size batches: chunk c of kSmallUpdate staged keys sorted by
-// key with their staging indices.  Padding (KEY_MAX, ~0) has digit 255 in every pass and sorts after
-// every staged key.
-__global__ __launch_bounds__(kSortThreads) void chunk_sort_kernel(const uint64_t* __restrict__ pk, uint32_t n,
-                                                                  uint64_t* __restrict__ ko,
-                                                                  uint32_t* __restrict__ io) {
-  __shared__ RadixLds L;
-  const uint32_t c0 = blockIdx.x * kSmallUpdate;
-  const uint32_t cnt = n - c0 < kSmallUpdate ? n - c0 : kSmallUpdate;
-  for (uint32_t i = threadIdx.x; i < kSmallUpdate; i += kSortThreads) {
-    L.sk[0][i] = i < cnt ? pk[c0 + i] : KEY_MAX;
-    L.si[0][i] = i < cnt ? c0 + i : 0xFFFFFFFFu;
-  }
-  const int cur = radix_sort_lds(L);
-  for (uint32_t i = threadIdx.x; i < cnt; i += kSortThreads) {
-    ko[c0 + i] = L.sk[cur][i];
-    io[c0 + i] = L.si[cur][i];
-  }
-}
-
-// One merge pass over sorted runs of length L (pairs [2gL, 2gL + L) and [2gL + L, 2gL + 2L)): each
-// element goes to its own rank in the run plus the number of elements of the other run that order
-// before it.  (key, index) pairs are all distinct, so the ranks never collide and the merge keeps
-// the staging order of equal keys.
-__global__ __launch_bounds__(256) void merge_pass_kernel(const uint64_t* __restrict__ kin,
-                                                         const uint32_t* __restrict__ iin,
-                                                         uint64_t* __restrict__ kout, uint32_t* __restrict__ iout,
-                                                         uint32_t n, uint32_t L) {
-  const uint32_t e = blockIdx.x * 256u + threadIdx.x;
-  if (e >= n) return;
-  const uint32_t base = e / (2 * L) * (2 * L);
-  const uint32_t mid = base + L < n ? base + L : n;
-  const uint32_t end = mid + L < n ? mid + L : n;
-  const uint64_t k = kin[e];
-  const uint32_t ix = iin[e];
-  const bool in_a = e < mid;
-  uint32_t lo = in_a ? mid : base, hi = in_a ? end : mid;  // search the other run
-  while (lo < hi) {
-    const uint32_t m = (lo + hi) >> 1;
-    const uint64_t km = kin[m];
-    if (km < k || (km == k && iin[m] < ix))
-      lo = m + 1;
-    else
-      hi = m;
-  }
-  const uint32_t pos = in_a ? base + (e - base) + (lo - mid) : base + (e - mid) + (lo - base);
-  kout[pos] = k;
-  iout[pos] = ix;
-}
-
-__global__ void gather_by_index_kernel(const uint64_t* __restrict__ v, const uint32_t* __restrict__ ix, uint32_t n,
-                                       uint64_t* __restrict__ out) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = v[ix[i]];
-}
-
 // Small batches (n <= kSmallUpdate), first kernel: every staged key's place in the order by (key, staging
 // index), counted against all n keys held in LDS.  A block places 16 keys, 32 slices of the batch each, so
 // 4096 keys take 256 blocks and 128 steps of two compares per thread.  One block sorting 4096 keys (LSD
@@ -449,11 +303,6 @@ __global__ __launch_bounds__(256) void dedupe_locate_kernel(TreeView tv, const u
     found_out[o] = eq ? 1 : 0;
   }
   if (threadIdx.x == 0 && base + kPer >= n) *dm = before + (uint32_t)__popc(km);
-}
-
-__global__ void unique_count_kernel(const uint32_t* __restrict__ keep, const uint32_t* __restrict__ scan, size_t n,
-                                    uint32_t* __restrict__ dm) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *dm = scan[n - 1] + keep[n - 1];
 }
 
 __device__ __forceinline__ bool run_head(const uint32_t* __restrict__ leaf, uint32_t i) {
@@ -770,31 +619,6 @@ hipError_t small_sort_locate(const TreeView& tv, const uint64_t* pk, const uint6
   return hipGetLastError();
 }
 
-hipError_t merge_sort_pairs(const uint64_t* pk, const uint64_t* pv, uint32_t n, uint64_t* k0, uint64_t* k1,
-                            uint32_t* i0, uint32_t* i1, uint64_t* vout, hipStream_t s, const uint64_t** sorted_keys) {
-  if (n == 0) return hipErrorInvalidValue;
-  ProfScope prof("update", s);
-  const uint32_t chunks = (n + kSmallUpdate - 1) / kSmallUpdate;
-  hipLaunchKernelGGL(chunk_sort_kernel, dim3(chunks), dim3(kSortThreads), 0, s, pk, n, k0, i0);
-  uint64_t *ka = k0, *kb = k1;
-  uint32_t *ia = i0, *ib = i1;
-  const unsigned grid = (unsigned)((n + 255) / 256);
-  for (uint64_t L = kSmallUpdate; L < n; L *= 2) {
-    hipLaunchKernelGGL(merge_pass_kernel, dim3(grid), dim3(256), 0, s, ka, ia, kb, ib, n, (uint32_t)L);
-    std::swap(ka, kb);
-    std::swap(ia, ib);
-  }
-  hipLaunchKernelGGL(gather_by_index_kernel, dim3(grid), dim3(256), 0, s, pv, ia, n, vout);
-  *sorted_keys = ka;
-  return hipGetLastError();
-}
-
-hipError_t unique_count(const uint32_t* keep, const uint32_t* keep_scan, size_t n, uint32_t* dm, hipStream_t s) {
-  if (!n) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(unique_count_kernel, dim3(1), dim3(64), 0, s, keep, keep_scan, n, dm);
-  return hipGetLastError();
-}
-
 hipError_t plan_runs(const Leaf* leaves, uint32_t n_leaves, int F, const uint32_t* leaf, const uint32_t* slot,
                      const uint8_t* found, const uint64_t* uk, size_t n, const uint32_t* dm, uint32_t* summary,
                      uint32_t* nlist, uint32_t* host, hipStream_t s) {
@@ -846,21 +670,6 @@ hipError_t apply_runs(Leaf* leaves, const uint32_t* leaf, const uint32_t* slot, 
   ProfScope prof("update", s);
   hipLaunchKernelGGL(apply_runs_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, leaves, leaf, slot, found, uk, uv, n,
                      dm);
-  return hipGetLastError();
-}
-
-hipError_t mark_last_of_runs(const uint64_t* sorted_keys, size_t n, uint32_t* keep, hipStream_t s) {
-  if (!n) return hipSuccess;
-  ProfScope prof("update", s);
-  hipLaunchKernelGGL(mark_last_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, sorted_keys, n, keep);
-  return hipGetLastError();
-}
-
-hipError_t compact_pairs(const uint64_t* k, const uint64_t* v, const uint32_t* keep, const uint32_t* keep_scan,
-                         size_t n, uint64_t* ko, uint64_t* vo, hipStream_t s) {
-  if (!n) return hipSuccess;
-  ProfScope prof("update", s);
-  hipLaunchKernelGGL(compact_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, k, v, keep, keep_scan, n, ko, vo);
   return hipGetLastError();
 }
 
