@@ -1165,7 +1165,7 @@ int publish_prepare(hm_tree* t, hipStream_t s, PublishPlan* plan) {
       HM_TRY(count_kept(sk, n, tile_kept, s));
     }
     HM_TRY(compact_last(sk, si, sv, n, tile_kept, b.uk, b.uv, dm, s));
-    HM_TRY(launch_locate(tv, b.uk, n, b.leaf, b.slot, b.found, s, dm));
+    HM_TRY(launch_locate(tv, t->lds_levels, b.uk, n, b.leaf, b.slot, b.found, s, dm));
   }
   HM_TRY(plan_runs(t->d_leaves, (uint32_t)t->n_leaves, t->F, b.leaf, b.slot, b.found, b.uk, n, dm, b.summary, b.nlist,
                    t->upd_host, s));

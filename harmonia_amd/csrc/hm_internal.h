@@ -181,9 +181,9 @@ hipError_t copy_u32s(uint32_t* dst, const uint32_t* src, size_t n, hipStream_t s
 hipError_t build_child_array(const uint32_t* prefix, uint32_t n_inner, int F, uint32_t* child, hipStream_t s);
 hipError_t launch_search_baseline(const TreeView& tv, const uint32_t* child, const uint64_t* q, uint64_t* out_vals,
                                   uint8_t* out_found, uint32_t n, int group, int kind, hipStream_t s);
-// Locate (update path): leaf, lower_bound slot (low byte) with the leaf's free slots (next byte)
+// Locate sorted keys (update path): leaf, lower_bound slot (low byte) with the leaf's free slots (next byte)
 // and found flag per key; n sizes the grid, dn (device) may hold the actual count.
-hipError_t launch_locate(const TreeView& tv, const uint64_t* keys, size_t n, uint32_t* leaf_out, uint32_t* slot_out,
+hipError_t launch_locate(const TreeView& tv, int lds_levels, const uint64_t* keys, size_t n, uint32_t* leaf_out, uint32_t* slot_out,
                          uint8_t* found_out, hipStream_t s, const uint32_t* dn = nullptr);
 
 // ---- range (hm_range.hip) --------------------------------------------------------------
