@@ -244,6 +244,15 @@ PipeBufs carve_pipe(char*& cur, size_t n, int psa_bits, int out_mode) {
   return b;
 }
 
+// Searches that return results in input order split the batch once and order it further inside each
+// block.  The rule: the launch shape is the default one, which that kernel replaces (other shapes are asked
+// for by name or by the tuner), and two sort passes would be made, whose records' memory then holds the
+// partition's.  Over 2^18..2^26 keys, fanouts 32..128, 2^20..2^24 queries in every order it takes 0.45 to
+// 0.92 of the time of the two passes and search_span_kernel, and nowhere more.
+static bool partitions(const SearchLaunch& sl, int psa_bits) {
+  return sl.group == 2 && sl.queries_per_group == 4 && !sl.window && psa_bits > 8 && psa_bits <= 16;
+}
+
 int enqueue_pipeline(const TreeView& tv, const SearchLaunch& sl, int psa_bits, int out_mode, const uint64_t* dq,
                      size_t n, const uint32_t* dn, const PipeBufs& b, uint64_t* dvals, uint8_t* dfound,
                      uint32_t* dpos, hipStream_t s) {
@@ -256,6 +265,13 @@ int enqueue_pipeline(const TreeView& tv, const SearchLaunch& sl, int psa_bits, i
   // psa_top (the bits above it are equal for every key, so they would order nothing but misses outside
   // the key range).  PSA-order results keep the reference's window [64 - psa_bits, 64).
   const int top = out_mode == HM_OUT_PSA_ORDER ? 64 : std::max(std::min((int)tv.psa_top, 64), psa_bits);
+  if (out_mode == HM_OUT_UNPERMUTE && partitions(sl, psa_bits)) {
+    const int bits = partition_bits(n);
+    HM_TRY(partition_keys(dq, n, top, b.k0, b.replay, s, dn));
+    HM_TRY(launch_search_chunks(tv, b.k0, b.rv, b.rf, n, top, bits, s, dn));
+    HM_TRY(unpartition_results(b.rv, b.rf, n, b.replay, dvals, dfound, s, dn));
+    return HM_OK;
+  }
   if (out_mode == HM_OUT_UNPERMUTE) {
     // keys-only sort recording its passes; search in PSA order (coalesced result writes); then the
     // passes run backwards to put the results in input order

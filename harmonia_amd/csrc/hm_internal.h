@@ -107,6 +107,19 @@ hipError_t unsort_results(uint64_t* vals, uint8_t* found, size_t n, int bits, co
                           uint8_t* f_tmp, uint64_t* out_vals, uint8_t* out_found, hipStream_t s,
                           const uint32_t* dn = nullptr);
 
+// ---- partition (hm_part.hip) -----------------------------------------------------------
+// One pass that splits a batch by the key bits [top - b, top), b = partition_bits(n), into buckets of at
+// most kPartBucket queries on average (more once b is kPartMaxBits), in no particular order inside a
+// bucket, and records in rec (partition_bytes(n)) how to undo it.  n sizes the launches; dn (device) may
+// hold a smaller count.
+constexpr int kPartMinBits = 8, kPartMaxBits = 11, kPartBucket = 4096;
+int partition_bits(size_t n);
+size_t partition_bytes(size_t n);
+hipError_t partition_keys(const uint64_t* q, size_t n, int top, uint64_t* out, void* rec, hipStream_t s,
+                          const uint32_t* dn);
+hipError_t unpartition_results(const uint64_t* vals, const uint8_t* found, size_t n, const void* rec,
+                               uint64_t* out_vals, uint8_t* out_found, hipStream_t s, const uint32_t* dn);
+
 // ---- build (hm_build.hip) --------------------------------------------------------------
 // flags |= 1 if a key is KEY_MAX, |= 2 if keys are not strictly ascending.
 hipError_t validate_sorted(const uint64_t* keys, size_t n, uint32_t* d_flags, hipStream_t s);
@@ -166,6 +179,9 @@ enum SearchOut {
 hipError_t launch_search(const TreeView& tv, const SearchLaunch& sl, const uint64_t* q, const uint32_t* pos,
                          uint64_t* out_vals, uint8_t* out_found, size_t n, SearchOut mode, hipStream_t s,
                          const uint32_t* dn = nullptr);
+// Search of a partitioned batch (partition_keys over bits [top - bits, top)): result i of query q[i].
+hipError_t launch_search_chunks(const TreeView& tv, const uint64_t* q, uint64_t* out_vals, uint8_t* out_found, size_t n,
+                                int top, int bits, hipStream_t s, const uint32_t* dn);
 // Bytes of LDS the top `levels` need.
 size_t lds_bytes_for(const TreeView& tv, int levels);
 // *p = v as a one-thread kernel (a graph-safe way to hand a count to the next replay).

@@ -683,6 +683,279 @@ hipError_t launch_window(const TreeView& tv, const SearchLaunch& sl, const uint6
   return hipGetLastError();
 }
 
+// ---- chunk search (batches partitioned by bucket) ------------------------------------------------
+//
+// A block takes kChunk consecutive queries of the partitioned batch: a bucket or a part of one, so a narrow
+// key range in any order.  It orders them by the bits below the bucket's (an LDS atomic gives each key its
+// place, no order among equal digits), and each wave searches 512 neighbours, one lane per query:
+//   - every descent starts at the deepest node that holds the chunk's smallest and largest key;
+//   - per level, the run of nodes that 256 queries reach goes to LDS (LDS-direct loads, one round trip) and
+//     each lane ranks its key there by binary search;
+//   - 64 queries at a time, the distinct leaves among neighbours go to LDS, eight whole leaves per load, and
+//     each lane finds its key there.
+// Results go back to LDS and out in the order the queries came in, which the un-partition expects.
+//
+// What bounds it: the leaves' lines at the rate memory gives lines in key order.  2^24 queries of 2^26 keys
+// read 1.45 GB and write 0.15 in 404 us (4.0 TB/s; VALU 45% busy); search_span_kernel over the fully sorted
+// batch took 362 us for 1.54 GB, but the second sorting pass that needs cost 180.  2^20 queries of 2^20 keys:
+// 27 us against 21 plus 35 of sorting.
+constexpr int kChunkThreads = 512;
+constexpr int kChunkWaves = kChunkThreads / 64;
+constexpr int kChunkItems = 8;
+constexpr uint32_t kChunk = kChunkThreads * kChunkItems;
+constexpr int kChunkBits = 11;  // digit of the order inside a chunk
+constexpr uint32_t kChunkDigits = 1u << kChunkBits;
+constexpr int kChunkGroup = 4;  // rounds of 64 queries that share a node run
+// A wave's node run: 4 KiB (12 nodes of fanout 32, 7 of 64, 3 of 128); two blocks (16 waves) per CU.  2 KiB
+// was slower (421 us against 404 on 2^24 queries of 2^26 keys: more runs that do not fit), and so were five
+// or six waves per SIMD, whose registers spill (463 and 485 us).
+constexpr uint32_t kChunkNodeBytes = 4096;
+constexpr uint32_t kChunkLeaves = kChunk * 8 / kChunkWaves / sizeof(Leaf);  // leaves in a wave's share of the keys' LDS
+
+// upper_bound slot of t in a node held in LDS, one lane per query (the last key slot is KEY_MAX > t).
+template <int F>
+__device__ __forceinline__ uint32_t node_next_bin(const uint64_t* nd, uint64_t t) {
+  const uint64_t* k = nd + idx_slots(F);
+  uint32_t r = 0;
+#pragma unroll
+  for (uint32_t st = F / 2; st > 0; st >>= 1) r += k[r + st - 1] <= t ? st : 0u;
+  return (uint32_t)nd[idx_slots(F) - 1] + r;
+}
+
+// One level for R rounds of queries: the run of nodes they reach through LDS if it fits, else round by
+// round, else each lane reads its node.
+template <int F, int R>
+__device__ __forceinline__ void chunk_level(const uint64_t* __restrict__ inner, uint64_t* nbuf, const uint64_t* t,
+                                            uint32_t* node, int lane) {
+  constexpr int NS = node_slots(F);
+  constexpr int CH = NS / 2;
+  constexpr int SPAN = kChunkNodeBytes / (NS * 8);
+  constexpr int SPL = kChunkNodeBytes / 1024;
+  uint32_t lo = node[0], hi = node[0];
+#pragma unroll
+  for (int j = 1; j < R; ++j) {
+    lo = node[j] < lo ? node[j] : lo;
+    hi = node[j] > hi ? node[j] : hi;
+  }
+  lo = wave_min_u32(lo);
+  hi = wave_max_u32(hi);
+  if (hi - lo < (uint32_t)SPAN) {  // wave-uniform
+    wave_stage<SPL>(reinterpret_cast<const ulonglong2*>(inner + (size_t)lo * NS), (int)(hi - lo + 1) * CH, nbuf, lane);
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+      node[j] = node_next_bin<F>(nbuf + (node[j] - lo) * NS, t[j] == KEY_MAX ? KEY_MAX - 1 : t[j]);
+    wave_lds_sync();  // the next run overwrites the buffer
+  } else if constexpr (R > 1) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) chunk_level<F, 1>(inner, nbuf, t + j, node + j, lane);
+  } else {
+    node[0] = node_next<F, 1>(inner + (size_t)node[0] * NS, t[0] == KEY_MAX ? KEY_MAX - 1 : t[0], 0, lane);
+  }
+}
+
+// q: partitioned keys, by bits [top - bits, top).
+template <int F>
+__global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv, const uint64_t* __restrict__ q,
+                                                                     uint64_t* __restrict__ out_vals,
+                                                                     uint8_t* __restrict__ out_found, uint32_t n,
+                                                                     int top, int bits,
+                                                                     const uint32_t* __restrict__ dn) {
+  constexpr int NS = node_slots(F);
+  constexpr int DPer = kChunkDigits / kChunkThreads;
+  __shared__ __align__(16) uint64_t sk[kChunk];  // sorted keys, then each wave's leaves, then values
+  __shared__ __align__(16) uint8_t sf[kChunk];                 // found flags (before: each wave's list of leaves)
+  __shared__ __align__(16) uint64_t nbufs[kChunkWaves * kChunkNodeBytes / 8];  // before: the digit counters
+  __shared__ uint64_t wmin[kChunkWaves], wmax[kChunkWaves];
+  __shared__ uint32_t scan_sh[kChunkWaves + 1];
+  static_assert(sizeof(nbufs) >= kChunkDigits * 4, "the counters fit under the node runs");
+  uint32_t* cnt = reinterpret_cast<uint32_t*>(nbufs);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (dn) n = *dn;
+  const uint32_t c0 = xcd_block(blockIdx.x, gridDim.x) * kChunk;
+  if (c0 >= n) return;  // block-uniform
+  const uint32_t m = n - c0 < kChunk ? n - c0 : kChunk;
+  uint64_t k[kChunkItems];
+#pragma unroll
+  for (int r = 0; r < kChunkItems; ++r) {
+    const uint32_t i = r * kChunkThreads + threadIdx.x;
+    k[r] = q[c0 + (i < m ? i : m - 1)];
+  }
+  const uint64_t kf = q[c0], kl = q[c0 + m - 1];  // uniform: the first and last bucket
+#pragma unroll
+  for (int j = 0; j < DPer; ++j) cnt[j * kChunkThreads + threadIdx.x] = 0;
+  // the order's digit: bits below the first bucket's, shifted so that the chunk's buckets fit
+  const int lo = top - bits > kChunkBits ? top - bits - kChunkBits : 0;
+  const int ext = top - bits - lo;  // bits kept per bucket
+  const uint32_t fmask = (1u << (bits + ext)) - 1u;
+  const uint32_t first = ((uint32_t)(kf >> lo) & fmask) >> ext << ext;
+  const uint32_t span = (((uint32_t)(kl >> lo) & fmask) >> ext << ext) - first + (1u << ext);  // buckets ascend
+  const int sh = span > kChunkDigits ? 32 - kChunkBits - __builtin_clz(span - 1) : 0;
+  uint64_t mn = ~0ull, mx = 0;
+#pragma unroll
+  for (int r = 0; r < kChunkItems; ++r) {
+    const uint64_t td = k[r] == KEY_MAX ? KEY_MAX - 1 : k[r];
+    mn = td < mn ? td : mn;
+    mx = td > mx ? td : mx;
+  }
+  mn = wave_min_u64(mn);
+  mx = wave_max_u64(mx);
+  if (lane == 0) {
+    wmin[w] = mn;
+    wmax[w] = mx;
+  }
+  __syncthreads();
+  uint32_t pos[kChunkItems];
+#pragma unroll
+  for (int r = 0; r < kChunkItems; ++r) {
+    const uint32_t i = r * kChunkThreads + threadIdx.x;
+    const uint32_t d = (((uint32_t)(k[r] >> lo) & fmask) - first) >> sh;
+    const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);
+    pos[r] = 0;
+    if (__ballot(i < m && d == f) == ~0ull) {  // one digit in the whole wave: one add
+      uint32_t b = 0;
+      if (lane == 0) b = atomicAdd(&cnt[f], 64u);
+      pos[r] = (uint32_t)__builtin_amdgcn_readfirstlane((int)b) + lane;
+    } else if (i < m) {
+      pos[r] = atomicAdd(&cnt[d], 1u);
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < kChunkWaves; ++x) {
+    mn = wmin[x] < mn ? wmin[x] : mn;
+    mx = wmax[x] > mx ? wmax[x] : mx;
+  }
+  __syncthreads();
+  {
+    uint32_t c[DPer], s = 0, total;
+#pragma unroll
+    for (int j = 0; j < DPer; ++j) {
+      c[j] = cnt[threadIdx.x * DPer + j];
+      s += c[j];
+    }
+    uint32_t run = block_exclusive_scan<uint32_t, kChunkThreads>(s, scan_sh, total);
+#pragma unroll
+    for (int j = 0; j < DPer; ++j) {
+      cnt[threadIdx.x * DPer + j] = run;
+      run += c[j];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kChunkItems; ++r) {
+    const uint32_t i = r * kChunkThreads + threadIdx.x;
+    const uint32_t d = (((uint32_t)(k[r] >> lo) & fmask) - first) >> sh;
+    if (i < m) {
+      pos[r] += cnt[d];
+      sk[pos[r]] = k[r];
+    }
+  }
+  // the deepest node above the leaves that holds the whole chunk (every wave finds it; uniform)
+  const uint64_t* __restrict__ inner = tv.inner;
+  const int last = tv.height - 1;
+  uint32_t start = 0;
+  int l0 = 0;
+  {
+    constexpr int GW = 32;
+    const uint64_t a = uniform_u64(mn), b = uniform_u64(mx);
+    while (l0 < last) {
+      const uint32_t c = node_next_wide<F, GW>(inner + (size_t)start * NS, lane < GW ? a : b, lane % GW, lane & GW);
+      const uint32_t ca = (uint32_t)__builtin_amdgcn_readlane((int)c, 0);
+      if (ca != (uint32_t)__builtin_amdgcn_readlane((int)c, GW)) break;
+      start = ca;
+      ++l0;
+    }
+  }
+  __syncthreads();  // keys are in place, the counters are free for the node runs
+  const uint32_t p0 = w * 64 * kChunkItems + lane;  // the lane's queries: p0 + 64 j
+  uint64_t t[kChunkItems];
+  uint32_t node[kChunkItems];
+#pragma unroll
+  for (int j = 0; j < kChunkItems; ++j) {
+    const uint32_t p = p0 + 64 * j;
+    t[j] = sk[p < m ? p : m - 1];
+    node[j] = start;
+  }
+  __syncthreads();  // every wave has its keys: their LDS holds leaves from here on
+  uint64_t* nbuf = nbufs + w * (kChunkNodeBytes / 8);
+  uint64_t* lbuf = sk + w * (kChunkLeaves * 16);
+  uint32_t* llist = reinterpret_cast<uint32_t*>(sf) + w * (kChunk / 4 / kChunkWaves);  // 128 words
+#pragma unroll
+  for (int g = 0; g < kChunkItems; g += kChunkGroup)
+    if (p0 - lane + 64 * g < m)  // wave-uniform
+      for (int l = l0; l <= last; ++l) chunk_level<F, kChunkGroup>(inner, nbuf, t + g, node + g, lane);
+  uint32_t found = 0;
+#pragma unroll
+  for (int j = 0; j < kChunkItems; ++j) {
+    if (p0 - lane + 64 * j >= m) break;  // wave-uniform
+    // the leaves that differ from the lane below's, numbered in lane order
+    const uint32_t prev = (uint32_t)__shfl_up((int)node[j], 1);
+    const bool head = lane == 0 || prev != node[j];
+    const uint64_t heads = __ballot(head);
+    const uint32_t mine = (uint32_t)__popcll(heads & ((2ull << lane) - 1ull)) - 1u;
+    const uint32_t nd = (uint32_t)__popcll(heads);
+    if (head) llist[mine] = node[j] - tv.n_inner;
+    wave_lds_sync();
+    uint64_t val = 0;
+    bool eq = false;
+    for (uint32_t b = 0; b < nd; b += kChunkLeaves) {  // wave-uniform: at most two rounds of 32 leaves
+      // eight leaves per load; a leaf's 16-byte piece p lands at place p ^ (number & 7), so lanes that read
+      // the same piece of different leaves spread over the banks
+#pragma unroll
+      for (uint32_t u = 0; u < kChunkLeaves / 8; ++u) {
+        if (b + 8 * u < nd) {
+          const uint32_t x = b + 8 * u + (lane >> 3);
+          const uint32_t lf = llist[x < nd ? x : nd - 1];
+          __builtin_amdgcn_global_load_lds(
+              (const global_void*)(reinterpret_cast<const ulonglong2*>(tv.leaves + lf) + ((lane ^ (lane >> 3)) & 7)),
+              (lds_void*)(lbuf + 128 * u), 16, 0, 0);
+        }
+      }
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the leaves have landed in LDS
+      wave_lds_sync();
+      if (mine - b < kChunkLeaves) {
+        const uint32_t sw = mine & 7;
+        const ulonglong2* lf = reinterpret_cast<const ulonglong2*>(lbuf + (mine - b) * 16);
+        uint32_t lt = 0;
+#pragma unroll
+        for (uint32_t p = 0; p < 4; ++p) {
+          const ulonglong2 x = lf[p ^ sw];
+          lt += (x.x < t[j] ? 1u : 0u) + (x.y < t[j] ? 1u : 0u);
+          eq |= x.x == t[j] || x.y == t[j];
+        }
+        eq = eq && t[j] != KEY_MAX;  // KEY_MAX is padding, never a stored key
+        if (eq) val = reinterpret_cast<const uint64_t*>(lf + ((4 + lt / 2) ^ sw))[lt & 1];
+      }
+      wave_lds_sync();  // the next loads overwrite the leaves
+    }
+    t[j] = val;
+    found |= eq ? 1u << j : 0u;
+  }
+  __syncthreads();  // every wave is done with its leaves
+#pragma unroll
+  for (int j = 0; j < kChunkItems; ++j) {
+    sk[p0 + 64 * j] = t[j];
+    sf[p0 + 64 * j] = (found >> j) & 1u;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kChunkItems; ++r) {
+    const uint32_t i = r * kChunkThreads + threadIdx.x;
+    if (i < m) {
+      out_vals[c0 + i] = sk[pos[r]];
+      out_found[c0 + i] = sf[pos[r]];
+    }
+  }
+}
+
+template <int F>
+hipError_t launch_chunk(const TreeView& tv, const uint64_t* q, uint64_t* out_vals, uint8_t* out_found, size_t n,
+                        int top, int bits, hipStream_t s, const uint32_t* dn) {
+  const size_t nb = ((n + kChunk - 1) / kChunk + 7) / 8 * 8;
+  hipLaunchKernelGGL(search_chunk_kernel<F>, dim3((unsigned)nb), dim3(kChunkThreads), 0, s, tv, q,
+                     out_vals, out_found, (uint32_t)n, top, bits, dn);
+  return hipGetLastError();
+}
+
 // Locate for the update path: leaf id, lower_bound slot (low byte) with the leaf's free slots (next byte),
 // and found flag per key (input order).
 template <int F, int G>
@@ -886,6 +1159,18 @@ hipError_t launch_search(const TreeView& tv, const SearchLaunch& sl, const uint6
     case 32: return launch_f<32>(tv, sl, q, pos, out_vals, out_found, n, mode, s, dn);
     case 64: return launch_f<64>(tv, sl, q, pos, out_vals, out_found, n, mode, s, dn);
     case 128: return launch_f<128>(tv, sl, q, pos, out_vals, out_found, n, mode, s, dn);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_search_chunks(const TreeView& tv, const uint64_t* q, uint64_t* out_vals, uint8_t* out_found, size_t n,
+                                int top, int bits, hipStream_t s, const uint32_t* dn) {
+  if (n == 0) return hipSuccess;
+  ProfScope prof("search", s);
+  switch (tv.fanout) {
+    case 32: return launch_chunk<32>(tv, q, out_vals, out_found, n, top, bits, s, dn);
+    case 64: return launch_chunk<64>(tv, q, out_vals, out_found, n, top, bits, s, dn);
+    case 128: return launch_chunk<128>(tv, q, out_vals, out_found, n, top, bits, s, dn);
     default: return hipErrorInvalidValue;
   }
 }
