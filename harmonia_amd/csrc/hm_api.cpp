@@ -152,13 +152,13 @@ int ensure_ws(hm_tree* t, hipStream_t s, size_t bytes, Workspace** out) {
     const size_t old = w.bytes;
     if (w.buf) {
       HM_TRY(hipStreamSynchronize(s));
-      HM_TRY(hipFree(w.buf));
+      HM_TRY(dev_free(w.buf));
       w.buf = nullptr;
       w.bytes = 0;
     }
     // geometric growth: a hipFree synchronizes the whole device
     size_t want = std::max(std::max(bytes, 2 * old), (size_t)1 << 20);
-    HM_TRY(hipMalloc(&w.buf, want));
+    HM_TRY(dev_malloc(&w.buf, want));
     w.bytes = want;
   }
   *out = &w;
@@ -330,11 +330,11 @@ int ensure_rl(hm_tree* t, size_t bytes, hipStream_t s) {
                    (unsigned long long)want);
   if (t->rl_buf) {
     HM_TRY(hipStreamSynchronize(s));
-    HM_TRY(hipFree(t->rl_buf));
+    HM_TRY(dev_free(t->rl_buf));
     t->rl_buf = nullptr;
     t->rl_bytes = 0;
   }
-  HM_TRY(hipMalloc(&t->rl_buf, want));
+  HM_TRY(dev_malloc(&t->rl_buf, want));
   t->rl_bytes = want;
   return HM_OK;
 }
@@ -391,13 +391,13 @@ int rebuild_inner(hm_tree* t, hipStream_t s) {
       return set_err(HM_EBUDGET, "inner levels need %llu more bytes than the budget allows",
                      (unsigned long long)extra);
     HM_TRY(hipStreamSynchronize(s));
-    if (t->d_inner) HM_TRY(hipFree(t->d_inner));
-    if (t->d_prefix) HM_TRY(hipFree(t->d_prefix));
+    HM_TRY(dev_free(t->d_inner));
+    HM_TRY(dev_free(t->d_prefix));
     t->d_inner = nullptr;
     t->d_prefix = nullptr;
     const uint32_t cap = lv.n_inner + lv.n_inner / 8 + 8;
-    HM_TRY(hipMalloc(&t->d_inner, (size_t)cap * t->NS * 8));
-    HM_TRY(hipMalloc(&t->d_prefix, (size_t)cap * 4));
+    HM_TRY(dev_malloc(&t->d_inner, (size_t)cap * t->NS * 8));
+    HM_TRY(dev_malloc(&t->d_prefix, (size_t)cap * 4));
     t->inner_cap = cap;
   }
   int rc = ensure_rl(t, inner_scratch_bytes(t->n_leaves, t->F, lv.n_inner), s);
@@ -414,24 +414,25 @@ void free_tree(hm_tree* t) {
   if (t->own) (void)hipStreamSynchronize(t->own);
   for (hipStream_t h : t->hs)
     if (h) (void)hipStreamSynchronize(h);
+  (void)hipDeviceSynchronize();  // work on any stream may still use the arrays
   for (auto& kv : t->ws) {
-    if (kv.second.buf) (void)hipFree(kv.second.buf);
+    (void)dev_free(kv.second.buf, true);
     if (kv.second.last_use) (void)hipEventDestroy(kv.second.last_use);
   }
-  if (t->d_inner) (void)hipFree(t->d_inner);
-  if (t->d_prefix) (void)hipFree(t->d_prefix);
-  if (t->d_leaves) (void)hipFree(t->d_leaves);
-  if (t->pend_k) (void)hipFree(t->pend_k);
-  if (t->pend_v) (void)hipFree(t->pend_v);
-  if (t->upd_buf) (void)hipFree(t->upd_buf);
+  (void)dev_free(t->d_inner, true);
+  (void)dev_free(t->d_prefix, true);
+  (void)dev_free(t->d_leaves, true);
+  (void)dev_free(t->pend_k, true);
+  (void)dev_free(t->pend_v, true);
+  (void)dev_free(t->upd_buf, true);
   if (t->upd_host) (void)hipHostFree(t->upd_host);
   if (t->pin_stage) (void)hipHostFree(t->pin_stage);
   if (t->stage_ev) (void)hipEventDestroy(t->stage_ev);
-  if (t->sb_leaves) (void)hipFree(t->sb_leaves);
-  if (t->sb_inner) (void)hipFree(t->sb_inner);
-  if (t->sb_prefix) (void)hipFree(t->sb_prefix);
-  if (t->rl_buf) (void)hipFree(t->rl_buf);
-  if (t->bl_child) (void)hipFree(t->bl_child);
+  (void)dev_free(t->sb_leaves, true);
+  (void)dev_free(t->sb_inner, true);
+  (void)dev_free(t->sb_prefix, true);
+  (void)dev_free(t->rl_buf, true);
+  (void)dev_free(t->bl_child, true);
   for (int k = 0; k < 2; ++k) {
     if (t->hs_stage[k]) (void)hipHostFree(t->hs_stage[k]);
     if (t->hs_ev[k]) (void)hipEventDestroy(t->hs_ev[k]);
@@ -439,7 +440,7 @@ void free_tree(hm_tree* t) {
   }
   if (t->publish_ev) (void)hipEventDestroy(t->publish_ev);
   if (t->na_ev) (void)hipEventDestroy(t->na_ev);
-  if (t->own) (void)hipStreamDestroy(t->own);
+  if (t->own) stream_give(t->own, t->device);
   delete t;
 }
 
@@ -487,7 +488,7 @@ static int create_tree(const hm_params* p, hm_tree** out) {
   int rc = HM_OK;
   if (hipGetDevice(&t->device) != hipSuccess)
     rc = set_err(HM_EDEVICE, "no HIP device");
-  else if (hipStreamCreateWithFlags(&t->own, hipStreamNonBlocking) != hipSuccess)
+  else if (stream_take(&t->own) != hipSuccess)
     rc = set_err(HM_EDEVICE, "hipStreamCreate failed");
   else if (hipEventCreateWithFlags(&t->publish_ev, hipEventDisableTiming) != hipSuccess ||
            hipEventCreateWithFlags(&t->na_ev, hipEventDisableTiming) != hipSuccess)
@@ -529,16 +530,22 @@ int hm_tree_build(const uint64_t* keys, const uint64_t* vals, uint64_t n, const 
                           (unsigned long long)p->mem_budget));
   }
 
-  // stage input, sort (key, value) pairs, validate
-  uint64_t *k_in = nullptr, *v_in = nullptr, *k0 = nullptr, *v0 = nullptr, *k1 = nullptr, *v1 = nullptr;
-  void* tmp = nullptr;
-  uint32_t* d_flags = nullptr;
-  uint64_t* d_orand = nullptr;
+  // Stage the input, sort (key, value) pairs, validate.  One scratch block holds everything that ends with
+  // the call; the sort's second pair of buffers is the leaf array, which is filled from the first pair
+  // afterwards.
+  struct Summary {  // device words, zeroed; read back in two copies
+    uint64_t key_or, key_nor;  // or of the keys, or of their complements
+    uint32_t flags, pad;
+    uint64_t edge[2];
+  };
+  const bool hk = n > 0 && !is_device_ptr(keys), hv = n > 0 && !is_device_ptr(vals);
+  const bool unsorted = n > 1 && !(p->flags & HM_FLAG_KEYS_SORTED);
+  const size_t nb = align256(std::max<uint64_t>(n, 1) * 8);
+  const bool fits = t->leaf_cap * sizeof(Leaf) >= 2 * nb;  // (a tree of one or two leaves may be smaller)
+  char* scratch = nullptr;
   auto cleanup = [&]() {
     (void)hipStreamSynchronize(s);
-    for (void* q : {(void*)k_in, (void*)v_in, (void*)k0, (void*)v0, (void*)k1, (void*)v1, tmp, (void*)d_flags,
-                    (void*)d_orand})
-      if (q) (void)hipFree(q);
+    (void)dev_free(scratch, true);
   };
 #define BUILD_TRY(expr)            \
   do {                             \
@@ -552,63 +559,68 @@ int hm_tree_build(const uint64_t* keys, const uint64_t* vals, uint64_t n, const 
     }                              \
   } while (0)
 
-  const size_t nb = std::max<uint64_t>(n, 1) * 8;
   const uint64_t* dk = keys;
   const uint64_t* dv = vals;
-  BUILD_TRY(hipMalloc(&d_flags, 256));
-  BUILD_TRY(hipMalloc(&d_orand, 256));
-  BUILD_TRY(hipMemsetAsync(d_flags, 0, 256, s));
-  if (n > 0 && !is_device_ptr(keys)) {
-    BUILD_TRY(hipMalloc(&k_in, nb));
-    BUILD_TRY(hipMemcpyAsync(k_in, keys, n * 8, hipMemcpyHostToDevice, s));
-    dk = k_in;
+  const size_t need = 256 + (hk ? nb : 0) + (hv ? nb : 0) +
+                      (unsorted ? 2 * nb + (fits ? 0 : 2 * nb) + align256(radix_tmp_bytes(n)) : 0);
+  BUILD_TRY(dev_malloc(&scratch, need));
+  BUILD_TRY(dev_malloc(&t->d_leaves, t->leaf_cap * sizeof(Leaf)));
+  char* cur = scratch;
+  auto take = [&](size_t b) {
+    char* r = cur;
+    cur += b;
+    return r;
+  };
+  Summary* d_sum = (Summary*)take(256);
+  Summary sum{};
+  BUILD_TRY(hipMemsetAsync(d_sum, 0, 256, s));
+  if (hk) {
+    uint64_t* b = (uint64_t*)take(nb);
+    BUILD_TRY(hipMemcpyAsync(b, keys, n * 8, hipMemcpyHostToDevice, s));
+    dk = b;
   }
-  if (n > 0 && !is_device_ptr(vals)) {
-    BUILD_TRY(hipMalloc(&v_in, nb));
-    BUILD_TRY(hipMemcpyAsync(v_in, vals, n * 8, hipMemcpyHostToDevice, s));
-    dv = v_in;
+  if (hv) {
+    uint64_t* b = (uint64_t*)take(nb);
+    BUILD_TRY(hipMemcpyAsync(b, vals, n * 8, hipMemcpyHostToDevice, s));
+    dv = b;
   }
-  if (n > 1 && !(p->flags & HM_FLAG_KEYS_SORTED)) {
-    uint64_t orand_init[2] = {0ull, ~0ull}, orand[2];
-    BUILD_TRY(hipMemcpyAsync(d_orand, orand_init, 16, hipMemcpyHostToDevice, s));
-    BUILD_TRY(key_bit_summary(dk, n, d_orand, s));
-    BUILD_TRY(hipMemcpyAsync(orand, d_orand, 16, hipMemcpyDeviceToHost, s));
+  if (unsorted) {
+    BUILD_TRY(key_bit_summary(dk, n, &d_sum->key_or, s));
+    BUILD_TRY(hipMemcpyAsync(&sum, d_sum, sizeof(Summary), hipMemcpyDeviceToHost, s));
     BUILD_TRY(hipStreamSynchronize(s));
-    const uint64_t varying = orand[0] ^ orand[1];
+    const uint64_t varying = sum.key_or & sum.key_nor;  // bits that are set in some key and clear in another
     if (varying) {
       const int lo = (__builtin_ctzll(varying) / 8) * 8;
       const int hi = 64 - __builtin_clzll(varying);
-      BUILD_TRY(hipMalloc(&k0, nb));
-      BUILD_TRY(hipMalloc(&v0, nb));
-      BUILD_TRY(hipMalloc(&k1, nb));
-      BUILD_TRY(hipMalloc(&v1, nb));
-      BUILD_TRY(hipMalloc(&tmp, radix_tmp_bytes(n)));
+      uint64_t* a0 = (uint64_t*)take(nb);
+      uint64_t* a1 = (uint64_t*)take(nb);
+      uint64_t* b0 = fits ? (uint64_t*)t->d_leaves : (uint64_t*)take(nb);
+      uint64_t* b1 = fits ? (uint64_t*)((char*)t->d_leaves + nb) : (uint64_t*)take(nb);
+      void* tmp = take(align256(radix_tmp_bytes(n)));
       int which = 0;
-      BUILD_TRY(radix_sort_u64pay(dk, dv, n, lo, hi, k0, v0, k1, v1, tmp, s, &which));
-      dk = which ? k1 : k0;
-      dv = which ? v1 : v0;
+      // an even number of passes ends in the second pair it is given, an odd one in the first: (a0, a1)
+      const bool even = ((hi - lo + 7) / 8) % 2 == 0;
+      BUILD_TRY(radix_sort_u64pay(dk, dv, n, lo, hi, even ? b0 : a0, even ? b1 : a1, even ? a0 : b0, even ? a1 : b1, tmp,
+                                  s, &which));
+      dk = a0;
+      dv = a1;
     }
   }
-  uint32_t flags = 0;
   uint64_t edge[2] = {~0ull, 0ull};
-  BUILD_TRY(validate_sorted(dk, n, d_flags, s));
-  BUILD_TRY(hipMemcpyAsync(&flags, d_flags, 4, hipMemcpyDeviceToHost, s));
-  if (n) {
-    BUILD_TRY(hipMemcpyAsync(&edge[0], dk, 8, hipMemcpyDeviceToHost, s));
-    BUILD_TRY(hipMemcpyAsync(&edge[1], dk + n - 1, 8, hipMemcpyDeviceToHost, s));
-  }
+  BUILD_TRY(validate_sorted(dk, n, &d_sum->flags, d_sum->edge, s));
+  BUILD_TRY(hipMemcpyAsync(&sum, d_sum, sizeof(Summary), hipMemcpyDeviceToHost, s));
   BUILD_TRY(hipStreamSynchronize(s));
-  if (flags & 1u) {
+  if (n) edge[0] = sum.edge[0], edge[1] = sum.edge[1];
+  if (sum.flags & 1u) {
     cleanup();
     return fail(set_err(HM_EINVAL, "key 0xFFFFFFFFFFFFFFFF is reserved for padding"));
   }
-  if (flags & 2u) {
+  if (sum.flags & 2u) {
     cleanup();
     return fail(set_err(HM_EINVAL, (p->flags & HM_FLAG_KEYS_SORTED) ? "keys flagged sorted are not strictly ascending"
                                                                      : "duplicate keys in build input"));
   }
   t->widen_key_range(edge[0], edge[1]);
-  BUILD_TRY(hipMalloc(&t->d_leaves, t->leaf_cap * sizeof(Leaf)));
   BUILD_TRY(fill_leaves(dk, dv, n, t->fill, t->d_leaves, t->n_leaves, s));
   {
     int r = rebuild_inner(t, s);
@@ -842,11 +854,11 @@ int hm_baseline_search(hm_tree* t, int kind, uint32_t group_size, const uint64_t
       return set_err(HM_EBUDGET, "baseline child array exceeds the device-memory budget");
     if (t->bl_child) {
       HM_TRY(hipDeviceSynchronize());  // searches on any stream may still read it
-      HM_TRY(hipFree(t->bl_child));
+      HM_TRY(dev_free(t->bl_child));
       t->bl_child = nullptr;
       t->bl_cap = 0;
     }
-    HM_TRY(hipMalloc(&t->bl_child, need * 4));
+    HM_TRY(dev_malloc(&t->bl_child, need * 4));
     t->bl_cap = need;
     t->bl_version = ~0ull;
   }
@@ -1027,11 +1039,11 @@ static int ensure_upd(hm_tree* t, size_t n, hipStream_t s) {
     return set_err(HM_EBUDGET, "update scratch for %llu keys exceeds the device-memory budget", (unsigned long long)n);
   if (t->upd_buf) {
     HM_TRY(hipStreamSynchronize(s));
-    HM_TRY(hipFree(t->upd_buf));
+    HM_TRY(dev_free(t->upd_buf));
     t->upd_buf = nullptr;
     t->upd_bytes = 0;
   }
-  HM_TRY(hipMalloc(&t->upd_buf, want));
+  HM_TRY(dev_malloc(&t->upd_buf, want));
   t->upd_bytes = want;
   return HM_OK;
 }
@@ -1071,16 +1083,16 @@ int stage_updates(hm_tree* t, const uint64_t* keys, const uint64_t* vals, uint64
     if (t->p.mem_budget && t->device_bytes() + (cap - t->pend_cap) * 16 > t->p.mem_budget)
       return set_err(HM_EBUDGET, "staging %llu updates exceeds the device-memory budget", (unsigned long long)n);
     uint64_t *nk = nullptr, *nv = nullptr;
-    HM_TRY(hipMalloc(&nk, cap * 8));
-    HM_TRY(hipMalloc(&nv, cap * 8));
+    HM_TRY(dev_malloc(&nk, cap * 8));
+    HM_TRY(dev_malloc(&nv, cap * 8));
     if (t->pend_n) {
       if (t->stage_valid) HM_TRY(hipStreamWaitEvent(s, t->stage_ev, 0));  // staged on other streams
       HM_TRY(copy_words(nk, t->pend_k, t->pend_n, s));
       HM_TRY(copy_words(nv, t->pend_v, t->pend_n, s));
     }
     HM_TRY(hipStreamSynchronize(s));
-    if (t->pend_k) HM_TRY(hipFree(t->pend_k));
-    if (t->pend_v) HM_TRY(hipFree(t->pend_v));
+    HM_TRY(dev_free(t->pend_k));
+    HM_TRY(dev_free(t->pend_v));
     t->pend_k = nk;
     t->pend_v = nv;
     t->pend_cap = cap;
@@ -1248,10 +1260,10 @@ int publish_prepare(hm_tree* t, hipStream_t s, PublishPlan* plan) {
                    (unsigned long long)new_leaves);
   if (ib_need > t->rl_bytes) {  // not expected (sized above); keep the counts: grow and copy them over
     void* nb = nullptr;
-    HM_TRY(hipMalloc(&nb, ib_need));
+    HM_TRY(dev_malloc(&nb, ib_need));
     HM_TRY(copy_words((uint64_t*)nb, (const uint64_t*)t->rl_buf, ib_off / 8, s));
     HM_TRY(hipStreamSynchronize(s));
-    HM_TRY(hipFree(t->rl_buf));
+    HM_TRY(dev_free(t->rl_buf));
     t->rl_buf = nb;
     t->rl_bytes = ib_need;
     cur = (char*)t->rl_buf;
@@ -1261,21 +1273,21 @@ int publish_prepare(hm_tree* t, hipStream_t s, PublishPlan* plan) {
   }
   if (leaf_cap != t->sb_leaf_cap) {
     HM_TRY(hipStreamSynchronize(s));
-    if (t->sb_leaves) HM_TRY(hipFree(t->sb_leaves));
+    HM_TRY(dev_free(t->sb_leaves));
     t->sb_leaves = nullptr;
     t->sb_leaf_cap = 0;
-    HM_TRY(hipMalloc(&t->sb_leaves, leaf_cap * sizeof(Leaf)));
+    HM_TRY(dev_malloc(&t->sb_leaves, leaf_cap * sizeof(Leaf)));
     t->sb_leaf_cap = leaf_cap;
   }
   if (inner_cap != t->sb_inner_cap) {
     HM_TRY(hipStreamSynchronize(s));
-    if (t->sb_inner) HM_TRY(hipFree(t->sb_inner));
-    if (t->sb_prefix) HM_TRY(hipFree(t->sb_prefix));
+    HM_TRY(dev_free(t->sb_inner));
+    HM_TRY(dev_free(t->sb_prefix));
     t->sb_inner = nullptr;
     t->sb_prefix = nullptr;
     t->sb_inner_cap = 0;
-    HM_TRY(hipMalloc(&t->sb_inner, (size_t)inner_cap * t->NS * 8));
-    HM_TRY(hipMalloc(&t->sb_prefix, (size_t)inner_cap * 4));
+    HM_TRY(dev_malloc(&t->sb_inner, (size_t)inner_cap * t->NS * 8));
+    HM_TRY(dev_malloc(&t->sb_prefix, (size_t)inner_cap * 4));
     t->sb_inner_cap = inner_cap;
   }
   // the standby arrays were the active ones before the last swap: searches issued before it may
@@ -1314,15 +1326,15 @@ int reserve_updates(hm_tree* t, size_t n, hipStream_t s) {
     if (t->p.mem_budget && t->device_bytes() + (n - t->pend_cap) * 16 > t->p.mem_budget)
       return set_err(HM_EBUDGET, "update staging exceeds the device-memory budget");
     uint64_t *nk = nullptr, *nv = nullptr;
-    HM_TRY(hipMalloc(&nk, n * 8));
-    HM_TRY(hipMalloc(&nv, n * 8));
+    HM_TRY(dev_malloc(&nk, n * 8));
+    HM_TRY(dev_malloc(&nv, n * 8));
     if (t->pend_n) {
       HM_TRY(hipMemcpyAsync(nk, t->pend_k, t->pend_n * 8, hipMemcpyDeviceToDevice, s));
       HM_TRY(hipMemcpyAsync(nv, t->pend_v, t->pend_n * 8, hipMemcpyDeviceToDevice, s));
     }
     HM_TRY(hipStreamSynchronize(s));
-    if (t->pend_k) HM_TRY(hipFree(t->pend_k));
-    if (t->pend_v) HM_TRY(hipFree(t->pend_v));
+    HM_TRY(dev_free(t->pend_k));
+    HM_TRY(dev_free(t->pend_v));
     t->pend_k = nk;
     t->pend_v = nv;
     t->pend_cap = n;
@@ -1350,20 +1362,20 @@ int reserve_relayout(hm_tree* t, hipStream_t s) {
     return set_err(HM_EBUDGET, "no room for a standby layout under the memory budget");
   HM_TRY(hipStreamSynchronize(s));
   if (t->sb_leaf_cap < leaf_cap) {
-    if (t->sb_leaves) HM_TRY(hipFree(t->sb_leaves));
+    HM_TRY(dev_free(t->sb_leaves));
     t->sb_leaves = nullptr;
     t->sb_leaf_cap = 0;
-    HM_TRY(hipMalloc(&t->sb_leaves, leaf_cap * sizeof(Leaf)));
+    HM_TRY(dev_malloc(&t->sb_leaves, leaf_cap * sizeof(Leaf)));
     t->sb_leaf_cap = leaf_cap;
   }
   if (t->sb_inner_cap < inner_cap) {
-    if (t->sb_inner) HM_TRY(hipFree(t->sb_inner));
-    if (t->sb_prefix) HM_TRY(hipFree(t->sb_prefix));
+    HM_TRY(dev_free(t->sb_inner));
+    HM_TRY(dev_free(t->sb_prefix));
     t->sb_inner = nullptr;
     t->sb_prefix = nullptr;
     t->sb_inner_cap = 0;
-    HM_TRY(hipMalloc(&t->sb_inner, (size_t)inner_cap * t->NS * 8));
-    HM_TRY(hipMalloc(&t->sb_prefix, (size_t)inner_cap * 4));
+    HM_TRY(dev_malloc(&t->sb_inner, (size_t)inner_cap * t->NS * 8));
+    HM_TRY(dev_malloc(&t->sb_prefix, (size_t)inner_cap * 4));
     t->sb_inner_cap = inner_cap;
   }
   return ensure_rl(t, rl, s);
@@ -1579,7 +1591,7 @@ static int tree_load_impl(const char* path, const hm_params* p, hm_tree** out) {
     free_tree(t);
     return code;
   };
-  if (hipMalloc(&t->d_leaves, t->leaf_cap * sizeof(Leaf)) != hipSuccess)
+  if (dev_malloc(&t->d_leaves, t->leaf_cap * sizeof(Leaf)) != hipSuccess)
     return fail(set_err(HM_ENOMEM, "leaf allocation failed"));
   if (hipMemcpy(t->d_leaves, leaves.data(), leaves.size() * 8, hipMemcpyHostToDevice) != hipSuccess)
     return fail(set_err(HM_EDEVICE, "leaf upload failed"));
@@ -1667,12 +1679,12 @@ int hm_psa_sort(const uint64_t* keys, uint64_t n, int begin_bit, int end_bit, ui
     ~Scratch() {
       if (p) {
         (void)hipStreamSynchronize(s);
-        (void)hipFree(p);
+        (void)dev_free(p, true);
       }
     }
   } scratch;
   scratch.s = s;
-  HM_TRY(hipMalloc(&scratch.p, 3 * kq + 2 * kp + align256(radix_tmp_bytes(n))));
+  HM_TRY(dev_malloc(&scratch.p, 3 * kq + 2 * kp + align256(radix_tmp_bytes(n))));
   char* cur = scratch.p;
   const uint64_t* dk = keys;
   if (!is_device_ptr(keys)) {
@@ -1734,6 +1746,7 @@ int hm_profile_get(const char* stage, double* total_ms, uint64_t* launches) {
 
 int hm_device_synchronize(void) {
   HM_TRY(hipDeviceSynchronize());
+  dev_pool_trim();
   return HM_OK;
 }
 

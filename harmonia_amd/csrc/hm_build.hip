@@ -20,8 +20,10 @@ constexpr int kReduceBlocks = 4096;
 constexpr int kUnroll = 4;  // independent loads in flight per thread
 
 __global__ __launch_bounds__(256) void validate_sorted_kernel(const uint64_t* __restrict__ k, size_t n,
-                                                              uint32_t* __restrict__ flags) {
+                                                              uint32_t* __restrict__ flags,
+                                                              uint64_t* __restrict__ edge) {
   __shared__ uint32_t block_f;
+  if (blockIdx.x == 0 && threadIdx.x < 2) edge[threadIdx.x] = k[threadIdx.x == 0 ? 0 : n - 1];
   if (threadIdx.x == 0) block_f = 0;
   __syncthreads();
   const size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -50,42 +52,37 @@ __global__ __launch_bounds__(256) void validate_sorted_kernel(const uint64_t* __
   if (threadIdx.x == 0 && block_f) atomicOr(flags, block_f);
 }
 
+// ornor[0] |= or of the keys, ornor[1] |= or of their complements: the bits set in both vary.
 __global__ __launch_bounds__(256) void key_bits_kernel(const uint64_t* __restrict__ k, size_t n,
-                                                       uint64_t* __restrict__ orand) {
-  __shared__ unsigned long long block_o, block_a;
-  if (threadIdx.x == 0) {
-    block_o = 0ull;
-    block_a = ~0ull;
-  }
+                                                       uint64_t* __restrict__ ornor) {
+  __shared__ unsigned long long block_o[2];
+  if (threadIdx.x < 2) block_o[threadIdx.x] = 0ull;
   __syncthreads();
   const size_t stride = (size_t)gridDim.x * blockDim.x;
-  uint64_t o = 0, a = ~0ull;
+  uint64_t o = 0, c = 0;
   for (size_t b = (size_t)blockIdx.x * blockDim.x + threadIdx.x; b < n; b += kUnroll * stride) {
     uint64_t x[kUnroll];
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       const size_t i = b + u * stride;
-      x[u] = i < n ? k[i] : k[b];  // k[b] leaves the or / and unchanged
+      x[u] = i < n ? k[i] : k[b];  // k[b] again changes nothing
     }
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       o |= x[u];
-      a &= x[u];
+      c |= ~x[u];
     }
   }
   for (int off = 32; off > 0; off >>= 1) {
     o |= __shfl_xor(o, off, 64);
-    a &= __shfl_xor(a, off, 64);
+    c |= __shfl_xor(c, off, 64);
   }
   if ((threadIdx.x & 63) == 0) {
-    atomicOr(&block_o, (unsigned long long)o);
-    atomicAnd(&block_a, (unsigned long long)a);
+    atomicOr(&block_o[0], (unsigned long long)o);
+    atomicOr(&block_o[1], (unsigned long long)c);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    atomicOr((unsigned long long*)&orand[0], block_o);
-    atomicAnd((unsigned long long*)&orand[1], block_a);
-  }
+  if (threadIdx.x < 2) atomicOr((unsigned long long*)&ornor[threadIdx.x], block_o[threadIdx.x]);
 }
 
 __global__ void fill_leaves_kernel(const uint64_t* __restrict__ keys, const uint64_t* __restrict__ vals, size_t n,
@@ -157,21 +154,21 @@ int grid_for(size_t work, int threads) {
 
 }  // namespace
 
-hipError_t validate_sorted(const uint64_t* keys, size_t n, uint32_t* d_flags, hipStream_t s) {
+hipError_t validate_sorted(const uint64_t* keys, size_t n, uint32_t* d_flags, uint64_t* edge, hipStream_t s) {
   if (n == 0) return hipSuccess;
   ProfScope prof("build", s);
   int g = grid_for(n, 256);
   if (g > kReduceBlocks) g = kReduceBlocks;
-  hipLaunchKernelGGL(validate_sorted_kernel, dim3(g), dim3(256), 0, s, keys, n, d_flags);
+  hipLaunchKernelGGL(validate_sorted_kernel, dim3(g), dim3(256), 0, s, keys, n, d_flags, edge);
   return hipGetLastError();
 }
 
-hipError_t key_bit_summary(const uint64_t* keys, size_t n, uint64_t* d_orand, hipStream_t s) {
+hipError_t key_bit_summary(const uint64_t* keys, size_t n, uint64_t* ornor, hipStream_t s) {
   if (n == 0) return hipSuccess;
   ProfScope prof("build", s);
   int g = grid_for(n, 256);
   if (g > kReduceBlocks) g = kReduceBlocks;
-  hipLaunchKernelGGL(key_bits_kernel, dim3(g), dim3(256), 0, s, keys, n, d_orand);
+  hipLaunchKernelGGL(key_bits_kernel, dim3(g), dim3(256), 0, s, keys, n, ornor);
   return hipGetLastError();
 }
 

@@ -121,10 +121,12 @@ hipError_t unpartition_results(const uint64_t* vals, const uint8_t* found, size_
                                uint64_t* out_vals, uint8_t* out_found, hipStream_t s, const uint32_t* dn);
 
 // ---- build (hm_build.hip) --------------------------------------------------------------
-// flags |= 1 if a key is KEY_MAX, |= 2 if keys are not strictly ascending.
-hipError_t validate_sorted(const uint64_t* keys, size_t n, uint32_t* d_flags, hipStream_t s);
-// OR / AND over keys (to skip radix passes whose digit is constant).
-hipError_t key_bit_summary(const uint64_t* keys, size_t n, uint64_t* d_orand /*2 u64*/, hipStream_t s);
+// flags |= 1 if a key is KEY_MAX, |= 2 if keys are not strictly ascending; edge[0], edge[1] = the first and
+// last key.
+hipError_t validate_sorted(const uint64_t* keys, size_t n, uint32_t* d_flags, uint64_t* edge, hipStream_t s);
+// ornor[0] |= the or of the keys, ornor[1] |= the or of their complements (to skip radix passes whose digit
+// is constant).
+hipError_t key_bit_summary(const uint64_t* keys, size_t n, uint64_t* ornor, hipStream_t s);
 hipError_t fill_leaves(const uint64_t* keys, const uint64_t* vals, size_t n, int fill, Leaf* leaves, size_t n_leaves,
                        hipStream_t s);
 // Leaf minimum keys (KEY_MAX for an empty leaf) -> child_min.

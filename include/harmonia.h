@@ -323,6 +323,8 @@ int hm_profile_reset(void);
 /* stage: "search", "psa_hist", "psa_scatter", "scan", "range", "build", "update" ... */
 int hm_profile_get(const char* stage, double* total_ms, uint64_t* launches);
 
+/* Wait for the device, and give back to the driver the device memory that destroyed trees left for reuse
+ * (at most 512 MiB per device). */
 int hm_device_synchronize(void);
 int hm_last_error(char* buf, uint64_t len);
 
