@@ -380,13 +380,13 @@ void set_levels(hm_tree* t, const Levels& lv) {
   t->layout_version++;  // captured pipelines hold the old pointers and level table
 }
 
-// Rebuild every inner level and the prefix array of the active leaves in place (build / load).
-int rebuild_inner(hm_tree* t, hipStream_t s) {
-  Levels lv;
-  lv.height = plan_levels(t->n_leaves, t->F, lv.level_start, &lv.n_inner);
-  if (lv.height < 0) return set_err(HM_EINVAL, "tree would exceed %d levels", MAX_LEVELS);
-  if (lv.n_inner > t->inner_cap) {
-    const uint64_t extra = (uint64_t)(lv.n_inner - t->inner_cap) * (t->NS * 8 + 4);
+// Room for every inner level and the prefix array of the active leaves (build / load), and for the scratch
+// of building them, whose first array takes the leaf minima.
+int prepare_inner(hm_tree* t, Levels* lv, hipStream_t s) {
+  lv->height = plan_levels(t->n_leaves, t->F, lv->level_start, &lv->n_inner);
+  if (lv->height < 0) return set_err(HM_EINVAL, "tree would exceed %d levels", MAX_LEVELS);
+  if (lv->n_inner > t->inner_cap) {
+    const uint64_t extra = (uint64_t)(lv->n_inner - t->inner_cap) * (t->NS * 8 + 4);
     if (t->p.mem_budget && t->device_bytes() + extra > t->p.mem_budget)
       return set_err(HM_EBUDGET, "inner levels need %llu more bytes than the budget allows",
                      (unsigned long long)extra);
@@ -395,14 +395,17 @@ int rebuild_inner(hm_tree* t, hipStream_t s) {
     HM_TRY(dev_free(t->d_prefix));
     t->d_inner = nullptr;
     t->d_prefix = nullptr;
-    const uint32_t cap = lv.n_inner + lv.n_inner / 8 + 8;
+    const uint32_t cap = lv->n_inner + lv->n_inner / 8 + 8;
     HM_TRY(dev_malloc(&t->d_inner, (size_t)cap * t->NS * 8));
     HM_TRY(dev_malloc(&t->d_prefix, (size_t)cap * 4));
     t->inner_cap = cap;
   }
-  int rc = ensure_rl(t, inner_scratch_bytes(t->n_leaves, t->F, lv.n_inner), s);
-  if (rc) return rc;
-  rc = build_inner_into(t, t->d_leaves, t->n_leaves, t->d_inner, t->d_prefix, lv, 0, s, false);
+  return ensure_rl(t, inner_scratch_bytes(t->n_leaves, t->F, lv->n_inner), s);
+}
+
+// Every inner level and the prefix array of the active leaves, in place, after prepare_inner.
+int rebuild_inner(hm_tree* t, const Levels& lv, bool mins_ready, hipStream_t s) {
+  int rc = build_inner_into(t, t->d_leaves, t->n_leaves, t->d_inner, t->d_prefix, lv, 0, s, mins_ready);
   if (rc) return rc;
   HM_TRY(hipStreamSynchronize(s));
   set_levels(t, lv);
@@ -535,9 +538,10 @@ int hm_tree_build(const uint64_t* keys, const uint64_t* vals, uint64_t n, const 
   // afterwards.
   struct Summary {  // device words, zeroed; read back in two copies
     uint64_t key_or, key_nor;  // or of the keys, or of their complements
-    uint32_t flags, pad;
+    uint32_t flags, pad;        // 1: a key is KEY_MAX, 2: equal keys, kCrowded
     uint64_t edge[2];
   };
+  constexpr uint32_t kCrowded = 4;  // a bucket holds more pairs than a block sorts
   const bool hk = n > 0 && !is_device_ptr(keys), hv = n > 0 && !is_device_ptr(vals);
   const bool unsorted = n > 1 && !(p->flags & HM_FLAG_KEYS_SORTED);
   const size_t nb = align256(std::max<uint64_t>(n, 1) * 8);
@@ -561,10 +565,21 @@ int hm_tree_build(const uint64_t* keys, const uint64_t* vals, uint64_t n, const 
 
   const uint64_t* dk = keys;
   const uint64_t* dv = vals;
-  const size_t need = 256 + (hk ? nb : 0) + (hv ? nb : 0) +
-                      (unsorted ? 2 * nb + (fits ? 0 : 2 * nb) + align256(radix_tmp_bytes(n)) : 0);
+  // Unsorted pairs go to buckets that one block each can sort (uniform keys, up to 9.4 million of them); more
+  // pairs, or keys that crowd into few buckets, go through the radix sort of every varying byte.
+  const int bbits = unsorted ? pair_bits(n) : 0;
+  const size_t tmp_bytes =
+      unsorted ? std::max(align256(radix_tmp_bytes(n)), bbits ? align256(partition_pairs_bytes(n)) : 0) : 0;
+  const size_t need =
+      256 + (hk ? nb : 0) + (hv ? nb : 0) + (unsorted ? 2 * nb + (fits ? 0 : 2 * nb) + tmp_bytes : 0);
   BUILD_TRY(dev_malloc(&scratch, need));
   BUILD_TRY(dev_malloc(&t->d_leaves, t->leaf_cap * sizeof(Leaf)));
+  Levels lv;
+  if ((rc = prepare_inner(t, &lv, s))) {
+    cleanup();
+    return fail(rc);
+  }
+  uint64_t* mins = (uint64_t*)t->rl_buf;
   char* cur = scratch;
   auto take = [&](size_t b) {
     char* r = cur;
@@ -584,6 +599,7 @@ int hm_tree_build(const uint64_t* keys, const uint64_t* vals, uint64_t n, const 
     BUILD_TRY(hipMemcpyAsync(b, vals, n * 8, hipMemcpyHostToDevice, s));
     dv = b;
   }
+  bool filled = false;
   if (unsorted) {
     BUILD_TRY(key_bit_summary(dk, n, &d_sum->key_or, s));
     BUILD_TRY(hipMemcpyAsync(&sum, d_sum, sizeof(Summary), hipMemcpyDeviceToHost, s));
@@ -596,20 +612,33 @@ int hm_tree_build(const uint64_t* keys, const uint64_t* vals, uint64_t n, const 
       uint64_t* a1 = (uint64_t*)take(nb);
       uint64_t* b0 = fits ? (uint64_t*)t->d_leaves : (uint64_t*)take(nb);
       uint64_t* b1 = fits ? (uint64_t*)((char*)t->d_leaves + nb) : (uint64_t*)take(nb);
-      void* tmp = take(align256(radix_tmp_bytes(n)));
-      int which = 0;
-      // an even number of passes ends in the second pair it is given, an odd one in the first: (a0, a1)
-      const bool even = ((hi - lo + 7) / 8) % 2 == 0;
-      BUILD_TRY(radix_sort_u64pay(dk, dv, n, lo, hi, even ? b0 : a0, even ? b1 : a1, even ? a0 : b0, even ? a1 : b1, tmp,
-                                  s, &which));
-      dk = a0;
-      dv = a1;
+      void* tmp = take(tmp_bytes);
+      if (bbits) {
+        const uint32_t* totals = nullptr;
+        BUILD_TRY(partition_pairs(dk, dv, n, hi, a0, a1, tmp, &d_sum->flags, kCrowded, &totals, s));
+        BUILD_TRY(bucket_sort_fill(a0, a1, n, bbits, totals, t->fill, t->d_leaves, mins, &d_sum->flags, kCrowded,
+                                   d_sum->edge, s));
+        BUILD_TRY(hipMemcpyAsync(&sum, d_sum, sizeof(Summary), hipMemcpyDeviceToHost, s));
+        BUILD_TRY(hipStreamSynchronize(s));
+        filled = !(sum.flags & kCrowded);
+      }
+      if (!filled) {
+        int which = 0;
+        // an even number of passes ends in the second pair it is given, an odd one in the first: (a0, a1)
+        const bool even = ((hi - lo + 7) / 8) % 2 == 0;
+        BUILD_TRY(radix_sort_u64pay(dk, dv, n, lo, hi, even ? b0 : a0, even ? b1 : a1, even ? a0 : b0, even ? a1 : b1,
+                                    tmp, s, &which));
+        dk = a0;
+        dv = a1;
+      }
     }
   }
   uint64_t edge[2] = {~0ull, 0ull};
-  BUILD_TRY(validate_sorted(dk, n, &d_sum->flags, d_sum->edge, s));
-  BUILD_TRY(hipMemcpyAsync(&sum, d_sum, sizeof(Summary), hipMemcpyDeviceToHost, s));
-  BUILD_TRY(hipStreamSynchronize(s));
+  if (!filled) {
+    BUILD_TRY(validate_sorted(dk, n, &d_sum->flags, d_sum->edge, s));
+    BUILD_TRY(hipMemcpyAsync(&sum, d_sum, sizeof(Summary), hipMemcpyDeviceToHost, s));
+    BUILD_TRY(hipStreamSynchronize(s));
+  }
   if (n) edge[0] = sum.edge[0], edge[1] = sum.edge[1];
   if (sum.flags & 1u) {
     cleanup();
@@ -621,9 +650,9 @@ int hm_tree_build(const uint64_t* keys, const uint64_t* vals, uint64_t n, const 
                                                                      : "duplicate keys in build input"));
   }
   t->widen_key_range(edge[0], edge[1]);
-  BUILD_TRY(fill_leaves(dk, dv, n, t->fill, t->d_leaves, t->n_leaves, s));
+  if (!filled) BUILD_TRY(fill_leaves(dk, dv, n, t->fill, t->d_leaves, t->n_leaves, mins, s));
   {
-    int r = rebuild_inner(t, s);
+    int r = rebuild_inner(t, lv, true, s);
     if (r) {
       cleanup();
       return fail(r);
@@ -1595,7 +1624,9 @@ static int tree_load_impl(const char* path, const hm_params* p, hm_tree** out) {
     return fail(set_err(HM_ENOMEM, "leaf allocation failed"));
   if (hipMemcpy(t->d_leaves, leaves.data(), leaves.size() * 8, hipMemcpyHostToDevice) != hipSuccess)
     return fail(set_err(HM_EDEVICE, "leaf upload failed"));
-  rc = rebuild_inner(t, t->own);
+  Levels lv;
+  rc = prepare_inner(t, &lv, t->own);
+  if (!rc) rc = rebuild_inner(t, lv, false, t->own);
   if (rc) return fail(rc);
   // the stored inner levels and prefix must be the ones the leaves define
   if (t->n_inner != h.n_inner || (uint32_t)t->height != h.height ||

@@ -120,6 +120,17 @@ hipError_t partition_keys(const uint64_t* q, size_t n, int top, uint64_t* out, v
 hipError_t unpartition_results(const uint64_t* vals, const uint8_t* found, size_t n, const void* rec,
                                uint64_t* out_vals, uint8_t* out_found, hipStream_t s, const uint32_t* dn);
 
+// (key, value) pairs into buckets by the key bits [top - b, top), b = pair_bits(n) (0: too many pairs for
+// buckets of kPairBucket on average).  *totals = the 2^b bucket sizes (device).  A bucket above kBucketSortMax
+// sets `flag` in *flags, and the pairs are then not moved.  tmp: partition_pairs_bytes(n).
+constexpr uint32_t kBucketSortMax = 5120;
+constexpr int kPairBucket = 4608;  // 5120 is seven standard deviations above it for uniform keys
+int pair_bits(size_t n);
+size_t partition_pairs_bytes(size_t n);
+hipError_t partition_pairs(const uint64_t* keys, const uint64_t* vals, size_t n, int top, uint64_t* kout,
+                           uint64_t* vout, void* tmp, uint32_t* flags, uint32_t flag, const uint32_t** totals,
+                           hipStream_t s);
+
 // ---- build (hm_build.hip) --------------------------------------------------------------
 // flags |= 1 if a key is KEY_MAX, |= 2 if keys are not strictly ascending; edge[0], edge[1] = the first and
 // last key.
@@ -127,7 +138,9 @@ hipError_t validate_sorted(const uint64_t* keys, size_t n, uint32_t* d_flags, ui
 // ornor[0] |= the or of the keys, ornor[1] |= the or of their complements (to skip radix passes whose digit
 // is constant).
 hipError_t key_bit_summary(const uint64_t* keys, size_t n, uint64_t* ornor, hipStream_t s);
+// mins[leaf] = the leaf's smallest key (KEY_MAX for the one leaf of an empty tree).
 hipError_t fill_leaves(const uint64_t* keys, const uint64_t* vals, size_t n, int fill, Leaf* leaves, size_t n_leaves,
+                       uint64_t* mins,
                        hipStream_t s);
 // Leaf minimum keys (KEY_MAX for an empty leaf) -> child_min.
 hipError_t leaf_min_keys(const Leaf* leaves, size_t n_leaves, uint64_t* child_min, hipStream_t s);
@@ -242,6 +255,11 @@ hipError_t count_kept(const uint64_t* sorted_keys, size_t n, uint32_t* tile_kept
 // uv, the number of them to *dm.
 hipError_t compact_last(const uint64_t* sorted_keys, const uint32_t* index, const uint64_t* vals, size_t n,
                         const uint32_t* tile_kept, uint64_t* uk, uint64_t* uv, uint32_t* dm, hipStream_t s);
+// The buckets of partition_pairs sorted, one block each, straight into the leaves (and mins); flags |= 1 if a
+// key is KEY_MAX, |= 2 if two keys are equal; edge = the first and last key.  Nothing once *flags has `skip`.
+hipError_t bucket_sort_fill(const uint64_t* keys, const uint64_t* vals, size_t n, int bits, const uint32_t* totals,
+                            int fill, Leaf* leaves, uint64_t* mins, uint32_t* flags, uint32_t skip, uint64_t* edge,
+                            hipStream_t s);
 // Over the m located unique keys (sorted, so each leaf's keys form one run and each last-level
 // node's keys one range): counts the new keys; summary[0] |= 1 if some leaf would exceed
 // 8 keys.  Such a node goes on the re-spread list (nlist: pairs of node index within the last level and

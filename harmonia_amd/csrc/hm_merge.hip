@@ -74,6 +74,20 @@ __device__ __forceinline__ void put_eight(MergeLds<NT>& m, const uint64_t (&k)[k
   }
 }
 
+// A thread's eight keys: odd-even transposition, which moves no key past an equal one.
+__device__ __forceinline__ void sort_eight(uint64_t (&k)[kPer], uint32_t (&ix)[kPer]) {
+#pragma unroll
+  for (int p = 0; p < kPer; ++p)
+#pragma unroll
+    for (int r = p & 1; r + 1 < kPer; r += 2)
+      if (k[r] > k[r + 1]) {
+        const uint64_t x = k[r];
+        const uint32_t y = ix[r];
+        k[r] = k[r + 1], ix[r] = ix[r + 1];
+        k[r + 1] = x, ix[r + 1] = y;
+      }
+}
+
 // Chunk c of 4096 staged keys sorted by (key, index); block 0 zeroes the epoch's 8 summary words.
 __global__ __launch_bounds__(kChunkThreads) void chunk_sort_kernel(const uint64_t* __restrict__ pk, uint32_t n,
                                                                    uint64_t* __restrict__ ko,
@@ -90,17 +104,7 @@ __global__ __launch_bounds__(kChunkThreads) void chunk_sort_kernel(const uint64_
     k[r] = e0 + r < n ? pk[e0 + r] : KEY_MAX;
     ix[r] = e0 + r;
   }
-  // the thread's eight keys: odd-even transposition, which moves no key past an equal one
-#pragma unroll
-  for (int p = 0; p < kPer; ++p)
-#pragma unroll
-    for (int r = p & 1; r + 1 < kPer; r += 2)
-      if (k[r] > k[r + 1]) {
-        const uint64_t x = k[r];
-        const uint32_t y = ix[r];
-        k[r] = k[r + 1], ix[r] = ix[r + 1];
-        k[r + 1] = x, ix[r + 1] = y;
-      }
+  sort_eight(k, ix);
   for (uint32_t w = kPer; w < kChunk; w <<= 1) {  // uniform across the block
     put_eight(m, k, ix);
     __syncthreads();
@@ -282,7 +286,90 @@ __global__ __launch_bounds__(kTileThreads) void compact_last_kernel(const uint64
   if (threadIdx.x == 0 && (blockIdx.x + 1) * (uint64_t)kTile >= n) *dm = before + total;
 }
 
+// ---- bulk build ---------------------------------------------------------------------------------
+//
+// A bucket of the build's pairs (at most kBucketSortMax), sorted in LDS by merges like a chunk above, then
+// written to its leaves: sorted pair g goes to slot g % fill of leaf g / fill.  The values are read from the
+// bucket's own 40 KiB, which its block has just brought to L2.  4 million pairs: partition 45 us and this
+// kernel 132 (bound by the dependent LDS reads of its nine merges, two blocks per CU), where eight radix passes,
+// the validation, the leaf fill and the minima took 388; the build with one search of its keys went
+// 656 -> 385 us.
+constexpr int kBucketThreads = (int)kBucketSortMax / kPer;
+__global__ __launch_bounds__(kBucketThreads) void bucket_sort_fill_kernel(
+    const uint64_t* __restrict__ keys, const uint64_t* __restrict__ vals, size_t n, const uint32_t* __restrict__ totals,
+    uint32_t fill, Leaf* __restrict__ leaves, uint64_t* __restrict__ mins, uint32_t* __restrict__ flags, uint32_t skip,
+    uint64_t* __restrict__ edge) {
+  __shared__ MergeLds<kBucketThreads> m;
+  __shared__ uint32_t part_w[kBucketThreads / 64], bad;
+  if (*flags & skip) return;  // block-uniform: set before this launch
+  const uint32_t cnt = totals[blockIdx.x];
+  if (cnt == 0) return;
+  uint32_t part = 0;  // the pairs before this bucket
+  for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kBucketThreads) part += totals[b];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o);
+  if ((threadIdx.x & 63) == 0) part_w[threadIdx.x >> 6] = part;
+  if (threadIdx.x == 0) bad = 0;
+  __syncthreads();
+  uint32_t start = 0;
+#pragma unroll
+  for (int w = 0; w < kBucketThreads / 64; ++w) start += part_w[w];
+  const uint32_t t0 = threadIdx.x * kPer;
+  uint64_t k[kPer];
+  uint32_t ix[kPer];
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    k[r] = t0 + r < cnt ? keys[start + t0 + r] : KEY_MAX;
+    ix[r] = t0 + r;
+  }
+  sort_eight(k, ix);
+  for (uint32_t w = kPer; w < cnt; w <<= 1) {  // uniform across the block
+    put_eight(m, k, ix);
+    __syncthreads();
+    const uint32_t base = t0 & ~(2 * w - 1);
+    const uint32_t na = base + w < kBucketSortMax ? w : kBucketSortMax - base;
+    const uint32_t nb = base + na + w < kBucketSortMax ? w : kBucketSortMax - base - na;
+    merge_eight(m, base, na, base + na, nb, t0 - base, k, ix);
+    __syncthreads();
+  }
+  put_eight(m, k, ix);
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint32_t i = r * kBucketThreads + threadIdx.x;
+    if (i < cnt) {
+      const uint64_t key = m.k[slot_of(i)];
+      const uint32_t src = m.ix[slot_of(i)];
+      const uint32_t g = start + i, leaf = g / fill, slot = g - leaf * fill;
+      uint32_t f = key == KEY_MAX ? 1u : 0u;
+      if (i + 1 < cnt && m.k[slot_of(i + 1)] == key) f |= 2u;  // equal keys share a bucket
+      if (f) atomicOr(&bad, f);
+      leaves[leaf].key[slot] = key;
+      leaves[leaf].val[slot] = src < cnt ? vals[start + src] : 0ull;  // (a KEY_MAX key may stand for padding)
+      if (slot == 0) mins[leaf] = key;
+      if (slot + 1 == fill || g + 1 == n)
+        for (uint32_t p = slot + 1; p < (uint32_t)LEAF_KEYS; ++p) {
+          leaves[leaf].key[p] = KEY_MAX;
+          leaves[leaf].val[p] = 0ull;
+        }
+      if (g == 0) edge[0] = key;
+      if (g + 1 == n) edge[1] = key;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && bad) atomicOr(flags, bad);
+}
+
 }  // namespace
+
+hipError_t bucket_sort_fill(const uint64_t* keys, const uint64_t* vals, size_t n, int bits, const uint32_t* totals,
+                            int fill, Leaf* leaves, uint64_t* mins, uint32_t* flags, uint32_t skip, uint64_t* edge,
+                            hipStream_t s) {
+  ProfScope prof("build", s);
+  hipLaunchKernelGGL(bucket_sort_fill_kernel, dim3(1u << bits), dim3(kBucketThreads), 0, s, keys, vals, n, totals,
+                     (uint32_t)fill, leaves, mins, flags, skip, edge);
+  return hipGetLastError();
+}
 
 size_t dedupe_tmp_bytes(size_t n) { return ((n + kTile - 1) / kTile) * sizeof(uint32_t); }
 

@@ -90,7 +90,8 @@ constexpr int kScanDigits = 16;
 constexpr int kScanSegs = kScanThreads / kScanDigits;
 constexpr int kScanBatch = 8;
 __global__ __launch_bounds__(kScanThreads) void part_scan_kernel(uint32_t* __restrict__ counts, uint32_t nd,
-                                                                 uint32_t nb) {
+                                                                 uint32_t nb, uint32_t limit,
+                                                                 uint32_t* __restrict__ flags, uint32_t flag) {
   __shared__ uint32_t sums[kScanSegs][kScanDigits];
   const uint32_t j = threadIdx.x % kScanDigits, seg = threadIdx.x / kScanDigits;
   uint32_t* col = counts + blockIdx.x * kScanDigits + j;
@@ -122,7 +123,10 @@ __global__ __launch_bounds__(kScanThreads) void part_scan_kernel(uint32_t* __res
       run += v[u];
     }
   }
-  if (seg == 0) col[(size_t)nb * nd] = total;
+  if (seg == 0) {
+    col[(size_t)nb * nd] = total;
+    if (flags && total > limit) atomicOr(flags, flag);  // a bucket that its block could not hold
+  }
 }
 
 __device__ __forceinline__ void load_digits(const uint32_t* __restrict__ row, uint32_t d0, uint32_t nd,
@@ -351,6 +355,71 @@ __global__ __launch_bounds__(kThreads) void part_unscatter_kernel(const uint64_t
   }
 }
 
+// The same for (key, value) pairs: 128 KiB of pairs, one block of 1024 threads per CU.  Nothing is recorded.
+// Does nothing once *flags has `skip`.
+constexpr int kPairThreads = 1024;
+constexpr int kPairItems = kTile / kPairThreads;
+constexpr int kPairDPer = kDigits / kPairThreads;
+__global__ __launch_bounds__(kPairThreads) void part_pairs_kernel(const uint64_t* __restrict__ kin,
+                                                                  const uint64_t* __restrict__ vin,
+                                                                  uint64_t* __restrict__ kout,
+                                                                  uint64_t* __restrict__ vout, size_t n, int shift,
+                                                                  uint32_t nd, const uint32_t* __restrict__ offsets,
+                                                                  uint32_t nb, const uint32_t* __restrict__ flags,
+                                                                  uint32_t skip) {
+  __shared__ uint64_t skeys[kTile], svals[kTile];
+  __shared__ __align__(16) uint32_t dig[kDigits];
+  __shared__ uint32_t scan_sh[kPairThreads / 64 + 1];
+  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  if (tile >= nb || (*flags & skip)) return;  // block-uniform
+  const uint32_t mask = nd - 1, d0 = threadIdx.x * kPairDPer;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const size_t tile0 = (size_t)tile * kTile, base = tile0 + (size_t)w * 64 * kPairItems;
+  uint32_t tot[kPairDPer], g[kPairDPer], all;
+#pragma unroll
+  for (int j = 0; j < kPairDPer; ++j) {
+    tot[j] = d0 < nd ? offsets[(size_t)nb * nd + d0 + j] : 0u;
+    g[j] = d0 < nd ? offsets[(size_t)tile * nd + d0 + j] : 0u;
+  }
+  uint64_t kk[kPairItems], vv[kPairItems];
+#pragma unroll
+  for (int r = 0; r < kPairItems; ++r) {
+    const size_t i = base + (size_t)r * 64 + lane, c = i < n ? i : n - 1;
+    kk[r] = kin[c];
+    vv[r] = vin[c];
+  }
+  for (uint32_t d = threadIdx.x; d < nd; d += kPairThreads) dig[d] = 0;
+  uint32_t dbase = block_exclusive_scan<uint32_t, kPairThreads>(tot[0] + tot[1], scan_sh, all);  // ends with a barrier
+  uint32_t rank[kPairItems];
+#pragma unroll
+  for (int r = 0; r < kPairItems; ++r)
+    rank[r] = base + (size_t)r * 64 + lane < n ? atomicAdd(&dig[(uint32_t)(kk[r] >> shift) & mask], 1u) : 0u;
+  __syncthreads();
+  const uint32_t c0 = d0 < nd ? dig[d0] : 0u, c1 = d0 < nd ? dig[d0 + 1] : 0u;
+  const uint32_t b0 = block_exclusive_scan<uint32_t, kPairThreads>(c0 + c1, scan_sh, all), b1 = b0 + c0;
+  if (d0 < nd) dig[d0] = b0, dig[d0 + 1] = b1;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kPairItems; ++r)
+    if (base + (size_t)r * 64 + lane < n) {
+      const uint32_t lp = dig[(uint32_t)(kk[r] >> shift) & mask] + rank[r];
+      skeys[lp] = kk[r];
+      svals[lp] = vv[r];
+    }
+  __syncthreads();
+  if (d0 < nd) dig[d0] = dbase + g[0] - b0, dig[d0 + 1] = dbase + tot[0] + g[1] - b1;
+  __syncthreads();
+  const uint32_t cnt = (uint32_t)(n - tile0 < (size_t)kTile ? n - tile0 : (size_t)kTile);
+#pragma unroll 4
+  for (uint32_t i = threadIdx.x; i < cnt; i += kPairThreads) {
+    const uint64_t k = skeys[i];
+    const uint32_t p = dig[(uint32_t)(k >> shift) & mask] + i;
+    kout[p] = k;
+    vout[p] = svals[i];
+  }
+}
+static_assert(kPairDPer == 2, "the offsets above are written for two digits per thread");
+
 size_t offsets_bytes(size_t n, int bits) {
   const size_t nb = (n + kTile - 1) / kTile;
   return ((nb + 1) * ((size_t)4 << bits) + 255) / 256 * 256;
@@ -386,11 +455,43 @@ hipError_t partition_keys(const uint64_t* q, size_t n, int top, uint64_t* out, v
   }
   {
     ProfScope prof("scan", s);
-    hipLaunchKernelGGL(part_scan_kernel, dim3(nd / kScanDigits), dim3(kScanThreads), 0, s, offsets, nd, nb);
+    hipLaunchKernelGGL(part_scan_kernel, dim3(nd / kScanDigits), dim3(kScanThreads), 0, s, offsets, nd, nb, 0u,
+                       (uint32_t*)nullptr, 0u);
   }
   ProfScope prof("psa_scatter", s);
   hipLaunchKernelGGL(part_scatter_kernel, dim3(grid_for(nb)), dim3(kThreads), 0, s, q, out, place, n, shift, nd,
                      (const uint32_t*)offsets, nb, dn);
+  return hipGetLastError();
+}
+
+int pair_bits(size_t n) {
+  int b = kPartMinBits;
+  while (b <= kPartMaxBits && (n >> b) > (size_t)kPairBucket) ++b;
+  return b <= kPartMaxBits ? b : 0;
+}
+
+size_t partition_pairs_bytes(size_t n) { return offsets_bytes(n, pair_bits(n)); }
+
+hipError_t partition_pairs(const uint64_t* keys, const uint64_t* vals, size_t n, int top, uint64_t* kout,
+                           uint64_t* vout, void* tmp, uint32_t* flags, uint32_t flag, const uint32_t** totals,
+                           hipStream_t s) {
+  const int bits = n ? pair_bits(n) : 0;
+  if (!bits || top < 1 || top > 64) return hipErrorInvalidValue;
+  const uint32_t nd = 1u << bits, nb = (uint32_t)((n + kTile - 1) / kTile);
+  const int shift = top > bits ? top - bits : 0;  // fewer varying bits than digits: the digits above stay empty
+  uint32_t* offsets = reinterpret_cast<uint32_t*>(tmp);
+  ProfScope prof("build", s);
+  if ((reinterpret_cast<uintptr_t>(keys) & 15) == 0)
+    hipLaunchKernelGGL(part_hist_kernel<true>, dim3(grid_for(nb)), dim3(kThreads), 0, s, keys, n, shift, nd, offsets, nb,
+                       (const uint32_t*)nullptr);
+  else
+    hipLaunchKernelGGL(part_hist_kernel<false>, dim3(grid_for(nb)), dim3(kThreads), 0, s, keys, n, shift, nd, offsets,
+                       nb, (const uint32_t*)nullptr);
+  hipLaunchKernelGGL(part_scan_kernel, dim3(nd / kScanDigits), dim3(kScanThreads), 0, s, offsets, nd, nb,
+                     kBucketSortMax, flags, flag);
+  hipLaunchKernelGGL(part_pairs_kernel, dim3(grid_for(nb)), dim3(kPairThreads), 0, s, keys, vals, kout, vout, n, shift,
+                     nd, (const uint32_t*)offsets, nb, (const uint32_t*)flags, flag);
+  *totals = offsets + (size_t)nb * nd;
   return hipGetLastError();
 }
 
