@@ -145,9 +145,13 @@ ProfScope::~ProfScope() {
 // tree object helpers
 namespace hm {
 
+// Events that only order streams of one device (every search records one): without the system-scope fence
+// a launch and its event take 4.9 us on the stream instead of 6.4.
+constexpr unsigned kOrderEvent = hipEventDisableTiming | hipEventDisableSystemFence;
+
 int ensure_ws(hm_tree* t, hipStream_t s, size_t bytes, Workspace** out) {
   Workspace& w = t->ws[s];
-  if (!w.last_use) HM_TRY(hipEventCreateWithFlags(&w.last_use, hipEventDisableTiming));
+  if (!w.last_use) HM_TRY(hipEventCreateWithFlags(&w.last_use, kOrderEvent));
   if (w.bytes < bytes) {
     const size_t old = w.bytes;
     if (w.buf) {
@@ -196,6 +200,13 @@ int resolve_search(const hm_tree* t, uint64_t n, const hm_search_opts* o, Search
   sl->lds_levels = (o && o->lds_levels >= 0) ? choose_lds_levels(t, o->lds_levels) : t->lds_levels;
   sl->blocks_per_cu = (o && o->blocks_per_cu) ? (int)o->blocks_per_cu : base.blocks_per_cu;
   sl->queries_per_group = (o && o->queries_per_group) ? (int)o->queries_per_group : base.queries_per_group;
+  // An unsorted batch that one round of resident blocks holds with one query per group takes one: nothing is
+  // gained by more in flight, and a query's chain is shorter (kernel, 20011 queries on 2^25 keys: 4.4-5.2 us
+  // against 6.0-6.2 with four; 2^16: 6.2-6.4 against 7.0-7.2; 2^18, four rounds: 18.0-19.6 against 18.9).  Tuned
+  // trees and explicit shapes keep theirs.
+  if (!psa && !t->tuned && !(o && (o->group_size || o->queries_per_group || o->blocks_per_cu)) &&
+      n * (uint64_t)sl->group <= (uint64_t)launch_cfg().num_cus * (uint64_t)sl->blocks_per_cu * 256)
+    sl->queries_per_group = 1;
   if (sl->queries_per_group != 1 && sl->queries_per_group != 2 && sl->queries_per_group != 4)
     return set_err(HM_EINVAL, "queries_per_group %d not in {1,2,4}", sl->queries_per_group);
   int mode = (o && o->output_mode) ? (int)o->output_mode : base.output_mode;
@@ -493,8 +504,8 @@ static int create_tree(const hm_params* p, hm_tree** out) {
     rc = set_err(HM_EDEVICE, "no HIP device");
   else if (stream_take(&t->own) != hipSuccess)
     rc = set_err(HM_EDEVICE, "hipStreamCreate failed");
-  else if (hipEventCreateWithFlags(&t->publish_ev, hipEventDisableTiming) != hipSuccess ||
-           hipEventCreateWithFlags(&t->na_ev, hipEventDisableTiming) != hipSuccess)
+  else if (hipEventCreateWithFlags(&t->publish_ev, kOrderEvent) != hipSuccess ||
+           hipEventCreateWithFlags(&t->na_ev, kOrderEvent) != hipSuccess)
     rc = set_err(HM_EDEVICE, "hipEventCreate failed");
   if (rc) {
     free_tree(t);

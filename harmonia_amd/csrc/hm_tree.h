@@ -71,6 +71,7 @@ struct hm_tree {
   hm::Leaf* d_leaves = nullptr;
   int lds_levels = 0;
   uint64_t layout_version = 0;  // bumped whenever a device array of the layout is reallocated
+  bool tuned = false;  // the tuner has set cfg_direct and cfg_psa
   hm::SearchCfg cfg_direct{4, 4, 4, HM_OUT_UNPERMUTE};  // unsorted batches: memory-transaction bound
   // PSA-ordered batches: neighbours share nodes.  10 blocks per CU = two full rounds of the five
   // blocks of this shape that fit on a CU (96 VGPRs): a partial last round of the persistent grid

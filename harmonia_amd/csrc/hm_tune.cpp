@@ -159,6 +159,7 @@ int tune_tree(hm_tree* t, const uint64_t* sample, uint64_t n, uint32_t flags, hm
   }
   if (threshold == ~0ull && bp.ms < bd.ms) threshold = n;
   // apply
+  t->tuned = true;
   t->cfg_direct = SearchCfg{bd.sl.group, bd.sl.queries_per_group, bd.sl.blocks_per_cu, HM_OUT_UNPERMUTE};
   t->cfg_psa = SearchCfg{bp.sl.group, bp.sl.queries_per_group, bp.sl.blocks_per_cu, bp.mode};
   t->lds_levels = bd.sl.lds_levels;
