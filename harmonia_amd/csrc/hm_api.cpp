@@ -264,6 +264,15 @@ static bool partitions(const SearchLaunch& sl, int psa_bits) {
   return sl.group == 2 && sl.queries_per_group == 4 && !sl.window && psa_bits > 8 && psa_bits <= 16;
 }
 
+// PSA-order results need both passes, and the same kernel may search what they sorted: if the window orders
+// the tree's keys at all (it starts at bit 63, so for small keys it does not), and the batch is one and a
+// half rounds of blocks or more.  Whole calls over 2^18..2^26 keys, fanouts 32..128, take 0.67 to 0.99 of the
+// time with search_span_kernel; at 2^20 + 3 queries, with three blocks in the second round, 0.93 to 1.12, and
+// with keys that share the whole window 0.95 to 1.23.
+static bool chunks_psa_order(const TreeView& tv, const SearchLaunch& sl, int psa_bits, size_t n) {
+  return partitions(sl, psa_bits) && tv.psa_top > 64 - psa_bits && n >= (size_t)launch_cfg().num_cus * 6144;
+}
+
 int enqueue_pipeline(const TreeView& tv, const SearchLaunch& sl, int psa_bits, int out_mode, const uint64_t* dq,
                      size_t n, const uint32_t* dn, const PipeBufs& b, uint64_t* dvals, uint8_t* dfound,
                      uint32_t* dpos, hipStream_t s) {
@@ -300,7 +309,10 @@ int enqueue_pipeline(const TreeView& tv, const SearchLaunch& sl, int psa_bits, i
   SearchLaunch ss = sl;
   ss.sorted = true;
   if (out_mode == HM_OUT_PSA_ORDER) {
-    HM_TRY(launch_search(tv, ss, sk, sp, dvals, dfound, n, OUT_DIRECT, s, dn));
+    if (chunks_psa_order(tv, sl, psa_bits, n))
+      HM_TRY(launch_search_chunks(tv, sk, dvals, dfound, n, top, psa_bits, s, dn));
+    else
+      HM_TRY(launch_search(tv, ss, sk, sp, dvals, dfound, n, OUT_DIRECT, s, dn));
     HM_TRY(hipMemcpyAsync(dpos, sp, n * 4, hipMemcpyDeviceToDevice, s));
   } else {
     HM_TRY(launch_search(tv, ss, sk, sp, dvals, dfound, n, OUT_SCATTER, s, dn));

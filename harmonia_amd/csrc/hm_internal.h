@@ -48,6 +48,7 @@ struct TreeView {
   // Every key agrees with the others above it, so a PSA window that ends there orders queries in the
   // key range as finely as its width allows.
   int32_t psa_top;
+  uint64_t any_key;  // a key of the tree: its bits from psa_top on are every key's
 };
 
 // ---- launch helpers (host) -------------------------------------------------------------

@@ -3,10 +3,10 @@
 //
 // Measured, 2^24 queries: histogram 32 us, scan 17, scatter 71, un-scatter 120, where the two 8-bit passes
 // took 58, 10, 132 and 159; 2^20 queries: 4.2, 4.8, 8.3 and 9.3 against 8.7, 8.5, 25 and 20.  The whole
-// search went 699 -> 640 us at 2^24 on 2^26 keys and 83 -> 55 us at 2^20 on 2^20.  What bounds it: memory at
+// search went 699 -> 589 us at 2^24 on 2^26 keys and 82 -> 46 us at 2^20 on 2^20.  What bounds it: memory at
 // the copy rate (the histogram reads 134 MB, the scatter moves 318 MB); the un-scatter's tiles wait for
 // their barriers and for 2048 short runs (nine or ten bits instead of eleven: 81 and 96 us, but the search
-// reads more leaves twice, 455 and 423 us against 404).
+// reads more leaves twice, 455 and 423 us for 404).
 //
 // Such a search may take its queries in any order that brings neighbours together, so the batch is split
 // once by the top bits of the tree's key range into buckets of a few thousand queries (histogram, scan,

@@ -685,32 +685,33 @@ hipError_t launch_window(const TreeView& tv, const SearchLaunch& sl, const uint6
 
 // ---- chunk search (batches partitioned by bucket) ------------------------------------------------
 //
-// A block takes kChunk consecutive queries of the partitioned batch: a bucket or a part of one, so a narrow
-// key range in any order.  It orders them by the bits below the bucket's (an LDS atomic gives each key its
-// place, no order among equal digits), and each wave searches 512 neighbours, one lane per query:
-//   - every descent starts at the deepest node that holds the chunk's smallest and largest key;
+// A block takes 2048 or 4096 consecutive queries of the partitioned batch: a bucket or a part of one, so a
+// narrow key range in any order.  It orders them by the bits below the bucket's (an LDS atomic gives each key its
+// place, no order among equal digits), and each wave searches its neighbours, one lane per query:
+//   - every descent starts at the deepest node that holds the chunk's buckets, found from the buckets' bounds;
 //   - per level, the run of nodes that 256 queries reach goes to LDS (LDS-direct loads, one round trip) and
 //     each lane ranks its key there by binary search;
-//   - 64 queries at a time, the distinct leaves among neighbours go to LDS, eight whole leaves per load, and
-//     each lane finds its key there.
-// Results go back to LDS and out in the order the queries came in, which the un-partition expects.
+//   - the distinct leaves among neighbours pass through a ring in LDS, eight whole leaves per load, two
+//     batches of 16 on their way while 64 queries are found in a third.
+// Results go back to LDS and out in the order the queries came in, which the un-partition expects and a batch
+// sorted in full has anyway.
 //
-// What bounds it: the leaves' lines at the rate memory gives lines in key order.  2^24 queries of 2^26 keys
-// read 1.45 GB and write 0.15 in 404 us (4.0 TB/s; VALU 45% busy); search_span_kernel over the fully sorted
-// batch took 362 us for 1.54 GB, but the second sorting pass that needs cost 180.  2^20 queries of 2^20 keys:
-// 27 us against 21 plus 35 of sorting.
+// What bounds it: the leaves' lines at the rate memory gives lines in key order, and nearly as much the
+// instructions it issues.  2^24 queries of 2^26 keys read 1.45 GB and write 0.15 in 366 us (4.4 TB/s; 404
+// without the ring, with a reduction over each chunk's keys for the start node and over each run's nodes);
+// search_span_kernel over the fully sorted batch takes 362 us for 1.54 GB, but the second sorting pass that
+// needs costs 180.  2^20 queries of 2^20 keys: 19 us (27) against 21 plus 35 of sorting.  Over batches that
+// two passes sorted (PSA-order results), search_span_kernel's time in brackets: 2^24 of 2^26 keys 313 us
+// (386), 3000001 of 2^25 93 (101).
 constexpr int kChunkThreads = 512;
 constexpr int kChunkWaves = kChunkThreads / 64;
-constexpr int kChunkItems = 8;
-constexpr uint32_t kChunk = kChunkThreads * kChunkItems;
 constexpr int kChunkBits = 11;  // digit of the order inside a chunk
 constexpr uint32_t kChunkDigits = 1u << kChunkBits;
 constexpr int kChunkGroup = 4;  // rounds of 64 queries that share a node run
-// A wave's node run: 4 KiB (12 nodes of fanout 32, 7 of 64, 3 of 128); two blocks (16 waves) per CU.  2 KiB
-// was slower (421 us against 404 on 2^24 queries of 2^26 keys: more runs that do not fit), and so were five
-// or six waves per SIMD, whose registers spill (463 and 485 us).
+// A wave's node run: 4 KiB (12 nodes of fanout 32, 7 of 64, 3 of 128); two blocks (16 waves) per CU.  On 2^24
+// queries of 2^26 keys 2 KiB took 421 us for 404 (more runs that do not fit), and five or six waves per SIMD,
+// whose registers spill, 463 and 485.
 constexpr uint32_t kChunkNodeBytes = 4096;
-constexpr uint32_t kChunkLeaves = kChunk * 8 / kChunkWaves / sizeof(Leaf);  // leaves in a wave's share of the keys' LDS
 
 // upper_bound slot of t in a node held in LDS, one lane per query (the last key slot is KEY_MAX > t).
 template <int F>
@@ -722,8 +723,32 @@ __device__ __forceinline__ uint32_t node_next_bin(const uint64_t* nd, uint64_t t
   return (uint32_t)nd[idx_slots(F) - 1] + r;
 }
 
+// Lane I's value to the four lanes of each quad.
+template <int I>
+__device__ __forceinline__ uint32_t quad_lane(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, I * 0x55, 0xF, 0xF, false);
+}
+template <int I>
+__device__ __forceinline__ uint64_t quad_lane(uint64_t v) {
+  return (uint64_t)quad_lane<I>((uint32_t)(v >> 32)) << 32 | quad_lane<I>((uint32_t)v);
+}
+
+// One level for a round of queries that reach nodes anywhere: each quad of lanes reads its four queries'
+// nodes together, four coalesced reads under way at a time.  A lane per query that reads its node alone made
+// searches of trees whose keys crowd at one end of their range (so that the batch's bits order nothing) take
+// 1.2 to 2 times as long, a binary search in memory more.
+template <int F>
+__device__ __forceinline__ void quad_level(const uint64_t* __restrict__ inner, uint64_t t, uint32_t& node, int lane) {
+  const uint64_t td = t == KEY_MAX ? KEY_MAX - 1 : t;
+  const uint64_t tq[4] = {quad_lane<0>(td), quad_lane<1>(td), quad_lane<2>(td), quad_lane<3>(td)};
+  uint32_t nq[4] = {quad_lane<0>(node), quad_lane<1>(node), quad_lane<2>(node), quad_lane<3>(node)};
+  level_q<F, 4, 4>(inner, tq, nq, lane & 3, lane & ~3);
+  const uint32_t a = lane & 1 ? nq[1] : nq[0], b = lane & 1 ? nq[3] : nq[2];
+  node = lane & 2 ? b : a;
+}
+
 // One level for R rounds of queries: the run of nodes they reach through LDS if it fits, else round by
-// round, else each lane reads its node.
+// round, else node by node.
 template <int F, int R>
 __device__ __forceinline__ void chunk_level(const uint64_t* __restrict__ inner, uint64_t* nbuf, const uint64_t* t,
                                             uint32_t* node, int lane) {
@@ -731,14 +756,22 @@ __device__ __forceinline__ void chunk_level(const uint64_t* __restrict__ inner, 
   constexpr int CH = NS / 2;
   constexpr int SPAN = kChunkNodeBytes / (NS * 8);
   constexpr int SPL = kChunkNodeBytes / 1024;
-  uint32_t lo = node[0], hi = node[0];
+  // the queries are nearly in key order: the first one's node to the last one's, if that holds for all
+  uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)node[0], 0);
+  uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)node[R - 1], 63);
+  bool in = true;
 #pragma unroll
-  for (int j = 1; j < R; ++j) {
-    lo = node[j] < lo ? node[j] : lo;
-    hi = node[j] > hi ? node[j] : hi;
+  for (int j = 0; j < R; ++j) in = in && node[j] - lo <= hi - lo;
+  if (!__all(in)) {  // wave-uniform
+    lo = hi = node[0];
+#pragma unroll
+    for (int j = 1; j < R; ++j) {
+      lo = node[j] < lo ? node[j] : lo;
+      hi = node[j] > hi ? node[j] : hi;
+    }
+    lo = wave_min_u32(lo);
+    hi = wave_max_u32(hi);
   }
-  lo = wave_min_u32(lo);
-  hi = wave_max_u32(hi);
   if (hi - lo < (uint32_t)SPAN) {  // wave-uniform
     wave_stage<SPL>(reinterpret_cast<const ulonglong2*>(inner + (size_t)lo * NS), (int)(hi - lo + 1) * CH, nbuf, lane);
 #pragma unroll
@@ -749,12 +782,36 @@ __device__ __forceinline__ void chunk_level(const uint64_t* __restrict__ inner, 
 #pragma unroll
     for (int j = 0; j < R; ++j) chunk_level<F, 1>(inner, nbuf, t + j, node + j, lane);
   } else {
-    node[0] = node_next<F, 1>(inner + (size_t)node[0] * NS, t[0] == KEY_MAX ? KEY_MAX - 1 : t[0], 0, lane);
+    quad_level<F>(inner, t[0], node[0], lane);
   }
 }
 
+// LDS reads that do not wait for LDS-direct loads in flight to other places: before an ordinary read of LDS
+// the compiler waits for every one of them.  Each block waits for its own reads.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
+}
+__device__ __forceinline__ void lds_read_4x16(uint32_t a, uint32_t b, uint32_t c, uint32_t d, ulonglong2 (&x)[4]) {
+  u32x4 r[4];
+  asm volatile(
+      "ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
+      : "v"(a), "v"(b), "v"(c), "v"(d)
+      : "memory");
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    x[i] = make_ulonglong2((uint64_t)r[i].y << 32 | r[i].x, (uint64_t)r[i].w << 32 | r[i].z);
+}
+__device__ __forceinline__ uint64_t lds_read_8(uint32_t a) {
+  uint64_t r;
+  asm volatile("ds_read_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(r) : "v"(a) : "memory");
+  return r;
+}
+
 // q: partitioned keys, by bits [top - bits, top).
-template <int F>
+template <int F, int I>
 __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv, const uint64_t* __restrict__ q,
                                                                      uint64_t* __restrict__ out_vals,
                                                                      uint8_t* __restrict__ out_found, uint32_t n,
@@ -762,11 +819,13 @@ __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv
                                                                      const uint32_t* __restrict__ dn) {
   constexpr int NS = node_slots(F);
   constexpr int DPer = kChunkDigits / kChunkThreads;
-  __shared__ __align__(16) uint64_t sk[kChunk];  // sorted keys, then each wave's leaves, then values
-  __shared__ __align__(16) uint8_t sf[kChunk];                 // found flags (before: each wave's list of leaves)
-  __shared__ __align__(16) uint64_t nbufs[kChunkWaves * kChunkNodeBytes / 8];  // before: the digit counters
-  __shared__ uint64_t wmin[kChunkWaves], wmax[kChunkWaves];
-  __shared__ uint32_t scan_sh[kChunkWaves + 1];
+  constexpr uint32_t kChunk = kChunkThreads * I;
+  constexpr uint32_t kRing2 = kChunkWaves * 2 * 256;  // two batches of 16 leaves per wave
+  __shared__ __align__(16) uint64_t sk[kChunk > kRing2 ? kChunk : kRing2];  // keys, then two thirds of the leaf rings, then values
+  __shared__ __align__(16) uint8_t sf[kChunk];   // found flags
+  // the digit counters, then the node runs, then the lists of leaves and the last third of the rings
+  __shared__ __align__(16) uint64_t nbufs[kChunkWaves * kChunkNodeBytes / 8];
+  __shared__ uint32_t scan_sh[kChunkWaves + 1], at_root;
   static_assert(sizeof(nbufs) >= kChunkDigits * 4, "the counters fit under the node runs");
   uint32_t* cnt = reinterpret_cast<uint32_t*>(nbufs);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -774,15 +833,16 @@ __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv
   const uint32_t c0 = xcd_block(blockIdx.x, gridDim.x) * kChunk;
   if (c0 >= n) return;  // block-uniform
   const uint32_t m = n - c0 < kChunk ? n - c0 : kChunk;
-  uint64_t k[kChunkItems];
+  uint64_t k[I];
 #pragma unroll
-  for (int r = 0; r < kChunkItems; ++r) {
+  for (int r = 0; r < I; ++r) {
     const uint32_t i = r * kChunkThreads + threadIdx.x;
     k[r] = q[c0 + (i < m ? i : m - 1)];
   }
   const uint64_t kf = q[c0], kl = q[c0 + m - 1];  // uniform: the first and last bucket
 #pragma unroll
   for (int j = 0; j < DPer; ++j) cnt[j * kChunkThreads + threadIdx.x] = 0;
+  if (threadIdx.x == 0) at_root = 0;
   // the order's digit: bits below the first bucket's, shifted so that the chunk's buckets fit
   const int lo = top - bits > kChunkBits ? top - bits - kChunkBits : 0;
   const int ext = top - bits - lo;  // bits kept per bucket
@@ -790,25 +850,36 @@ __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv
   const uint32_t first = ((uint32_t)(kf >> lo) & fmask) >> ext << ext;
   const uint32_t span = (((uint32_t)(kl >> lo) & fmask) >> ext << ext) - first + (1u << ext);  // buckets ascend
   const int sh = span > kChunkDigits ? 32 - kChunkBits - __builtin_clz(span - 1) : 0;
-  uint64_t mn = ~0ull, mx = 0;
-#pragma unroll
-  for (int r = 0; r < kChunkItems; ++r) {
-    const uint64_t td = k[r] == KEY_MAX ? KEY_MAX - 1 : k[r];
-    mn = td < mn ? td : mn;
-    mx = td > mx ? td : mx;
-  }
-  mn = wave_min_u64(mn);
-  mx = wave_max_u64(mx);
-  if (lane == 0) {
-    wmin[w] = mn;
-    wmax[w] = mx;
+  // The deepest node above the leaves that holds the chunk's buckets (every wave finds it; uniform), the bits
+  // above them taken from a stored key.  A chunk with a query outside the buckets' bounds starts at the root.
+  const uint64_t* __restrict__ inner = tv.inner;
+  const int last = tv.height - 1;
+  uint32_t start = 0;
+  int l0 = 0;
+  const uint64_t above = top < 64 ? tv.any_key >> top << top : 0ull;
+  const uint64_t bmask = (1ull << bits) - 1ull;  // bits <= 16
+  const uint64_t ka = above | ((kf >> (top - bits)) & bmask) << (top - bits);
+  uint64_t kb = above | ((kl >> (top - bits)) & bmask) << (top - bits) | ((1ull << (top - bits)) - 1ull);
+  kb = kb == KEY_MAX ? KEY_MAX - 1 : kb;
+  {
+    constexpr int GW = 32;
+    while (l0 < last) {
+      const uint32_t c = node_next_wide<F, GW>(inner + (size_t)start * NS, lane < GW ? ka : kb, lane % GW, lane & GW);
+      const uint32_t ca = (uint32_t)__builtin_amdgcn_readlane((int)c, 0);
+      if (ca != (uint32_t)__builtin_amdgcn_readlane((int)c, GW)) break;
+      start = ca;
+      ++l0;
+    }
   }
   __syncthreads();
-  uint32_t pos[kChunkItems];
+  uint32_t pos[I], dig[I];
+  bool outside = false;
 #pragma unroll
-  for (int r = 0; r < kChunkItems; ++r) {
+  for (int r = 0; r < I; ++r) {
     const uint32_t i = r * kChunkThreads + threadIdx.x;
+    outside |= k[r] < ka || (k[r] > kb && k[r] != KEY_MAX) || (k[r] == KEY_MAX && kb != KEY_MAX - 1);
     const uint32_t d = (((uint32_t)(k[r] >> lo) & fmask) - first) >> sh;
+    dig[r] = d;
     const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);
     pos[r] = 0;
     if (__ballot(i < m && d == f) == ~0ull) {  // one digit in the whole wave: one add
@@ -819,12 +890,12 @@ __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv
       pos[r] = atomicAdd(&cnt[d], 1u);
     }
   }
-#pragma unroll
-  for (int x = 0; x < kChunkWaves; ++x) {
-    mn = wmin[x] < mn ? wmin[x] : mn;
-    mx = wmax[x] > mx ? wmax[x] : mx;
-  }
+  if (__any(outside) && lane == 0) at_root = 1;
   __syncthreads();
+  if (at_root) {
+    start = 0;
+    l0 = 0;
+  }
   {
     uint32_t c[DPer], s = 0, total;
 #pragma unroll
@@ -841,104 +912,118 @@ __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < kChunkItems; ++r) {
+  for (int r = 0; r < I; ++r) {
     const uint32_t i = r * kChunkThreads + threadIdx.x;
-    const uint32_t d = (((uint32_t)(k[r] >> lo) & fmask) - first) >> sh;
     if (i < m) {
-      pos[r] += cnt[d];
+      pos[r] += cnt[dig[r]];
       sk[pos[r]] = k[r];
     }
   }
-  // the deepest node above the leaves that holds the whole chunk (every wave finds it; uniform)
-  const uint64_t* __restrict__ inner = tv.inner;
-  const int last = tv.height - 1;
-  uint32_t start = 0;
-  int l0 = 0;
-  {
-    constexpr int GW = 32;
-    const uint64_t a = uniform_u64(mn), b = uniform_u64(mx);
-    while (l0 < last) {
-      const uint32_t c = node_next_wide<F, GW>(inner + (size_t)start * NS, lane < GW ? a : b, lane % GW, lane & GW);
-      const uint32_t ca = (uint32_t)__builtin_amdgcn_readlane((int)c, 0);
-      if (ca != (uint32_t)__builtin_amdgcn_readlane((int)c, GW)) break;
-      start = ca;
-      ++l0;
-    }
-  }
   __syncthreads();  // keys are in place, the counters are free for the node runs
-  const uint32_t p0 = w * 64 * kChunkItems + lane;  // the lane's queries: p0 + 64 j
-  uint64_t t[kChunkItems];
-  uint32_t node[kChunkItems];
+  const uint32_t p0 = w * 64 * I + lane;  // the lane's queries: p0 + 64 j
+  uint64_t t[I];
+  uint32_t node[I];
 #pragma unroll
-  for (int j = 0; j < kChunkItems; ++j) {
+  for (int j = 0; j < I; ++j) {
     const uint32_t p = p0 + 64 * j;
     t[j] = sk[p < m ? p : m - 1];
     node[j] = start;
   }
   __syncthreads();  // every wave has its keys: their LDS holds leaves from here on
   uint64_t* nbuf = nbufs + w * (kChunkNodeBytes / 8);
-  uint64_t* lbuf = sk + w * (kChunkLeaves * 16);
-  uint32_t* llist = reinterpret_cast<uint32_t*>(sf) + w * (kChunk / 4 / kChunkWaves);  // 128 words
+  uint64_t* lbuf = sk + w * (2 * 256);
+  uint32_t* llist = reinterpret_cast<uint32_t*>(nbuf);  // 512 words, once the node runs are done
+  uint32_t before = ~0u;
 #pragma unroll
-  for (int g = 0; g < kChunkItems; g += kChunkGroup)
+  for (int g = 0; g < I; g += kChunkGroup)
     if (p0 - lane + 64 * g < m)  // wave-uniform
       for (int l = l0; l <= last; ++l) chunk_level<F, kChunkGroup>(inner, nbuf, t + g, node + g, lane);
-  uint32_t found = 0;
+  // The wave's leaves, each that differs from the one before it, numbered in query order: the numbers in
+  // node[], the leaves in the list.  They pass through a ring of three batches of 16 (2 KiB each), so two
+  // are on their way while one is searched.
+  uint32_t nl = 0;
 #pragma unroll
-  for (int j = 0; j < kChunkItems; ++j) {
+  for (int j = 0; j < I; ++j) {
     if (p0 - lane + 64 * j >= m) break;  // wave-uniform
-    // the leaves that differ from the lane below's, numbered in lane order
-    const uint32_t prev = (uint32_t)__shfl_up((int)node[j], 1);
-    const bool head = lane == 0 || prev != node[j];
+    const uint32_t up = (uint32_t)__shfl_up((int)node[j], 1);
+    const uint32_t prev = lane > 0 ? up : before;
+    before = (uint32_t)__builtin_amdgcn_readlane((int)node[j], 63);
+    const bool head = prev != node[j];
     const uint64_t heads = __ballot(head);
-    const uint32_t mine = (uint32_t)__popcll(heads & ((2ull << lane) - 1ull)) - 1u;
-    const uint32_t nd = (uint32_t)__popcll(heads);
+    const uint32_t mine = nl + (uint32_t)__popcll(heads & ((2ull << lane) - 1ull)) - 1u;
     if (head) llist[mine] = node[j] - tv.n_inner;
-    wave_lds_sync();
+    node[j] = mine;
+    nl += (uint32_t)__popcll(heads);
+  }
+  wave_lds_sync();
+  // eight leaves per load; a leaf's 16-byte piece p lands at place p ^ (number & 7), so lanes that read the
+  // same piece of different leaves spread over the banks
+  auto ring = [&](uint32_t bt) -> uint64_t* {
+    const uint32_t r = bt % 3;
+    return r < 2 ? lbuf + r * 256 : nbuf + 256;
+  };
+  auto issue = [&](uint32_t bt) {
+    uint64_t* buf = ring(bt);
+#pragma unroll
+    for (uint32_t u = 0; u < 2; ++u) {
+      const uint32_t x = 16 * bt + 8 * u + (lane >> 3);
+      const uint32_t lf = llist[x < nl ? x : nl - 1];
+      __builtin_amdgcn_global_load_lds(
+          (const global_void*)(reinterpret_cast<const ulonglong2*>(tv.leaves + lf) + ((lane ^ (lane >> 3)) & 7)),
+          (lds_void*)(buf + 128 * u), 16, 0, 0);
+    }
+  };
+  const uint32_t nbt = (nl + 15) / 16;
+  for (uint32_t bt = 0; bt < 3 && bt < nbt; ++bt) issue(bt);
+  uint32_t found = 0, cur = 0;
+#pragma unroll
+  for (int j = 0; j < I; ++j) {
+    if (p0 - lane + 64 * j >= m) break;  // wave-uniform
+    const uint32_t mine = node[j];
+    const uint32_t b0 = (uint32_t)__builtin_amdgcn_readlane((int)mine, 0) / 16;
+    const uint32_t b1 = (uint32_t)__builtin_amdgcn_readlane((int)mine, 63) / 16;
     uint64_t val = 0;
     bool eq = false;
-    for (uint32_t b = 0; b < nd; b += kChunkLeaves) {  // wave-uniform: at most two rounds of 32 leaves
-      // eight leaves per load; a leaf's 16-byte piece p lands at place p ^ (number & 7), so lanes that read
-      // the same piece of different leaves spread over the banks
-#pragma unroll
-      for (uint32_t u = 0; u < kChunkLeaves / 8; ++u) {
-        if (b + 8 * u < nd) {
-          const uint32_t x = b + 8 * u + (lane >> 3);
-          const uint32_t lf = llist[x < nd ? x : nd - 1];
-          __builtin_amdgcn_global_load_lds(
-              (const global_void*)(reinterpret_cast<const ulonglong2*>(tv.leaves + lf) + ((lane ^ (lane >> 3)) & 7)),
-              (lds_void*)(lbuf + 128 * u), 16, 0, 0);
-        }
-      }
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the leaves have landed in LDS
+    for (uint32_t bt = b0; bt <= b1;) {  // wave-uniform
+      const uint32_t be = bt + 2 < b1 ? bt + 2 : b1;  // batches bt .. be at once: nearly always the whole round
+      for (; cur < bt; ++cur)  // a batch that is done: its place takes the next one
+        if (cur + 3 < nbt) issue(cur + 3);
+      const uint32_t later = (bt + 3 < nbt ? bt + 3 : nbt) - 1 - be;  // batches on their way that can wait
+      if (later == 2)
+        __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4)
+      else if (later == 1)
+        __builtin_amdgcn_s_waitcnt(0x0F72);  // vmcnt(2)
+      else
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
       wave_lds_sync();
-      if (mine - b < kChunkLeaves) {
-        const uint32_t sw = mine & 7;
-        const ulonglong2* lf = reinterpret_cast<const ulonglong2*>(lbuf + (mine - b) * 16);
+      if (mine / 16 - bt <= be - bt) {
+        const uint32_t r = (mine / 16) % 3;
+        const uint32_t sw = mine & 7, lf = (r < 2 ? lds_address(lbuf) + r * 2048 : lds_address(nbuf) + 2048) + (mine & 15) * 128;
+        ulonglong2 x[4];
+        lds_read_4x16(lf + 16 * sw, lf + 16 * (1 ^ sw), lf + 16 * (2 ^ sw), lf + 16 * (3 ^ sw), x);
         uint32_t lt = 0;
 #pragma unroll
-        for (uint32_t p = 0; p < 4; ++p) {
-          const ulonglong2 x = lf[p ^ sw];
-          lt += (x.x < t[j] ? 1u : 0u) + (x.y < t[j] ? 1u : 0u);
-          eq |= x.x == t[j] || x.y == t[j];
+        for (int p = 0; p < 4; ++p) {
+          lt += (x[p].x < t[j] ? 1u : 0u) + (x[p].y < t[j] ? 1u : 0u);
+          eq |= x[p].x == t[j] || x[p].y == t[j];
         }
         eq = eq && t[j] != KEY_MAX;  // KEY_MAX is padding, never a stored key
-        if (eq) val = reinterpret_cast<const uint64_t*>(lf + ((4 + lt / 2) ^ sw))[lt & 1];
+        if (eq) val = lds_read_8(lf + 16 * ((4 + lt / 2) ^ sw) + 8 * (lt & 1));
       }
-      wave_lds_sync();  // the next loads overwrite the leaves
+      bt = be + 1;
     }
     t[j] = val;
     found |= eq ? 1u << j : 0u;
   }
   __syncthreads();  // every wave is done with its leaves
 #pragma unroll
-  for (int j = 0; j < kChunkItems; ++j) {
+  for (int j = 0; j < I; ++j) {
     sk[p0 + 64 * j] = t[j];
     sf[p0 + 64 * j] = (found >> j) & 1u;
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < kChunkItems; ++r) {
+  for (int r = 0; r < I; ++r) {
     const uint32_t i = r * kChunkThreads + threadIdx.x;
     if (i < m) {
       out_vals[c0 + i] = sk[pos[r]];
@@ -947,13 +1032,28 @@ __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv
   }
 }
 
+template <int F, int I>
+hipError_t launch_chunk_i(const TreeView& tv, const uint64_t* q, uint64_t* out_vals, uint8_t* out_found, size_t n,
+                        int top, int bits, hipStream_t s, const uint32_t* dn) {
+  constexpr size_t kChunk = kChunkThreads * I;
+  const size_t nb = ((n + kChunk - 1) / kChunk + 7) / 8 * 8;
+  hipLaunchKernelGGL((search_chunk_kernel<F, I>), dim3((unsigned)nb), dim3(kChunkThreads), 0, s, tv, q,
+                     out_vals, out_found, (uint32_t)n, top, bits, dn);
+  return hipGetLastError();
+}
+
 template <int F>
 hipError_t launch_chunk(const TreeView& tv, const uint64_t* q, uint64_t* out_vals, uint8_t* out_found, size_t n,
                         int top, int bits, hipStream_t s, const uint32_t* dn) {
-  const size_t nb = ((n + kChunk - 1) / kChunk + 7) / 8 * 8;
-  hipLaunchKernelGGL(search_chunk_kernel<F>, dim3((unsigned)nb), dim3(kChunkThreads), 0, s, tv, q,
-                     out_vals, out_found, (uint32_t)n, top, bits, dn);
-  return hipGetLastError();
+  // 2048 queries per block while 4096 leave the chip idle (2^20 queries of 2^20 keys, the whole search: 46 us
+  // for 51; 3 * 2^20 of 2^26: 159 for 170, of 2^20: 78 for 79), then 4096, whose ends read fewer leaves twice
+  // (2^22 of 2^20 and of 2^23: 93 us for 94, 120 for 124; 2^23: 184 for 188, 229 for 239): where neighbours
+  // share no leaves, a little later (2^22 of 2^26: 194 us with 2048 for 198, 5 * 2^20: 248 for 260, 2^23: 344
+  // for 346).
+  const size_t round = (size_t)launch_cfg().num_cus * kChunkThreads * 8;
+  if (n <= 3 * round || (n <= 5 * round && n <= tv.n_leaves))
+    return launch_chunk_i<F, kChunkGroup>(tv, q, out_vals, out_found, n, top, bits, s, dn);
+  return launch_chunk_i<F, 2 * kChunkGroup>(tv, q, out_vals, out_found, n, top, bits, s, dn);
 }
 
 // Locate for the update path: leaf id, lower_bound slot (low byte) with the leaf's free slots (next byte),

@@ -134,6 +134,7 @@ struct hm_tree {
     tv.fanout = F;
     for (int i = 0; i <= hm::MAX_LEVELS; ++i) tv.level_start[i] = level_start[i];
     tv.psa_top = psa_top;
+    tv.any_key = key_lo;
     return tv;
   }
   // Widen the key range [key_lo, key_hi] by [lo, hi] (lo > hi: nothing) and recompute psa_top.

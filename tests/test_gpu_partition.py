@@ -1,5 +1,5 @@
 """Searches through the one-pass partition (PSA on, results in input order) at the sizes where its pieces
-change: one query, a wave's 64, a wave's 512, chunks of 4096, tiles of 8192, the batch sizes where a digit
+change: one query, a wave's 64, a wave's 512, chunks of 2048 and 4096, tiles of 8192, the batch sizes where a digit
 bit is added, results at odd addresses, every query equal, clustered keys, misses outside the key range, and
 trees of one to four levels.  Against the oracle's sorted-array search; whole numbers, equal."""
 import numpy as np
@@ -79,4 +79,73 @@ def test_partition_shapes(gpu, F, kind):
     tree = BPlusTree.from_keys(sk, sv, keys_sorted=True, fanout=F, leaf_fill=8)
     check(tree, sk, sv, q)
     check(tree, sk, sv, q, lds_levels=0)
+    tree.close()
+
+
+@pytest.mark.parametrize("psa", [True, False])
+def test_captured_search_after_the_key_range_widens(gpu, psa):
+    """A batcher's captured searches see keys that an in-place epoch adds outside the old key range."""
+    from harmonia_amd import Batcher
+
+    keys = (np.uint64(3) << np.uint64(40)) + np.arange(50000, dtype=np.uint64) * np.uint64(16)
+    tree = BPlusTree.from_keys(keys, keys, keys_sorted=True, fanout=64, leaf_fill=5)
+    b = Batcher(tree, 60000, psa_bits=16 if psa else 0)
+    new = np.array([5, 1 << 20, (3 << 40) + 7, (5 << 40) + 1, (1 << 60) + 3, HM_KEY_MAX - 1], dtype=np.uint64)
+    q = np.concatenate([keys, new])
+    want = np.zeros(len(q), dtype=np.uint8)
+    want[:len(keys)] = 1
+    for step in range(4):
+        off = b.add(q)
+        b.flush()
+        v, f = b.copy_out(off, len(q))
+        assert np.array_equal(f, want) and np.array_equal(v, np.where(want == 1, q, 0))
+        if step % 2 == 0:  # an epoch between flushes: two keys further out each time
+            k = new[step + 1:step + 4]
+            before = tree.stats().relayouts
+            tree.update(k, k)
+            tree.publish()
+            assert tree.stats().relayouts == before
+            want[len(keys) + step + 1:len(keys) + step + 4] = 1
+    b.close()
+    tree.close()
+
+
+@pytest.mark.parametrize("F", [32, 64, 128])
+@pytest.mark.parametrize("n", [70001, 3 * (1 << 20), 3 * (1 << 20) + 1])
+def test_partition_by_bits_that_order_nothing(gpu, F, n):
+    """One key far from dense ids: every query falls into one bucket, and each quad reads its nodes."""
+    sk = np.append(np.arange(1, 200000, dtype=np.uint64) * np.uint64(3), np.uint64((1 << 63) + 5))
+    sv = W.splitmix64_mix(sk)
+    tree = BPlusTree.from_keys(sk, sv, keys_sorted=True, fanout=F, leaf_fill=5)
+    g = np.random.RandomState(9)
+    q = g.randint(0, 610000, n).astype(np.uint64)
+    q[g.randint(0, n, 50)] = np.uint64((1 << 63) + 5)
+    q[-1] = np.uint64(HM_KEY_MAX)
+    check(tree, sk, sv, q)
+    tree.close()
+
+
+@pytest.mark.parametrize("F", [32, 64, 128])
+@pytest.mark.parametrize("n", [3 * (1 << 19) - 1, 3 * (1 << 19), 3 * (1 << 20) + 1])
+@pytest.mark.parametrize("low", [False, True])
+def test_psa_order_results(gpu, F, n, low):
+    """Results in PSA order where the searching kernel changes: the batch's size, and keys below the window."""
+    import torch
+
+    g = np.random.RandomState(10)
+    sk = np.unique(g.randint(0, 1 << (47 if low else 62), 300007)).astype(np.uint64)
+    sv = W.splitmix64_mix(sk)
+    tree = BPlusTree.from_keys(sk, sv, keys_sorted=True, fanout=F, leaf_fill=7)
+    q = np.where(g.rand(n) < 0.8, sk[g.randint(0, len(sk), n)], g.randint(0, 1 << 63, n).astype(np.uint64))
+    q[g.randint(0, n, 100)] = np.uint64(HM_KEY_MAX)
+    dq = torch.from_numpy(q.view(np.int64)).cuda()
+    v, f = torch.empty_like(dq), torch.empty(n, dtype=torch.uint8, device="cuda")
+    pos = torch.empty(n, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    tree.search_batch(dq, out_vals=v, out_found=f, out_pos=pos, psa_bits=16, sorted_output=True)
+    torch.cuda.synchronize()
+    want = np.argsort(q >> np.uint64(48), kind="stable")
+    ev, ef = oracle.search_sorted(sk, sv, q[want])
+    assert np.array_equal(pos.cpu().numpy(), want)
+    assert np.array_equal(f.cpu().numpy(), ef) and np.array_equal(v.cpu().numpy().view(np.uint64), ev)
     tree.close()
