@@ -1286,11 +1286,11 @@ int publish_prepare(hm_tree* t, hipStream_t s, PublishPlan* plan) {
   uint32_t* cnt = (uint32_t*)(cur + 2 * a4);
   uint32_t* nstart = (uint32_t*)(cur + 3 * a4);
   void* ntmp = cur + 4 * a4;
-  HM_TRY(hipMemsetAsync(ins, 0, nl * 4, s));
+  uint32_t* mask = (uint32_t*)b.k0;  // the sorted keys' memory: two words per batch entry
+  uint32_t* end = mask + n;
   HM_TRY(hipMemsetAsync(first, 0xFF, nl * 4, s));
-  HM_TRY(count_inserts(b.leaf, b.found, plan->m, ins, s));
-  HM_TRY(leaf_first_keys(b.leaf, plan->m, first, s));
-  HM_TRY(new_leaf_counts(t->d_leaves, ins, nl, t->fill, cnt, s));
+  HM_TRY(run_bounds(b.leaf, b.slot, b.found, plan->m, first, mask, end, s));
+  HM_TRY(new_leaf_counts(first, mask, end, b.slot, nl, t->fill, ins, cnt, s));
   HM_TRY(exclusive_scan_u32(cnt, nstart, nl, 0u, ntmp, s));
   HM_TRY(copy_u32s(t->upd_host + 4, nstart + nl - 1, 1, s));
   HM_TRY(copy_u32s(t->upd_host + 5, cnt + nl - 1, 1, s));
@@ -1351,7 +1351,7 @@ int publish_prepare(hm_tree* t, hipStream_t s, PublishPlan* plan) {
   if (rc) return rc;
   // the leaf minima go straight to the inner rebuild's scratch (its first array)
   uint64_t* new_mins = (uint64_t*)((char*)t->rl_buf + ib_off);
-  HM_TRY(relayout_touched(t->d_leaves, ins, b.leaf, b.slot, b.uk, b.uv, b.found, plan->m, nstart, t->fill,
+  HM_TRY(relayout_touched(t->d_leaves, ins, first, mask, b.leaf, b.slot, b.uk, b.uv, b.found, plan->m, nstart, t->fill,
                           t->sb_leaves, new_mins, s));
   // the streaming copy goes in paced chunks of 256 MiB (~0.1 ms): a search whose stream shares a
   // hardware queue with this one then waits behind one chunk, not the whole copy

@@ -228,9 +228,6 @@ hipError_t launch_range(const TreeView& tv, const uint64_t* start, const uint64_
                         uint64_t* out_keys, uint64_t* out_vals, uint32_t* out_counts, uint64_t capacity, hipStream_t s);
 
 // ---- update (hm_update.hip) ------------------------------------------------------------
-// Per-leaf insert counts for the not-found keys (keys sorted => leaf ids nondecreasing).
-hipError_t count_inserts(const uint32_t* leaf, const uint8_t* found, size_t n, uint32_t* ins_per_leaf,
-                         hipStream_t s);
 // Copy a batch into the staging arrays; *flag (mapped pinned memory, may be null) = 1 if a key is KEY_MAX.
 hipError_t stage_pairs(const uint64_t* k, const uint64_t* v, uint64_t* dk, uint64_t* dv, size_t n, uint32_t* flag,
                        hipStream_t s);
@@ -283,11 +280,14 @@ hipError_t node_respread(Leaf* leaves, uint64_t* last_level, uint32_t n_leaves, 
 // No leaf overflows: per run, overwrite the values of existing keys and merge the new keys in place.
 hipError_t apply_runs(Leaf* leaves, const uint32_t* leaf, const uint32_t* slot, const uint8_t* found,
                       const uint64_t* uk, const uint64_t* uv, size_t n, const uint32_t* dm, hipStream_t s);
-// Out of place: new leaf count per old leaf (1 if it fits, else ceil(total / fill)).
-hipError_t new_leaf_counts(const Leaf* leaves, const uint32_t* ins_per_leaf, size_t n_leaves, int fill,
-                           uint32_t* cnt, hipStream_t s);
-// first[leaf[j]] = j for the first batch index j of each leaf's run (first pre-filled with ~0).
-hipError_t leaf_first_keys(const uint32_t* leaf, size_t n, uint32_t* first, hipStream_t s);
+// The runs of the m located keys (sorted, so each leaf's form one): first[leaf] = its first entry h (first
+// pre-filled with ~0), mask[h] = the leaf's slots that entries overwrite, end[h] = the entry after the last.
+hipError_t run_bounds(const uint32_t* leaf, const uint32_t* slot, const uint8_t* found, size_t m, uint32_t* first,
+                      uint32_t* mask, uint32_t* end, hipStream_t s);
+// Out of place: new leaf count per old leaf (1 if it fits, else ceil(total / fill)), and the new keys (ins)
+// of each leaf with a run.
+hipError_t new_leaf_counts(const uint32_t* first, const uint32_t* mask, const uint32_t* end, const uint32_t* slot,
+                           size_t n_leaves, int fill, uint32_t* ins, uint32_t* cnt, hipStream_t s);
 // Re-layout into new_leaves (old leaves are only read); both parts also write each new leaf's
 // minimum key to new_mins[new leaf].
 //   relayout_copy: the old leaves in [lo, hi) that the batch does not touch, moved to new_start[i];
@@ -295,9 +295,9 @@ hipError_t leaf_first_keys(const uint32_t* leaf, size_t n, uint32_t* first, hipS
 //   overflowing leaves split evenly.
 hipError_t relayout_copy(const Leaf* old_leaves, size_t lo, size_t hi, const uint32_t* first, const uint32_t* new_start,
                          Leaf* new_leaves, uint64_t* new_mins, hipStream_t s);
-hipError_t relayout_touched(const Leaf* old_leaves, const uint32_t* ins_per_leaf, const uint32_t* bleaf,
-                            const uint32_t* bslot, const uint64_t* bkeys, const uint64_t* bvals, const uint8_t* found,
-                            size_t m, const uint32_t* new_start, int fill, Leaf* new_leaves, uint64_t* new_mins,
-                            hipStream_t s);
+hipError_t relayout_touched(const Leaf* old_leaves, const uint32_t* ins, const uint32_t* first, const uint32_t* mask,
+                            const uint32_t* bleaf, const uint32_t* bslot, const uint64_t* bkeys, const uint64_t* bvals,
+                            const uint8_t* found, size_t m, const uint32_t* new_start, int fill, Leaf* new_leaves,
+                            uint64_t* new_mins, hipStream_t s);
 
 }  // namespace hm

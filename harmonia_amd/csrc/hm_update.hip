@@ -13,7 +13,7 @@
 // launches: the keys are placed in order by counting, de-duplicated and located in one launch, each
 // leaf's keys form one run of the sorted batch, and one thread per run plans (overflow? how many new
 // keys?) and then applies it.  An epoch of 4001 keys (2^24 stored) with the read of its keys: 115 us in
-// 17 launches, now 60 us in six.
+// 17 launches, now 57 us in six.
 #include <algorithm>
 
 #include "hm_device.h"
@@ -89,13 +89,6 @@ __device__ __forceinline__ int leaf_count(const Leaf& l) {
   return c;
 }
 
-__global__ void count_inserts_kernel(const uint32_t* __restrict__ leaf, const uint8_t* __restrict__ found, size_t n,
-                                     uint32_t* __restrict__ ins) {
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-    if (!found[i]) atomicAdd(&ins[leaf[i]], 1u);
-}
-
 // Stream the merge of a leaf's keys with its inserts (the batch keys from `start` on that are not
 // found and map to this leaf; they are contiguous among the not-found keys because the batch is
 // sorted) in key order, calling emit(i, key, value) for i = 0, 1, ...; returns the merged count.
@@ -123,24 +116,52 @@ __device__ __forceinline__ int merge_leaf(const LeafRegs& l, uint32_t n_ins, uin
   return c;
 }
 
-__global__ void new_counts_kernel(const Leaf* __restrict__ leaves, const uint32_t* __restrict__ ins, size_t n_leaves,
-                                  int fill, uint32_t* __restrict__ cnt) {
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_leaves; i += stride) {
-    const uint32_t a = ins[i];
-    if (!a) {  // most leaves: no new key, one leaf; the leaf itself is not read
-      cnt[i] = 1u;
-      continue;
-    }
-    const uint32_t total = (uint32_t)leaf_count(leaves[i]) + a;
-    cnt[i] = total <= (uint32_t)LEAF_KEYS ? 1u : (total + fill - 1) / fill;
+__device__ __forceinline__ bool run_head(const uint32_t* __restrict__ leaf, uint32_t i) {
+  return i == 0 || leaf[i] != leaf[i - 1];
+}
+
+// Re-layout, the batch's runs: first[leaf] = the run's first entry, and there (two passes: the second looks
+// its run up in first) the leaf's slots that the batch overwrites as a bit mask and the run's end.  A run's
+// new keys are its entries less the mask's bits, so no thread walks a run and no two add to one word: 2^16
+// keys appended after the largest took 40 ms in one thread of the plan, 18 in one of the merge and 0.7 in
+// additions to one word; now all of it takes 25 us (an epoch: 50 ms, now 0.25).
+__global__ void run_heads_kernel(const uint32_t* __restrict__ leaf, uint32_t m, uint32_t* __restrict__ first,
+                                 uint32_t* __restrict__ mask) {
+  const uint32_t stride = gridDim.x * blockDim.x;
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += stride) {
+    mask[i] = 0;
+    if (run_head(leaf, i)) first[leaf[i]] = i;  // one writer per leaf
   }
 }
 
-__global__ void leaf_first_kernel(const uint32_t* __restrict__ leaf, size_t n, uint32_t* __restrict__ first) {
+__global__ void run_ends_kernel(const uint32_t* __restrict__ leaf, const uint32_t* __restrict__ slot,
+                                const uint8_t* __restrict__ found, uint32_t m, const uint32_t* __restrict__ first,
+                                uint32_t* __restrict__ mask, uint32_t* __restrict__ end) {
+  const uint32_t stride = gridDim.x * blockDim.x;
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += stride) {
+    const uint32_t L = leaf[i];
+    if (found[i]) atomicOr(&mask[first[L]], 1u << (slot[i] & 255u));
+    if (i + 1 == m || leaf[i + 1] != L) end[first[L]] = i + 1;
+  }
+}
+
+// New leaves per old leaf, and the new keys of the leaves that the batch touches (the locate step left the
+// free slots beside the slot: no leaf is read).
+__global__ void new_counts_kernel(const uint32_t* __restrict__ first, const uint32_t* __restrict__ mask,
+                                  const uint32_t* __restrict__ end, const uint32_t* __restrict__ slot, size_t n_leaves,
+                                  int fill, uint32_t* __restrict__ ins, uint32_t* __restrict__ cnt) {
   const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-    if (i == 0 || leaf[i] != leaf[i - 1]) first[leaf[i]] = (uint32_t)i;  // run heads: one writer per leaf
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_leaves; i += stride) {
+    const uint32_t h = first[i];
+    if (h == 0xFFFFFFFFu) {
+      cnt[i] = 1u;
+      continue;
+    }
+    const uint32_t a = end[h] - h - (uint32_t)__popc(mask[h]);
+    const uint32_t total = (uint32_t)LEAF_KEYS - (slot[h] >> 8) + a;
+    ins[i] = a;
+    cnt[i] = total <= (uint32_t)LEAF_KEYS ? 1u : (total + fill - 1) / fill;
+  }
 }
 
 // Re-layout, part 1: every leaf in [lo, hi) the batch does not touch moves unchanged to
@@ -167,54 +188,57 @@ __global__ __launch_bounds__(256) void relayout_copy_kernel(const Leaf* __restri
   }
 }
 
-// Re-layout, part 2: one thread per leaf the batch touches (a run head of the sorted batch): existing
-// keys get their new value in the copy, new keys are merged in, and a leaf that overflows is split
-// evenly into ceil(total / fill) leaves at new_start[L].
-__global__ void relayout_touched_kernel(const Leaf* __restrict__ old_leaves, const uint32_t* __restrict__ ins,
-                                        const uint32_t* __restrict__ bleaf, const uint32_t* __restrict__ bslot,
-                                        const uint64_t* __restrict__ bk, const uint64_t* __restrict__ bv,
-                                        const uint8_t* __restrict__ found, size_t m,
-                                        const uint32_t* __restrict__ new_start, int fill,
-                                        Leaf* __restrict__ new_leaves, uint64_t* __restrict__ new_mins) {
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t h = (size_t)blockIdx.x * blockDim.x + threadIdx.x; h < m; h += stride) {
-    if (h > 0 && bleaf[h] == bleaf[h - 1]) continue;  // not a run head
-    const uint32_t L = bleaf[h];
-    const uint32_t a = ins[L];
-    LeafRegs l = load_leaf(old_leaves + L);
-    for (size_t j = h; j < m && bleaf[j] == L; ++j)
-      if (found[j]) put(l.val, (int)(bslot[j] & 255u), bv[j]);
+// Re-layout, part 2: one thread per batch entry.  A leaf that overflows is split evenly into
+// ceil(total / fill) leaves at new_start[L]: part p holds the merged keys [p c / parts, (p + 1) c / parts),
+// at most ceil(c / parts) <= fill <= 8 each.  The entry's place among the merged keys follows from its slot
+// and from the new keys before it (entries since the run's head less those that overwrite a slot below its
+// own).  It also moves the leaf's keys between its slot and the next entry's (the head those below its own),
+// with the new value if it overwrites one.  Whoever places a part's last key pads the part.
+__global__ __launch_bounds__(256) void relayout_touched_kernel(
+    const Leaf* __restrict__ old_leaves, const uint32_t* __restrict__ ins, const uint32_t* __restrict__ first,
+    const uint32_t* __restrict__ mask, const uint32_t* __restrict__ bleaf, const uint32_t* __restrict__ bslot,
+    const uint64_t* __restrict__ bk, const uint64_t* __restrict__ bv, const uint8_t* __restrict__ found, uint32_t m,
+    const uint32_t* __restrict__ new_start, int fill, Leaf* __restrict__ new_leaves, uint64_t* __restrict__ new_mins) {
+  const uint32_t stride = gridDim.x * blockDim.x;
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += stride) {
+    const uint32_t L = bleaf[i], h = first[L], sl = bslot[i], s = sl & 255u;
+    const uint32_t cur = (uint32_t)LEAF_KEYS - (sl >> 8);
+    const uint32_t c = cur + ins[L];
+    const uint32_t parts = c <= (uint32_t)LEAF_KEYS ? 1u : (c + (uint32_t)fill - 1u) / (uint32_t)fill;
+    const bool upd = found[i] != 0;
+    const uint32_t before = i - h - (uint32_t)__popc(mask[h] & ((1u << s) - 1u));
+    const uint32_t j0 = i == h ? 0u : s;
+    const uint32_t j1 = i + 1 < m && bleaf[i + 1] == L ? bslot[i + 1] & 255u : cur;
     Leaf* dst = new_leaves + new_start[L];
     uint64_t* dmin = new_mins + new_start[L];
-    if (!a) {
-      store_leaf(dst, l);
-      *dmin = l.key[0];
-      continue;
-    }
-    // split the merged run evenly: part p holds merged keys [p*c/parts, (p+1)*c/parts),
-    // at most ceil(c/parts) <= fill <= 8 keys each
-    const int c = leaf_count(l) + (int)a;
-    const int parts = c <= LEAF_KEYS ? 1 : (c + fill - 1) / fill;
-    for (int p = 0; p < parts; ++p)
+    auto place = [&](uint32_t r, uint64_t k, uint64_t v) {
+      uint32_t p = 0, lo = 0, hi = c;
+      if (c > 65535u) {
+        p = (uint32_t)(((uint64_t)(r + 1) * parts - 1) / c);
+        lo = (uint32_t)((uint64_t)p * c / parts);
+        hi = (uint32_t)((uint64_t)(p + 1) * c / parts);
+      } else if (parts > 1) {  // the same in 32 bits: parts <= c
+        p = ((r + 1) * parts - 1) / c;
+        lo = p * c / parts;
+        hi = (p + 1) * c / parts;
+      }
+      const uint32_t q = r - lo;
+      dst[p].key[q] = k;
+      dst[p].val[q] = v;
+      if (q == 0) dmin[p] = k;  // every part gets at least one key
+      if (r + 1 == hi)
+        for (uint32_t x = q + 1; x < (uint32_t)LEAF_KEYS; ++x) {
+          dst[p].key[x] = KEY_MAX;
+          dst[p].val[x] = 0ull;
+        }
+    };
+    if (!upd) place(s + before, bk[i], bv[i]);
+    if (j0 >= j1) continue;
+    const LeafRegs l = load_leaf(old_leaves + L);
 #pragma unroll
-      for (int s = 0; s < LEAF_KEYS; ++s) {
-        dst[p].key[s] = KEY_MAX;
-        dst[p].val[s] = 0ull;
-      }
-    int part = 0, lo = 0, hi = c / parts;
-    merge_leaf(l, a, (uint32_t)h, bk, bv, found, [&](int idx, uint64_t k, uint64_t v) {
-      while (idx >= hi && part + 1 < parts) {
-        ++part;
-        lo = hi;
-        hi = (int)(((long long)(part + 1) * c) / parts);
-      }
-      const int slot = idx - lo;
-      if (slot < LEAF_KEYS) {
-        dst[part].key[slot] = k;
-        dst[part].val[slot] = v;
-      }
-      if (slot == 0) dmin[part] = k;  // every part gets at least one key
-    });
+    for (uint32_t j = 0; j < (uint32_t)LEAF_KEYS; ++j)
+      if (j >= j0 && j < j1)
+        place(j < s ? j : j + before + (upd ? 0u : 1u), l.key[j], upd && j == s ? bv[i] : l.val[j]);
   }
 }
 
@@ -305,8 +329,14 @@ __global__ __launch_bounds__(256) void dedupe_locate_kernel(TreeView tv, const u
   if (threadIdx.x == 0 && base + kPer >= n) *dm = before + (uint32_t)__popc(km);
 }
 
-__device__ __forceinline__ bool run_head(const uint32_t* __restrict__ leaf, uint32_t i) {
-  return i == 0 || leaf[i] != leaf[i - 1];
+// Whether the run that starts at entry i overflows its leaf: at most 17 entries are read, for a leaf has at
+// most 8 keys to overwrite and 8 free slots.
+__device__ __forceinline__ bool run_overflows(const uint32_t* __restrict__ leaf, const uint32_t* __restrict__ slot,
+                                              const uint8_t* __restrict__ found, uint32_t i, uint32_t m) {
+  const uint32_t L = leaf[i], room = slot[i] >> 8;
+  uint32_t ins = 0;
+  for (uint32_t j = i; ins <= room && j < m && leaf[j] == L; ++j) ins += found[j] ? 0u : 1u;
+  return ins > room;
 }
 
 // Plan an epoch, one thread per leaf the batch touches (its first batch entry: the batch is sorted, so a
@@ -318,59 +348,101 @@ __device__ __forceinline__ bool run_head(const uint32_t* __restrict__ leaf, uint
 // epoch needs a full re-layout).
 // The locate step left each entry's leaf's free slots beside its slot, so the plan reads leaves only for
 // nodes that overflow, and a thread walks one leaf's entries, not a node's: 2^20 entries took 61 us with
-// one thread per node reading its leaves, now 22.  The block that
+// one thread per node reading its leaves, now 22.  A node that overflows is planned by the wave that holds
+// its first overflowing leaf, 64 entries at a step (2^16 new keys, most nodes of 2^16 overflowing: 109 us
+// with one thread per node, now 14), and not at all once some node has asked for the re-layout (2^20 new
+// keys of 2^22: 528 us on average over epochs of both kinds, now 107).  The block that
 // finishes last writes the summary and the smallest and largest key to `host` (mapped pinned memory:
 // words 0..4 and the two u64 at word 8), in place of two more launches.
-__global__ void plan_runs_kernel(const Leaf* __restrict__ leaves, uint32_t n_leaves, int F,
+constexpr uint32_t kPlanList = 256;  // nodes that a block lists in LDS
+__global__ __launch_bounds__(256) void plan_runs_kernel(const Leaf* __restrict__ leaves, uint32_t n_leaves, int F,
                                  const uint32_t* __restrict__ leaf, const uint32_t* __restrict__ slot,
                                  const uint8_t* __restrict__ found, const uint64_t* __restrict__ uk, size_t n_max,
                                  const uint32_t* __restrict__ dm, uint32_t* __restrict__ summary,
                                  uint32_t* __restrict__ nlist, uint32_t* __restrict__ host) {
-  __shared__ uint32_t block_new;
+  __shared__ uint32_t block_new, block_full, block_nodes, block_at;
+  __shared__ uint32_t list[2 * kPlanList];
   __shared__ bool last_block;
-  if (threadIdx.x == 0) block_new = 0;
+  if (threadIdx.x == 0) block_new = block_full = block_nodes = 0;
   __syncthreads();
   const uint32_t m = dm ? *dm : (uint32_t)n_max;
   const uint32_t stride = gridDim.x * blockDim.x;
   const uint32_t uF = (uint32_t)F;
+  const uint32_t lane = threadIdx.x & 63;
   uint32_t my_new = 0;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += stride) {
-    const uint32_t L = leaf[i];
-    my_new += found[i] ? 0u : 1u;
-    if (i > 0 && leaf[i - 1] == L) continue;  // not the leaf's first entry
-    uint32_t ins = 0;
-    for (uint32_t j = i; j < m && leaf[j] == L; ++j) ins += found[j] ? 0u : 1u;
-    if (ins <= slot[i] >> 8) continue;
-    // the leaf overflows: the first such leaf of a node plans the node, from its first entry i0 on
-    const uint32_t node = L / uF;
-    uint32_t i0 = i;
-    while (i0 > 0 && leaf[i0 - 1] / uF == node) --i0;
-    uint32_t node_ins = 0;
-    bool first = true;
-    for (uint32_t j = i0; first && j < m && leaf[j] / uF == node;) {
-      const uint32_t x = leaf[j], room = slot[j] >> 8;
-      uint32_t c = 0;
-      for (; j < m && leaf[j] == x; ++j) c += found[j] ? 0u : 1u;
-      first = c <= room || x >= L;
-      node_ins += c;
+  for (uint32_t w = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); w < m; w += stride) {  // wave-uniform
+    const uint32_t i = w + lane;
+    uint32_t node = ~0u;  // no node: there are fewer than 2^32 leaves
+    bool over = false, isnew = false;
+    if (i < m) {
+      node = leaf[i] / uF;
+      isnew = !found[i];
+      over = run_head(leaf, i) && run_overflows(leaf, slot, found, i, m);
     }
-    if (!first) continue;
-    atomicOr(&summary[0], 1u);
-    const uint32_t x0 = node * uF, x1 = x0 + uF < n_leaves ? x0 + uF : n_leaves;
-    uint32_t total = node_ins;
-    for (uint32_t x = x0; x < x1; ++x) total += (uint32_t)leaf_count(leaves[x]);
-    if (total <= (x1 - x0) * (uint32_t)LEAF_KEYS) {
-      const uint32_t k = atomicAdd(&summary[4], 1u);
-      nlist[2 * k] = node;
-      nlist[2 * k + 1] = i0;
-    } else {
-      atomicOr(&summary[0], 2u);
+    my_new += isnew ? 1u : 0u;
+    uint64_t todo = __ballot(over);
+    if (todo && (__builtin_amdgcn_readfirstlane((int)__hip_atomic_load(&summary[0], __ATOMIC_RELAXED,
+                                                                       __HIP_MEMORY_SCOPE_AGENT)) & 2))
+      todo = 0;
+    while (todo) {  // wave-uniform: the nodes of the wave's overflowing leaves, one after the other
+      const uint32_t nd = (uint32_t)__builtin_amdgcn_readlane((int)node, __builtin_ctzll(todo));
+      const uint64_t in0 = __ballot(node == nd);
+      todo &= ~in0;
+      uint32_t node_new = (uint32_t)__popcll(in0 & __ballot(isnew));
+      uint32_t i0 = w + (uint32_t)__builtin_ctzll(in0);  // the node's first entry
+      bool first = true;
+      for (uint32_t b = w; b > 0 && i0 == b;) {  // back to it, unless an earlier leaf of the node overflows
+        b -= 64;
+        const uint32_t j = b + lane;
+        const bool in = leaf[j] / uF == nd;
+        first = !__any(in && run_head(leaf, j) && run_overflows(leaf, slot, found, j, m));
+        const uint64_t inb = __ballot(in);
+        if (!first || !inb) break;
+        i0 = b + (uint32_t)__builtin_ctzll(inb);
+        node_new += (uint32_t)__popcll(__ballot(in && !found[j]));
+      }
+      if (!first) continue;
+      const uint32_t x0 = nd * uF, x1 = x0 + uF < n_leaves ? x0 + uF : n_leaves;
+      const uint32_t cap = (x1 - x0) * (uint32_t)LEAF_KEYS;
+      bool more = in0 >> 63;
+      for (uint32_t b = w + 64; more && b < m && node_new <= cap; b += 64) {  // on to its last
+        const uint32_t j = b + lane;
+        const bool in = j < m && leaf[j] / uF == nd;
+        node_new += (uint32_t)__popcll(__ballot(in && !found[j]));
+        more = __all(in);
+      }
+      uint32_t total = 0;
+      for (uint32_t x = x0 + lane; x < x1; x += 64) total += (uint32_t)leaf_count(leaves[x]);
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) total += (uint32_t)__shfl_xor((int)total, o);
+      total += node_new;
+      if (lane == 0) {
+        if (total > cap) {
+          if (!atomicExch(&block_full, 1u)) atomicOr(&summary[0], 3u);  // at once: the others need not go on
+        } else {
+          const uint32_t k = atomicAdd(&block_nodes, 1u);
+          uint32_t* to = k < kPlanList ? list + 2 * k : nlist + 2 * atomicAdd(&summary[4], 1u);
+          to[0] = nd;
+          to[1] = i0;
+        }
+      }
     }
   }
   // new-key count: wave sum, then one LDS atomic per wave and one global atomic per block
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) my_new += __shfl_xor(my_new, o);
   if ((threadIdx.x & 63) == 0 && my_new) atomicAdd(&block_new, my_new);
+  __syncthreads();
+  // the block's nodes: one addition for their places (each takes about 10 ns, one after the other)
+  const uint32_t nodes = block_nodes < kPlanList ? block_nodes : kPlanList;
+  if (nodes > 0) {  // block-uniform
+    if (threadIdx.x == 0) {
+      atomicOr(&summary[0], 1u);
+      block_at = atomicAdd(&summary[4], nodes);
+    }
+    __syncthreads();
+    for (uint32_t x = threadIdx.x; x < 2 * nodes; x += blockDim.x) nlist[2 * block_at + x] = list[x];
+  }
   __syncthreads();  // waits for every thread's summary atomics, so they come before the block's count
   if (threadIdx.x == 0) {
     // new keys in the low word, finished blocks in the high one: one atomic per block.  (A device-scope
@@ -673,26 +745,21 @@ hipError_t apply_runs(Leaf* leaves, const uint32_t* leaf, const uint32_t* slot, 
   return hipGetLastError();
 }
 
-hipError_t count_inserts(const uint32_t* leaf, const uint8_t* found, size_t n, uint32_t* ins_per_leaf,
-                         hipStream_t s) {
-  if (!n) return hipSuccess;
+hipError_t run_bounds(const uint32_t* leaf, const uint32_t* slot, const uint8_t* found, size_t m, uint32_t* first,
+                      uint32_t* mask, uint32_t* end, hipStream_t s) {
+  if (!m) return hipSuccess;
   ProfScope prof("update", s);
-  hipLaunchKernelGGL(count_inserts_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, leaf, found, n, ins_per_leaf);
+  const dim3 grid(grid_for(m, 256));
+  hipLaunchKernelGGL(run_heads_kernel, grid, dim3(256), 0, s, leaf, (uint32_t)m, first, mask);
+  hipLaunchKernelGGL(run_ends_kernel, grid, dim3(256), 0, s, leaf, slot, found, (uint32_t)m, first, mask, end);
   return hipGetLastError();
 }
 
-hipError_t new_leaf_counts(const Leaf* leaves, const uint32_t* ins_per_leaf, size_t n_leaves, int fill, uint32_t* cnt,
-                           hipStream_t s) {
+hipError_t new_leaf_counts(const uint32_t* first, const uint32_t* mask, const uint32_t* end, const uint32_t* slot,
+                           size_t n_leaves, int fill, uint32_t* ins, uint32_t* cnt, hipStream_t s) {
   ProfScope prof("update", s);
-  hipLaunchKernelGGL(new_counts_kernel, dim3(grid_for(n_leaves, 256)), dim3(256), 0, s, leaves, ins_per_leaf,
-                     n_leaves, fill, cnt);
-  return hipGetLastError();
-}
-
-hipError_t leaf_first_keys(const uint32_t* leaf, size_t n, uint32_t* first, hipStream_t s) {
-  if (!n) return hipSuccess;
-  ProfScope prof("update", s);
-  hipLaunchKernelGGL(leaf_first_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, leaf, n, first);
+  hipLaunchKernelGGL(new_counts_kernel, dim3(grid_for(n_leaves, 256)), dim3(256), 0, s, first, mask, end, slot,
+                     n_leaves, fill, ins, cnt);
   return hipGetLastError();
 }
 
@@ -710,14 +777,14 @@ hipError_t relayout_copy(const Leaf* old_leaves, size_t lo, size_t hi, const uin
   return hipGetLastError();
 }
 
-hipError_t relayout_touched(const Leaf* old_leaves, const uint32_t* ins_per_leaf, const uint32_t* bleaf,
-                            const uint32_t* bslot, const uint64_t* bkeys, const uint64_t* bvals, const uint8_t* found,
-                            size_t m, const uint32_t* new_start, int fill, Leaf* new_leaves, uint64_t* new_mins,
-                            hipStream_t s) {
+hipError_t relayout_touched(const Leaf* old_leaves, const uint32_t* ins, const uint32_t* first, const uint32_t* mask,
+                            const uint32_t* bleaf, const uint32_t* bslot, const uint64_t* bkeys, const uint64_t* bvals,
+                            const uint8_t* found, size_t m, const uint32_t* new_start, int fill, Leaf* new_leaves,
+                            uint64_t* new_mins, hipStream_t s) {
   if (!m) return hipSuccess;
   ProfScope prof("update", s);
-  hipLaunchKernelGGL(relayout_touched_kernel, dim3(grid_for(m, 256)), dim3(256), 0, s, old_leaves, ins_per_leaf,
-                     bleaf, bslot, bkeys, bvals, found, m, new_start, fill, new_leaves, new_mins);
+  hipLaunchKernelGGL(relayout_touched_kernel, dim3(grid_for(m, 256)), dim3(256), 0, s, old_leaves, ins, first, mask,
+                     bleaf, bslot, bkeys, bvals, found, (uint32_t)m, new_start, fill, new_leaves, new_mins);
   return hipGetLastError();
 }
 
