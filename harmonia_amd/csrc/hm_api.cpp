@@ -287,9 +287,10 @@ int enqueue_pipeline(const TreeView& tv, const SearchLaunch& sl, int psa_bits, i
   const int top = out_mode == HM_OUT_PSA_ORDER ? 64 : std::max(std::min((int)tv.psa_top, 64), psa_bits);
   if (out_mode == HM_OUT_UNPERMUTE && partitions(sl, psa_bits)) {
     const int bits = partition_bits(n);
-    HM_TRY(partition_keys(dq, n, top, b.k0, b.replay, s, dn));
-    HM_TRY(launch_search_chunks(tv, b.k0, b.rv, b.rf, n, top, bits, s, dn));
-    HM_TRY(unpartition_results(b.rv, b.rf, n, b.replay, dvals, dfound, s, dn));
+    const Clash clash{(uint32_t*)b.ft, (uint8_t*)b.vt};
+    HM_TRY(partition_keys(dq, n, top, b.k0, b.replay, clash, s, dn));
+    HM_TRY(launch_search_chunks(tv, b.k0, b.rv, b.rf, n, top, bits, kMissMark, clash, s, dn));
+    HM_TRY(unpartition_results(b.rv, b.rf, n, b.replay, clash, dvals, dfound, s, dn));
     return HM_OK;
   }
   if (out_mode == HM_OUT_UNPERMUTE) {
@@ -310,7 +311,7 @@ int enqueue_pipeline(const TreeView& tv, const SearchLaunch& sl, int psa_bits, i
   ss.sorted = true;
   if (out_mode == HM_OUT_PSA_ORDER) {
     if (chunks_psa_order(tv, sl, psa_bits, n))
-      HM_TRY(launch_search_chunks(tv, sk, dvals, dfound, n, top, psa_bits, s, dn));
+      HM_TRY(launch_search_chunks(tv, sk, dvals, dfound, n, top, psa_bits, 0ull, Clash{}, s, dn));
     else
       HM_TRY(launch_search(tv, ss, sk, sp, dvals, dfound, n, OUT_DIRECT, s, dn));
     HM_TRY(hipMemcpyAsync(dpos, sp, n * 4, hipMemcpyDeviceToDevice, s));

@@ -116,10 +116,20 @@ hipError_t unsort_results(uint64_t* vals, uint8_t* found, size_t n, int bits, co
 constexpr int kPartMinBits = 8, kPartMaxBits = 11, kPartBucket = 4096;
 int partition_bits(size_t n);
 size_t partition_bytes(size_t n);
-hipError_t partition_keys(const uint64_t* q, size_t n, int top, uint64_t* out, void* rec, hipStream_t s,
-                          const uint32_t* dn);
+// Results on their way back: the value kMissMark means not found, so the found flags need not travel.  Unless
+// a key that was found has that very value: then *any (zeroed by the partition) and part[i / kClashPart] of its
+// place i are set, and there the flags tell.
+struct Clash {
+  uint32_t* any = nullptr;
+  uint8_t* part = nullptr;  // n / kClashPart + 2
+};
+constexpr uint32_t kClashPart = 2048;
+constexpr uint64_t kMissMark = 0xB5D19F6E03C7A28Dull;  // any value: rarer among stored ones than 0
+hipError_t partition_keys(const uint64_t* q, size_t n, int top, uint64_t* out, void* rec, const Clash& clash,
+                          hipStream_t s, const uint32_t* dn);
 hipError_t unpartition_results(const uint64_t* vals, const uint8_t* found, size_t n, const void* rec,
-                               uint64_t* out_vals, uint8_t* out_found, hipStream_t s, const uint32_t* dn);
+                               const Clash& clash, uint64_t* out_vals, uint8_t* out_found, hipStream_t s,
+                               const uint32_t* dn);
 
 // (key, value) pairs into buckets by the key bits [top - b, top), b = pair_bits(n) (0: too many pairs for
 // buckets of kPairBucket on average).  *totals = the 2^b bucket sizes (device).  A bucket above kBucketSortMax
@@ -195,9 +205,10 @@ enum SearchOut {
 hipError_t launch_search(const TreeView& tv, const SearchLaunch& sl, const uint64_t* q, const uint32_t* pos,
                          uint64_t* out_vals, uint8_t* out_found, size_t n, SearchOut mode, hipStream_t s,
                          const uint32_t* dn = nullptr);
-// Search of a partitioned batch (partition_keys over bits [top - bits, top)): result i of query q[i].
+// Search of a partitioned batch (partition_keys over bits [top - bits, top)): result i of query q[i].  Keys that
+// are not found get the value `miss`; with a clash record the flags are written only where it says so.
 hipError_t launch_search_chunks(const TreeView& tv, const uint64_t* q, uint64_t* out_vals, uint8_t* out_found, size_t n,
-                                int top, int bits, hipStream_t s, const uint32_t* dn);
+                                int top, int bits, uint64_t miss, Clash clash, hipStream_t s, const uint32_t* dn);
 // Bytes of LDS the top `levels` need.
 size_t lds_bytes_for(const TreeView& tv, int levels);
 // *p = v as a one-thread kernel (a graph-safe way to hand a count to the next replay).

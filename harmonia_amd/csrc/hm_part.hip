@@ -1,12 +1,13 @@
 // One-pass partition of a query batch for searches that return their results in input order, and its
 // undoing.
 //
-// Measured, 2^24 queries: histogram 32 us, scan 17, scatter 71, un-scatter 120, where the two 8-bit passes
-// took 58, 10, 132 and 159; 2^20 queries: 4.2, 4.8, 8.3 and 9.3 against 8.7, 8.5, 25 and 20.  The whole
-// search went 699 -> 589 us at 2^24 on 2^26 keys and 82 -> 46 us at 2^20 on 2^20.  What bounds it: memory at
-// the copy rate (the histogram reads 134 MB, the scatter moves 318 MB); the un-scatter's tiles wait for
-// their barriers and for 2048 short runs (nine or ten bits instead of eleven: 81 and 96 us, but the search
-// reads more leaves twice, 455 and 423 us for 404).
+// Measured, 2^24 queries: histogram 33 us, scan 17, scatter 72, un-scatter 92, where the two 8-bit passes
+// took 58, 10, 132 and 159; 2^20 queries: 4.0, 4.7, 8.9 and 9.8 against 8.7, 8.5, 25 and 20.  The whole
+// search went 699 -> 564 us at 2^24 on 2^26 keys and 82 -> 46 us at 2^20 on 2^20.  What bounds it: memory at
+// the copy rate (the histogram reads 134 MB, the scatter moves 318 MB); the un-scatter's 2048 short runs per
+// tile (nine or ten bits instead of eleven: 81 and 96 us for then 120, but the search reads more leaves
+// twice, 455 and 423 us for 404; 1024 threads per tile: 124).  It gathered the found flags too, a second
+// line per run: 120 us until a mark among the values took their place.
 //
 // Such a search may take its queries in any order that brings neighbours together, so the batch is split
 // once by the top bits of the tree's key range into buckets of a few thousand queries (histogram, scan,
@@ -40,10 +41,12 @@ unsigned grid_for(size_t nb) { return (unsigned)((nb + 7) / 8 * 8); }
 template <bool VEC>
 __global__ __launch_bounds__(kThreads) void part_hist_kernel(const uint64_t* __restrict__ keys, size_t n, int shift,
                                                              uint32_t nd, uint32_t* __restrict__ counts, uint32_t nb,
+                                                             uint32_t* __restrict__ clash,
                                                              const uint32_t* __restrict__ dn) {
   __shared__ uint32_t h[kDigits];
   const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
   if (tile >= nb) return;  // block-uniform
+  if (clash && tile == 0 && threadIdx.x == 0) *clash = 0;
   if (dn) n = *dn;         // tiles past n count nothing
   const uint32_t mask = nd - 1;
   for (uint32_t d = threadIdx.x; d < nd; d += kThreads) h[d] = 0;
@@ -228,7 +231,8 @@ __global__ __launch_bounds__(kThreads) void part_unscatter_kernel(const uint64_t
                                                                   uint8_t* __restrict__ fout,
                                                                   const uint16_t* __restrict__ place, size_t n,
                                                                   uint32_t nd, const uint32_t* __restrict__ offsets,
-                                                                  uint32_t nb, const uint32_t* __restrict__ dn) {
+                                                                  uint32_t nb, Clash clash,
+                                                                  const uint32_t* __restrict__ dn) {
   __shared__ __align__(16) uint64_t sv[kTile];       // first the digit of each index (16 bits)
   __shared__ __align__(16) uint32_t adj[kDigits];    // output minus tile offset; then the found flags
   __shared__ uint32_t scan_sh[kThreads / 64 + 1];
@@ -238,6 +242,7 @@ __global__ __launch_bounds__(kThreads) void part_unscatter_kernel(const uint64_t
   const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
   if (dn) n = *dn;
   if (tile >= nb || (size_t)tile * kTile >= n) return;  // block-uniform
+  const bool flags = *clash.any != 0;  // uniform
   const uint32_t d0 = threadIdx.x * kDPer;
   const size_t tile0 = (size_t)tile * kTile;
   const uint32_t cnt = (uint32_t)(n - tile0 < (size_t)kTile ? n - tile0 : (size_t)kTile);
@@ -306,13 +311,16 @@ __global__ __launch_bounds__(kThreads) void part_unscatter_kernel(const uint64_t
   }
   __syncthreads();
   uint64_t v[kItems];
-  uint8_t f[kItems];
+  uint32_t ff = 0;
 #pragma unroll
   for (int r = 0; r < kItems; ++r) {
     const uint32_t i = threadIdx.x + r * kThreads;
     const uint32_t src = i < cnt ? adj[dg[i]] + i : 0u;
     v[r] = i < cnt ? vin[src] : 0ull;
-    f[r] = i < cnt ? fin[src] : (uint8_t)0;
+    if (flags) {
+      const bool mark = i < cnt && v[r] == kMissMark;
+      ff |= (mark ? clash.part[src / kClashPart] && fin[src] : i < cnt) ? 1u << r : 0u;
+    }
   }
   __syncthreads();  // marks and offsets are read: their memory takes the results
 #pragma unroll
@@ -320,25 +328,32 @@ __global__ __launch_bounds__(kThreads) void part_unscatter_kernel(const uint64_t
     const uint32_t i = threadIdx.x + r * kThreads;
     if (i < cnt) {
       sv[i] = v[r];
-      sf[i] = f[r];
+      if (flags) sf[i] = (ff >> r) & 1u;
     }
   }
   __syncthreads();
+  auto result = [&](uint32_t l, uint64_t& val) -> uint32_t {
+    const uint64_t x = sv[l];
+    const uint32_t found = flags ? (uint32_t)sf[l] : (x != kMissMark ? 1u : 0u);
+    val = found ? x : 0ull;
+    return found;
+  };
   if constexpr (VEC) {
 #pragma unroll
     for (int r = 0; r < kItems / 4; ++r) {
       const uint32_t j0 = (threadIdx.x + r * kThreads) * 4;
       if (j0 + 3 < cnt) {
         const uint32_t l0 = pw[r].x & 0xFFFFu, l1 = pw[r].x >> 16, l2 = pw[r].y & 0xFFFFu, l3 = pw[r].y >> 16;
-        *reinterpret_cast<ulonglong2*>(vout + tile0 + j0) = make_ulonglong2(sv[l0], sv[l1]);
-        *reinterpret_cast<ulonglong2*>(vout + tile0 + j0 + 2) = make_ulonglong2(sv[l2], sv[l3]);
-        *reinterpret_cast<uint32_t*>(fout + tile0 + j0) =
-            (uint32_t)sf[l0] | ((uint32_t)sf[l1] << 8) | ((uint32_t)sf[l2] << 16) | ((uint32_t)sf[l3] << 24);
+        uint64_t a, b, c, d;
+        const uint32_t f = result(l0, a) | result(l1, b) << 8 | result(l2, c) << 16 | result(l3, d) << 24;
+        *reinterpret_cast<ulonglong2*>(vout + tile0 + j0) = make_ulonglong2(a, b);
+        *reinterpret_cast<ulonglong2*>(vout + tile0 + j0 + 2) = make_ulonglong2(c, d);
+        *reinterpret_cast<uint32_t*>(fout + tile0 + j0) = f;
       } else {
         for (uint32_t j = j0; j < cnt; ++j) {  // at most 3
-          const uint32_t l = place[tile0 + j];
-          vout[tile0 + j] = sv[l];
-          fout[tile0 + j] = sf[l];
+          uint64_t a;
+          fout[tile0 + j] = (uint8_t)result(place[tile0 + j], a);
+          vout[tile0 + j] = a;
         }
       }
     }
@@ -347,9 +362,9 @@ __global__ __launch_bounds__(kThreads) void part_unscatter_kernel(const uint64_t
     for (int r = 0; r < kItems; ++r) {
       const uint32_t j = threadIdx.x + r * kThreads;
       if (j < cnt) {
-        const uint32_t l = place[tile0 + j];
-        vout[tile0 + j] = sv[l];
-        fout[tile0 + j] = sf[l];
+        uint64_t a;
+        fout[tile0 + j] = (uint8_t)result(place[tile0 + j], a);
+        vout[tile0 + j] = a;
       }
     }
   }
@@ -435,8 +450,8 @@ int partition_bits(size_t n) {
 
 size_t partition_bytes(size_t n) { return offsets_bytes(n, partition_bits(n)) + (n * 2 + 255) / 256 * 256; }
 
-hipError_t partition_keys(const uint64_t* q, size_t n, int top, uint64_t* out, void* rec, hipStream_t s,
-                          const uint32_t* dn) {
+hipError_t partition_keys(const uint64_t* q, size_t n, int top, uint64_t* out, void* rec, const Clash& clash,
+                          hipStream_t s, const uint32_t* dn) {
   if (n == 0) return hipSuccess;
   const int bits = partition_bits(n);
   if (top < bits || top > 64) return hipErrorInvalidValue;
@@ -448,10 +463,10 @@ hipError_t partition_keys(const uint64_t* q, size_t n, int top, uint64_t* out, v
     ProfScope prof("psa_hist", s);
     if ((reinterpret_cast<uintptr_t>(q) & 15) == 0)
       hipLaunchKernelGGL(part_hist_kernel<true>, dim3(grid_for(nb)), dim3(kThreads), 0, s, q, n, shift, nd, offsets, nb,
-                         dn);
+                         clash.any, dn);
     else
       hipLaunchKernelGGL(part_hist_kernel<false>, dim3(grid_for(nb)), dim3(kThreads), 0, s, q, n, shift, nd, offsets,
-                         nb, dn);
+                         nb, clash.any, dn);
   }
   {
     ProfScope prof("scan", s);
@@ -483,10 +498,10 @@ hipError_t partition_pairs(const uint64_t* keys, const uint64_t* vals, size_t n,
   ProfScope prof("build", s);
   if ((reinterpret_cast<uintptr_t>(keys) & 15) == 0)
     hipLaunchKernelGGL(part_hist_kernel<true>, dim3(grid_for(nb)), dim3(kThreads), 0, s, keys, n, shift, nd, offsets, nb,
-                       (const uint32_t*)nullptr);
+                       (uint32_t*)nullptr, (const uint32_t*)nullptr);
   else
     hipLaunchKernelGGL(part_hist_kernel<false>, dim3(grid_for(nb)), dim3(kThreads), 0, s, keys, n, shift, nd, offsets,
-                       nb, (const uint32_t*)nullptr);
+                       nb, (uint32_t*)nullptr, (const uint32_t*)nullptr);
   hipLaunchKernelGGL(part_scan_kernel, dim3(nd / kScanDigits), dim3(kScanThreads), 0, s, offsets, nd, nb,
                      kBucketSortMax, flags, flag);
   hipLaunchKernelGGL(part_pairs_kernel, dim3(grid_for(nb)), dim3(kPairThreads), 0, s, keys, vals, kout, vout, n, shift,
@@ -496,7 +511,8 @@ hipError_t partition_pairs(const uint64_t* keys, const uint64_t* vals, size_t n,
 }
 
 hipError_t unpartition_results(const uint64_t* vals, const uint8_t* found, size_t n, const void* rec,
-                               uint64_t* out_vals, uint8_t* out_found, hipStream_t s, const uint32_t* dn) {
+                               const Clash& clash, uint64_t* out_vals, uint8_t* out_found, hipStream_t s,
+                               const uint32_t* dn) {
   if (n == 0) return hipSuccess;
   const int bits = partition_bits(n);
   const uint32_t nd = 1u << bits, nb = (uint32_t)((n + kTile - 1) / kTile);
@@ -505,10 +521,10 @@ hipError_t unpartition_results(const uint64_t* vals, const uint8_t* found, size_
   ProfScope prof("unsort", s);
   if ((reinterpret_cast<uintptr_t>(out_vals) & 15) == 0 && (reinterpret_cast<uintptr_t>(out_found) & 3) == 0)
     hipLaunchKernelGGL(part_unscatter_kernel<true>, dim3(grid_for(nb)), dim3(kThreads), 0, s, vals, found, out_vals,
-                       out_found, place, n, nd, offsets, nb, dn);
+                       out_found, place, n, nd, offsets, nb, clash, dn);
   else
     hipLaunchKernelGGL(part_unscatter_kernel<false>, dim3(grid_for(nb)), dim3(kThreads), 0, s, vals, found, out_vals,
-                       out_found, place, n, nd, offsets, nb, dn);
+                       out_found, place, n, nd, offsets, nb, clash, dn);
   return hipGetLastError();
 }
 

@@ -701,7 +701,7 @@ hipError_t launch_window(const TreeView& tv, const SearchLaunch& sl, const uint6
 // without the ring, with a reduction over each chunk's keys for the start node and over each run's nodes);
 // search_span_kernel over the fully sorted batch takes 362 us for 1.54 GB, but the second sorting pass that
 // needs costs 180.  2^20 queries of 2^20 keys: 19 us (27) against 21 plus 35 of sorting.  Over batches that
-// two passes sorted (PSA-order results), search_span_kernel's time in brackets: 2^24 of 2^26 keys 313 us
+// two passes sorted (PSA-order results), search_span_kernel's time in brackets: 2^24 of 2^26 keys 314 us
 // (386), 3000001 of 2^25 93 (101).
 constexpr int kChunkThreads = 512;
 constexpr int kChunkWaves = kChunkThreads / 64;
@@ -810,12 +810,14 @@ __device__ __forceinline__ uint64_t lds_read_8(uint32_t a) {
   return r;
 }
 
-// q: partitioned keys, by bits [top - bits, top).
+// q: partitioned keys, by bits [top - bits, top).  Keys that are not found get the value `miss`.  With a
+// clash record the flags are written only where a key that is found has that value too.
 template <int F, int I>
 __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv, const uint64_t* __restrict__ q,
                                                                      uint64_t* __restrict__ out_vals,
                                                                      uint8_t* __restrict__ out_found, uint32_t n,
-                                                                     int top, int bits,
+                                                                     int top, int bits, uint64_t miss,
+                                                                     Clash clash,
                                                                      const uint32_t* __restrict__ dn) {
   constexpr int NS = node_slots(F);
   constexpr int DPer = kChunkDigits / kChunkThreads;
@@ -825,7 +827,7 @@ __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv
   __shared__ __align__(16) uint8_t sf[kChunk];   // found flags
   // the digit counters, then the node runs, then the lists of leaves and the last third of the rings
   __shared__ __align__(16) uint64_t nbufs[kChunkWaves * kChunkNodeBytes / 8];
-  __shared__ uint32_t scan_sh[kChunkWaves + 1], at_root;
+  __shared__ uint32_t scan_sh[kChunkWaves + 1], at_root, alike;
   static_assert(sizeof(nbufs) >= kChunkDigits * 4, "the counters fit under the node runs");
   uint32_t* cnt = reinterpret_cast<uint32_t*>(nbufs);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -842,7 +844,7 @@ __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv
   const uint64_t kf = q[c0], kl = q[c0 + m - 1];  // uniform: the first and last bucket
 #pragma unroll
   for (int j = 0; j < DPer; ++j) cnt[j * kChunkThreads + threadIdx.x] = 0;
-  if (threadIdx.x == 0) at_root = 0;
+  if (threadIdx.x == 0) at_root = alike = 0;
   // the order's digit: bits below the first bucket's, shifted so that the chunk's buckets fit
   const int lo = top - bits > kChunkBits ? top - bits - kChunkBits : 0;
   const int ext = top - bits - lo;  // bits kept per bucket
@@ -976,13 +978,14 @@ __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv
   const uint32_t nbt = (nl + 15) / 16;
   for (uint32_t bt = 0; bt < 3 && bt < nbt; ++bt) issue(bt);
   uint32_t found = 0, cur = 0;
+  bool like_miss = false;
 #pragma unroll
   for (int j = 0; j < I; ++j) {
     if (p0 - lane + 64 * j >= m) break;  // wave-uniform
     const uint32_t mine = node[j];
     const uint32_t b0 = (uint32_t)__builtin_amdgcn_readlane((int)mine, 0) / 16;
     const uint32_t b1 = (uint32_t)__builtin_amdgcn_readlane((int)mine, 63) / 16;
-    uint64_t val = 0;
+    uint64_t val = miss;
     bool eq = false;
     for (uint32_t bt = b0; bt <= b1;) {  // wave-uniform
       const uint32_t be = bt + 2 < b1 ? bt + 2 : b1;  // batches bt .. be at once: nearly always the whole round
@@ -1014,8 +1017,15 @@ __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv
     }
     t[j] = val;
     found |= eq ? 1u << j : 0u;
+    like_miss |= eq && val == miss;
   }
+  if (__any(like_miss) && lane == 0) alike = 1;
   __syncthreads();  // every wave is done with its leaves
+  const bool flags = !clash.any || alike;  // block-uniform
+  if (clash.any && threadIdx.x < I / 4) {  // one byte per 2048 queries
+    clash.part[c0 / kClashPart + threadIdx.x] = (uint8_t)alike;
+    if (alike) *clash.any = 1u;
+  }
 #pragma unroll
   for (int j = 0; j < I; ++j) {
     sk[p0 + 64 * j] = t[j];
@@ -1027,24 +1037,24 @@ __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv
     const uint32_t i = r * kChunkThreads + threadIdx.x;
     if (i < m) {
       out_vals[c0 + i] = sk[pos[r]];
-      out_found[c0 + i] = sf[pos[r]];
+      if (flags) out_found[c0 + i] = sf[pos[r]];
     }
   }
 }
 
 template <int F, int I>
 hipError_t launch_chunk_i(const TreeView& tv, const uint64_t* q, uint64_t* out_vals, uint8_t* out_found, size_t n,
-                        int top, int bits, hipStream_t s, const uint32_t* dn) {
+                        int top, int bits, uint64_t miss, Clash clash, hipStream_t s, const uint32_t* dn) {
   constexpr size_t kChunk = kChunkThreads * I;
   const size_t nb = ((n + kChunk - 1) / kChunk + 7) / 8 * 8;
   hipLaunchKernelGGL((search_chunk_kernel<F, I>), dim3((unsigned)nb), dim3(kChunkThreads), 0, s, tv, q,
-                     out_vals, out_found, (uint32_t)n, top, bits, dn);
+                     out_vals, out_found, (uint32_t)n, top, bits, miss, clash, dn);
   return hipGetLastError();
 }
 
 template <int F>
 hipError_t launch_chunk(const TreeView& tv, const uint64_t* q, uint64_t* out_vals, uint8_t* out_found, size_t n,
-                        int top, int bits, hipStream_t s, const uint32_t* dn) {
+                        int top, int bits, uint64_t miss, Clash clash, hipStream_t s, const uint32_t* dn) {
   // 2048 queries per block while 4096 leave the chip idle (2^20 queries of 2^20 keys, the whole search: 46 us
   // for 51; 3 * 2^20 of 2^26: 159 for 170, of 2^20: 78 for 79), then 4096, whose ends read fewer leaves twice
   // (2^22 of 2^20 and of 2^23: 93 us for 94, 120 for 124; 2^23: 184 for 188, 229 for 239): where neighbours
@@ -1052,8 +1062,8 @@ hipError_t launch_chunk(const TreeView& tv, const uint64_t* q, uint64_t* out_val
   // for 346).
   const size_t round = (size_t)launch_cfg().num_cus * kChunkThreads * 8;
   if (n <= 3 * round || (n <= 5 * round && n <= tv.n_leaves))
-    return launch_chunk_i<F, kChunkGroup>(tv, q, out_vals, out_found, n, top, bits, s, dn);
-  return launch_chunk_i<F, 2 * kChunkGroup>(tv, q, out_vals, out_found, n, top, bits, s, dn);
+    return launch_chunk_i<F, kChunkGroup>(tv, q, out_vals, out_found, n, top, bits, miss, clash, s, dn);
+  return launch_chunk_i<F, 2 * kChunkGroup>(tv, q, out_vals, out_found, n, top, bits, miss, clash, s, dn);
 }
 
 // Locate for the update path: leaf id, lower_bound slot (low byte) with the leaf's free slots (next byte),
@@ -1264,13 +1274,13 @@ hipError_t launch_search(const TreeView& tv, const SearchLaunch& sl, const uint6
 }
 
 hipError_t launch_search_chunks(const TreeView& tv, const uint64_t* q, uint64_t* out_vals, uint8_t* out_found, size_t n,
-                                int top, int bits, hipStream_t s, const uint32_t* dn) {
+                                int top, int bits, uint64_t miss, Clash clash, hipStream_t s, const uint32_t* dn) {
   if (n == 0) return hipSuccess;
   ProfScope prof("search", s);
   switch (tv.fanout) {
-    case 32: return launch_chunk<32>(tv, q, out_vals, out_found, n, top, bits, s, dn);
-    case 64: return launch_chunk<64>(tv, q, out_vals, out_found, n, top, bits, s, dn);
-    case 128: return launch_chunk<128>(tv, q, out_vals, out_found, n, top, bits, s, dn);
+    case 32: return launch_chunk<32>(tv, q, out_vals, out_found, n, top, bits, miss, clash, s, dn);
+    case 64: return launch_chunk<64>(tv, q, out_vals, out_found, n, top, bits, miss, clash, s, dn);
+    case 128: return launch_chunk<128>(tv, q, out_vals, out_found, n, top, bits, miss, clash, s, dn);
     default: return hipErrorInvalidValue;
   }
 }

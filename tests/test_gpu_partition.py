@@ -149,3 +149,21 @@ def test_psa_order_results(gpu, F, n, low):
     assert np.array_equal(pos.cpu().numpy(), want)
     assert np.array_equal(f.cpu().numpy(), ef) and np.array_equal(v.cpu().numpy().view(np.uint64), ev)
     tree.close()
+
+
+@pytest.mark.parametrize("n", [70001, 3 * (1 << 20) + 1])
+@pytest.mark.parametrize("share", [0.0001, 0.3])
+def test_partition_found_values_like_the_miss_mark(gpu, n, share):
+    """Stored values equal to the one that stands for a miss on the way back."""
+    g = np.random.RandomState(11)
+    sk = np.unique(g.randint(0, 1 << 62, 50003)).astype(np.uint64)
+    sv = W.splitmix64_mix(sk)
+    sv[g.rand(len(sk)) < share] = np.uint64(0xB5D19F6E03C7A28D)
+    sv[7] = np.uint64(0)
+    sv[len(sk) // 2] = np.uint64(0xB5D19F6E03C7A28D)
+    tree = BPlusTree.from_keys(sk, sv, keys_sorted=True, fanout=64, leaf_fill=8)
+    q = np.where(g.rand(n) < 0.7, sk[g.randint(0, len(sk), n)], g.randint(0, 1 << 62, n).astype(np.uint64))
+    q[:2] = sk[[7, len(sk) // 2]]
+    check(tree, sk, sv, q)
+    check(tree, sk, sv, q, odd=True)
+    tree.close()
