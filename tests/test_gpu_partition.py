@@ -167,3 +167,27 @@ def test_partition_found_values_like_the_miss_mark(gpu, n, share):
     check(tree, sk, sv, q)
     check(tree, sk, sv, q, odd=True)
     tree.close()
+
+
+@pytest.mark.parametrize("bits", [1, 8, 9, 16, 17, 25])
+def test_psa_order_positions(gpu, bits):
+    """Positions of PSA-order results, odd places in memory: one, two (written in place), three and four passes."""
+    import torch
+
+    g = np.random.RandomState(12)
+    sk = np.unique(g.randint(0, 1 << 62, 30007)).astype(np.uint64)
+    tree = BPlusTree.from_keys(sk, sk, keys_sorted=True, fanout=64, leaf_fill=8)
+    for n in (1, 4097, 60001):
+        q = g.randint(0, 1 << 63, n).astype(np.uint64)
+        dq = torch.from_numpy(q.view(np.int64)).cuda()
+        v, f = torch.empty_like(dq), torch.empty(n, dtype=torch.uint8, device="cuda")
+        pos = torch.full((n + 2,), -1, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        tree.search_batch(dq, out_vals=v, out_found=f, out_pos=pos[1:n + 1], psa_bits=bits, sorted_output=True)
+        torch.cuda.synchronize()
+        want = np.argsort(q >> np.uint64(64 - bits), kind="stable")
+        pos = pos.cpu().numpy()
+        assert np.array_equal(pos[1:n + 1], want) and pos[0] == -1 and pos[n + 1] == -1
+        ev, ef = oracle.search_sorted(sk, sk, q[want])
+        assert np.array_equal(f.cpu().numpy(), ef) and np.array_equal(v.cpu().numpy().view(np.uint64), ev)
+    tree.close()
