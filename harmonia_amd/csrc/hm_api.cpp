@@ -643,7 +643,7 @@ int hm_tree_build(const uint64_t* keys, const uint64_t* vals, uint64_t n, const 
       if (bbits) {
         const uint32_t* totals = nullptr;
         BUILD_TRY(partition_pairs(dk, dv, n, hi, a0, a1, tmp, &d_sum->flags, kCrowded, &totals, s));
-        BUILD_TRY(bucket_sort_fill(a0, a1, n, bbits, totals, t->fill, t->d_leaves, mins, &d_sum->flags, kCrowded,
+        BUILD_TRY(bucket_sort_fill(a0, a1, n, hi, bbits, totals, t->fill, t->d_leaves, mins, &d_sum->flags, kCrowded,
                                    d_sum->edge, s));
         BUILD_TRY(hipMemcpyAsync(&sum, d_sum, sizeof(Summary), hipMemcpyDeviceToHost, s));
         BUILD_TRY(hipStreamSynchronize(s));

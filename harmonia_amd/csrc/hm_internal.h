@@ -264,9 +264,10 @@ hipError_t count_kept(const uint64_t* sorted_keys, size_t n, uint32_t* tile_kept
 // uv, the number of them to *dm.
 hipError_t compact_last(const uint64_t* sorted_keys, const uint32_t* index, const uint64_t* vals, size_t n,
                         const uint32_t* tile_kept, uint64_t* uk, uint64_t* uv, uint32_t* dm, hipStream_t s);
-// The buckets of partition_pairs sorted, one block each, straight into the leaves (and mins); flags |= 1 if a
-// key is KEY_MAX, |= 2 if two keys are equal; edge = the first and last key.  Nothing once *flags has `skip`.
-hipError_t bucket_sort_fill(const uint64_t* keys, const uint64_t* vals, size_t n, int bits, const uint32_t* totals,
+// The buckets of partition_pairs (with its top) sorted, one block each, straight into the leaves (and mins);
+// flags |= 1 if a key is KEY_MAX, |= 2 if two keys are equal; edge = the first and last key.  Nothing once
+// *flags has `skip`.
+hipError_t bucket_sort_fill(const uint64_t* keys, const uint64_t* vals, size_t n, int top, int bits, const uint32_t* totals,
                             int fill, Leaf* leaves, uint64_t* mins, uint32_t* flags, uint32_t skip, uint64_t* edge,
                             hipStream_t s);
 // Over the m located unique keys (sorted, so each leaf's keys form one run and each last-level

@@ -1,15 +1,16 @@
 // Stable merge sort of (key, staging index) for upsert batches, and the removal of all but the last write
 // of each key.
 //
-// Chunks of 4096 keys are sorted in LDS, then every pass merges pairs of runs.  Both steps are merges of
-// two sorted runs by tiles: a diagonal search splits the runs for each tile (merge path), the tile's keys
-// go to LDS, and each thread finds its own diagonal there and merges eight keys in registers.  Equal keys
-// of the left run go first, so the order of equal keys is the staging order.
+// Chunks of 4096 keys are sorted in LDS, by a digit if their keys spread over it and by merges if not, then
+// every pass merges pairs of runs.  Merges of two sorted runs go by tiles: a diagonal search splits the runs
+// for each tile (merge path), the tile's keys go to LDS, and each thread finds its own diagonal there and
+// merges eight keys in registers.  Equal keys of the left run go first, so the order of equal keys is the
+// staging order.
 //
 // What bounds it: latency, not bytes (a pass over 2^20 keys moves 25 MB, 5 us at the copy rate).  A pass
 // in which every key searched the other run in global memory (20 dependent reads) took 17 us, now 12;
 // the chunks, sorted before by eight LSD radix passes in LDS (36 us for 2^20 keys, one block per CU, a block
-// barrier every few hundred cycles), take 30.
+// barrier every few hundred cycles), take 30 by merges and 18 by a digit.
 #include <utility>
 
 #include "hm_block.h"
@@ -88,38 +89,137 @@ __device__ __forceinline__ void sort_eight(uint64_t (&k)[kPer], uint32_t (&ix)[k
       }
 }
 
+// n elements sorted by (key, element) into m without merges: by a digit of up to 11 bits, counted and placed
+// in LDS, then each key's rank among the few that share its digit.  k[r] is the key of element r NT + thread;
+// no key is padding.  False, for the whole block, if the keys crowd into few digits: then nothing is in m.
+constexpr int kOrderBits = 11;
+constexpr uint32_t kOrderDigits = 1u << kOrderBits;
+constexpr uint32_t kOrderMost = 32;  // keys that share a digit; 4096 to 5120 evenly spread ones: 2 on average
+template <int NT>
+struct OrderLds {
+  uint32_t cnt[kOrderDigits], sh[NT / 64 + 1], most;
+};
+template <int NT>
+__device__ __forceinline__ bool order_by_digit(MergeLds<NT>& m, OrderLds<NT>& o, const uint64_t (&k)[kPer], uint32_t n,
+                                               int shift, uint32_t mask) {
+  constexpr uint32_t D = (kOrderDigits + NT - 1) / NT;  // digits per thread
+  for (uint32_t d = threadIdx.x; d < kOrderDigits; d += NT) o.cnt[d] = 0;
+  if (threadIdx.x == 0) o.most = 0;
+  __syncthreads();
+  uint32_t at[kPer];
+#pragma unroll
+  for (int r = 0; r < kPer; ++r)
+    at[r] = r * NT + threadIdx.x < n ? atomicAdd(&o.cnt[(uint32_t)(k[r] >> shift) & mask], 1u) : 0u;
+  __syncthreads();
+  uint32_t c[D], s = 0, most = 0, total;
+#pragma unroll
+  for (uint32_t j = 0; j < D; ++j) {
+    const uint32_t d = threadIdx.x * D + j;
+    c[j] = d < kOrderDigits ? o.cnt[d] : 0u;
+    s += c[j];
+    most = c[j] > most ? c[j] : most;
+  }
+  if (most > kOrderMost) o.most = 1;
+  uint32_t run = block_exclusive_scan<uint32_t, NT>(s, o.sh, total);  // ends with a barrier
+  if (o.most) return false;
+#pragma unroll
+  for (uint32_t j = 0; j < D; ++j) {
+    const uint32_t d = threadIdx.x * D + j;
+    if (d < kOrderDigits) o.cnt[d] = run;
+    run += c[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint32_t i = r * NT + threadIdx.x;
+    if (i < n) {
+      const uint32_t p = slot_of(o.cnt[(uint32_t)(k[r] >> shift) & mask] + at[r]);
+      m.k[p] = k[r];
+      m.ix[p] = i;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint32_t i = r * NT + threadIdx.x;
+    if (i < n) {
+      const uint32_t d = (uint32_t)(k[r] >> shift) & mask;
+      const uint32_t b = o.cnt[d], e = d + 1 < kOrderDigits ? o.cnt[d + 1] : n;
+      uint32_t rank = 0;
+      for (uint32_t q = b; q < e; ++q) {
+        const uint64_t x = m.k[slot_of(q)];
+        rank += x < k[r] || (x == k[r] && m.ix[slot_of(q)] < i) ? 1u : 0u;
+      }
+      at[r] = slot_of(b + rank);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint32_t i = r * NT + threadIdx.x;
+    if (i < n) {
+      m.k[at[r]] = k[r];
+      m.ix[at[r]] = i;
+    }
+  }
+  __syncthreads();
+  return true;
+}
+
 // Chunk c of 4096 staged keys sorted by (key, index); block 0 zeroes the epoch's 8 summary words.
 __global__ __launch_bounds__(kChunkThreads) void chunk_sort_kernel(const uint64_t* __restrict__ pk, uint32_t n,
                                                                    uint64_t* __restrict__ ko,
                                                                    uint32_t* __restrict__ io,
                                                                    uint32_t* __restrict__ summary) {
   __shared__ MergeLds<kChunkThreads> m;
+  __shared__ OrderLds<kChunkThreads> order;
+  __shared__ uint64_t differ;
   constexpr uint32_t kChunk = kChunkThreads * kPer;
   if (blockIdx.x == 0 && threadIdx.x < 8) summary[threadIdx.x] = 0;
-  const uint32_t c0 = blockIdx.x * kChunk, e0 = c0 + threadIdx.x * kPer;
+  const uint32_t c0 = blockIdx.x * kChunk, cnt = n - c0 < kChunk ? n - c0 : kChunk;
   uint64_t k[kPer];
-  uint32_t ix[kPer];
-#pragma unroll
-  for (int r = 0; r < kPer; ++r) {
-    k[r] = e0 + r < n ? pk[e0 + r] : KEY_MAX;
-    ix[r] = e0 + r;
-  }
-  sort_eight(k, ix);
-  for (uint32_t w = kPer; w < kChunk; w <<= 1) {  // uniform across the block
-    put_eight(m, k, ix);
-    __syncthreads();
-    const uint32_t t0 = threadIdx.x * kPer, base = t0 & ~(2 * w - 1);
-    merge_eight(m, base, w, base + w, w, t0 - base, k, ix);
-    __syncthreads();
-  }
-  put_eight(m, k, ix);
-  __syncthreads();
 #pragma unroll
   for (int r = 0; r < kPer; ++r) {
     const uint32_t i = r * kChunkThreads + threadIdx.x;
-    if (c0 + i < n) {
+    k[r] = pk[c0 + (i < cnt ? i : 0u)];
+  }
+  // the digit: the 11 bits from the topmost one in which the chunk's keys differ
+  const uint64_t k0 = pk[c0];
+  uint64_t diff = 0;
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) diff |= k[r] ^ k0;
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) diff |= __shfl_xor(diff, s);
+  if (threadIdx.x == 0) differ = 0;
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) atomicOr(reinterpret_cast<unsigned long long*>(&differ), (unsigned long long)diff);
+  __syncthreads();
+  const int top = 64 - __builtin_clzll(differ | 1ull), shift = top > kOrderBits ? top - kOrderBits : 0;
+  if (!order_by_digit(m, order, k, cnt, shift, (1u << (top - shift)) - 1u)) {
+    const uint32_t t0 = threadIdx.x * kPer;
+    uint32_t ix[kPer];
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+      k[r] = t0 + r < cnt ? pk[c0 + t0 + r] : KEY_MAX;
+      ix[r] = t0 + r;
+    }
+    sort_eight(k, ix);
+    for (uint32_t w = kPer; w < kChunk; w <<= 1) {  // uniform across the block
+      put_eight(m, k, ix);
+      __syncthreads();
+      const uint32_t base = t0 & ~(2 * w - 1);
+      merge_eight(m, base, w, base + w, w, t0 - base, k, ix);
+      __syncthreads();
+    }
+    put_eight(m, k, ix);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint32_t i = r * kChunkThreads + threadIdx.x;
+    if (i < cnt) {
       ko[c0 + i] = m.k[slot_of(i)];
-      io[c0 + i] = m.ix[slot_of(i)];
+      io[c0 + i] = c0 + m.ix[slot_of(i)];
     }
   }
 }
@@ -288,18 +388,18 @@ __global__ __launch_bounds__(kTileThreads) void compact_last_kernel(const uint64
 
 // ---- bulk build ---------------------------------------------------------------------------------
 //
-// A bucket of the build's pairs (at most kBucketSortMax), sorted in LDS by merges like a chunk above, then
-// written to its leaves: sorted pair g goes to slot g % fill of leaf g / fill.  The values are read from the
-// bucket's own 40 KiB, which its block has just brought to L2.  4 million pairs: partition 45 us and this
-// kernel 132 (bound by the dependent LDS reads of its nine merges, two blocks per CU), where eight radix passes,
-// the validation, the leaf fill and the minima took 388; the build with one search of its keys went
-// 656 -> 385 us.
+// A bucket of the build's pairs (at most kBucketSortMax), sorted in LDS like a chunk above, then written to
+// its leaves: sorted pair g goes to slot g % fill of leaf g / fill.  The values are read from the bucket's own
+// 40 KiB, which its block has just brought to L2.  4 million pairs: partition 45 us and this kernel 66 (132
+// with nine merges in place of the digit), where eight radix passes, the validation, the leaf fill and the
+// minima took 388; the build with one search of its keys went 656 -> 318 us.
 constexpr int kBucketThreads = (int)kBucketSortMax / kPer;
 __global__ __launch_bounds__(kBucketThreads) void bucket_sort_fill_kernel(
-    const uint64_t* __restrict__ keys, const uint64_t* __restrict__ vals, size_t n, const uint32_t* __restrict__ totals,
-    uint32_t fill, Leaf* __restrict__ leaves, uint64_t* __restrict__ mins, uint32_t* __restrict__ flags, uint32_t skip,
+    const uint64_t* __restrict__ keys, const uint64_t* __restrict__ vals, size_t n, int shift,
+    const uint32_t* __restrict__ totals, uint32_t fill, Leaf* __restrict__ leaves, uint64_t* __restrict__ mins, uint32_t* __restrict__ flags, uint32_t skip,
     uint64_t* __restrict__ edge) {
   __shared__ MergeLds<kBucketThreads> m;
+  __shared__ OrderLds<kBucketThreads> order;
   __shared__ uint32_t part_w[kBucketThreads / 64], bad;
   if (*flags & skip) return;  // block-uniform: set before this launch
   const uint32_t cnt = totals[blockIdx.x];
@@ -314,26 +414,34 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_sort_fill_kernel(
   uint32_t start = 0;
 #pragma unroll
   for (int w = 0; w < kBucketThreads / 64; ++w) start += part_w[w];
-  const uint32_t t0 = threadIdx.x * kPer;
   uint64_t k[kPer];
-  uint32_t ix[kPer];
 #pragma unroll
   for (int r = 0; r < kPer; ++r) {
-    k[r] = t0 + r < cnt ? keys[start + t0 + r] : KEY_MAX;
-    ix[r] = t0 + r;
+    const uint32_t i = r * kBucketThreads + threadIdx.x;
+    k[r] = keys[start + (i < cnt ? i : 0u)];
   }
-  sort_eight(k, ix);
-  for (uint32_t w = kPer; w < cnt; w <<= 1) {  // uniform across the block
+  const int bits = shift < kOrderBits ? shift : kOrderBits;  // the digit: the bits below the bucket's
+  if (!order_by_digit(m, order, k, cnt, shift - bits, (1u << bits) - 1u)) {
+    const uint32_t t0 = threadIdx.x * kPer;
+    uint32_t ix[kPer];
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+      k[r] = t0 + r < cnt ? keys[start + t0 + r] : KEY_MAX;
+      ix[r] = t0 + r;
+    }
+    sort_eight(k, ix);
+    for (uint32_t w = kPer; w < cnt; w <<= 1) {  // uniform across the block
+      put_eight(m, k, ix);
+      __syncthreads();
+      const uint32_t base = t0 & ~(2 * w - 1);
+      const uint32_t na = base + w < kBucketSortMax ? w : kBucketSortMax - base;
+      const uint32_t nb = base + na + w < kBucketSortMax ? w : kBucketSortMax - base - na;
+      merge_eight(m, base, na, base + na, nb, t0 - base, k, ix);
+      __syncthreads();
+    }
     put_eight(m, k, ix);
     __syncthreads();
-    const uint32_t base = t0 & ~(2 * w - 1);
-    const uint32_t na = base + w < kBucketSortMax ? w : kBucketSortMax - base;
-    const uint32_t nb = base + na + w < kBucketSortMax ? w : kBucketSortMax - base - na;
-    merge_eight(m, base, na, base + na, nb, t0 - base, k, ix);
-    __syncthreads();
   }
-  put_eight(m, k, ix);
-  __syncthreads();
 #pragma unroll
   for (int r = 0; r < kPer; ++r) {
     const uint32_t i = r * kBucketThreads + threadIdx.x;
@@ -362,11 +470,12 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_sort_fill_kernel(
 
 }  // namespace
 
-hipError_t bucket_sort_fill(const uint64_t* keys, const uint64_t* vals, size_t n, int bits, const uint32_t* totals,
-                            int fill, Leaf* leaves, uint64_t* mins, uint32_t* flags, uint32_t skip, uint64_t* edge,
+hipError_t bucket_sort_fill(const uint64_t* keys, const uint64_t* vals, size_t n, int top, int bits,
+                            const uint32_t* totals, int fill, Leaf* leaves, uint64_t* mins, uint32_t* flags, uint32_t skip, uint64_t* edge,
                             hipStream_t s) {
   ProfScope prof("build", s);
-  hipLaunchKernelGGL(bucket_sort_fill_kernel, dim3(1u << bits), dim3(kBucketThreads), 0, s, keys, vals, n, totals,
+  hipLaunchKernelGGL(bucket_sort_fill_kernel, dim3(1u << bits), dim3(kBucketThreads), 0, s, keys, vals, n,
+                     top > bits ? top - bits : 0, totals,
                      (uint32_t)fill, leaves, mins, flags, skip, edge);
   return hipGetLastError();
 }
