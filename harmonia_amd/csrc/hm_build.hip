@@ -53,7 +53,10 @@ __global__ __launch_bounds__(256) void validate_sorted_kernel(const uint64_t* __
 }
 
 // ornor[0] |= or of the keys, ornor[1] |= or of their complements: the bits set in both vary.
-__global__ __launch_bounds__(256) void key_bits_kernel(const uint64_t* __restrict__ k, size_t n,
+// 256 blocks: their atomics on one word each take about 10 ns, one after the other (4 million keys: 9.0 us, 12.9
+// with 512 blocks of 256 threads).
+constexpr int kBitsThreads = 512, kBitsBlocks = 256;
+__global__ __launch_bounds__(kBitsThreads) void key_bits_kernel(const uint64_t* __restrict__ k, size_t n,
                                                        uint64_t* __restrict__ ornor) {
   __shared__ unsigned long long block_o[2];
   if (threadIdx.x < 2) block_o[threadIdx.x] = 0ull;
@@ -169,9 +172,8 @@ hipError_t validate_sorted(const uint64_t* keys, size_t n, uint32_t* d_flags, ui
 hipError_t key_bit_summary(const uint64_t* keys, size_t n, uint64_t* ornor, hipStream_t s) {
   if (n == 0) return hipSuccess;
   ProfScope prof("build", s);
-  int g = grid_for(n, 256);
-  if (g > kReduceBlocks) g = kReduceBlocks;
-  hipLaunchKernelGGL(key_bits_kernel, dim3(g), dim3(256), 0, s, keys, n, ornor);
+  const int g = std::min(grid_for(n, kBitsThreads), kBitsBlocks);
+  hipLaunchKernelGGL(key_bits_kernel, dim3(g), dim3(kBitsThreads), 0, s, keys, n, ornor);
   return hipGetLastError();
 }
 

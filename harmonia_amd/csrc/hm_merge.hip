@@ -396,8 +396,8 @@ __global__ __launch_bounds__(kTileThreads) void compact_last_kernel(const uint64
 constexpr int kBucketThreads = (int)kBucketSortMax / kPer;
 __global__ __launch_bounds__(kBucketThreads) void bucket_sort_fill_kernel(
     const uint64_t* __restrict__ keys, const uint64_t* __restrict__ vals, size_t n, int shift,
-    const uint32_t* __restrict__ totals, uint32_t fill, Leaf* __restrict__ leaves, uint64_t* __restrict__ mins, uint32_t* __restrict__ flags, uint32_t skip,
-    uint64_t* __restrict__ edge) {
+    const uint32_t* __restrict__ totals, uint32_t fill, Leaf* __restrict__ leaves, uint64_t* __restrict__ mins,
+    uint32_t* __restrict__ flags, uint32_t skip, uint64_t* __restrict__ edge) {
   __shared__ MergeLds<kBucketThreads> m;
   __shared__ OrderLds<kBucketThreads> order;
   __shared__ uint32_t part_w[kBucketThreads / 64], bad;
@@ -471,8 +471,8 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_sort_fill_kernel(
 }  // namespace
 
 hipError_t bucket_sort_fill(const uint64_t* keys, const uint64_t* vals, size_t n, int top, int bits,
-                            const uint32_t* totals, int fill, Leaf* leaves, uint64_t* mins, uint32_t* flags, uint32_t skip, uint64_t* edge,
-                            hipStream_t s) {
+                            const uint32_t* totals, int fill, Leaf* leaves, uint64_t* mins, uint32_t* flags,
+                            uint32_t skip, uint64_t* edge, hipStream_t s) {
   ProfScope prof("build", s);
   hipLaunchKernelGGL(bucket_sort_fill_kernel, dim3(1u << bits), dim3(kBucketThreads), 0, s, keys, vals, n,
                      top > bits ? top - bits : 0, totals,

@@ -348,14 +348,14 @@ __device__ __forceinline__ bool run_overflows(const uint32_t* __restrict__ leaf,
 // epoch needs a full re-layout).
 // The locate step left each entry's leaf's free slots beside its slot, so the plan reads leaves only for
 // nodes that overflow, and a thread walks one leaf's entries, not a node's: 2^20 entries took 61 us with
-// one thread per node reading its leaves, now 22.  A node that overflows is planned by the wave that holds
+// one thread per node reading its leaves, now 12.  A node that overflows is planned by the wave that holds
 // its first overflowing leaf, 64 entries at a step (2^16 new keys, most nodes of 2^16 overflowing: 109 us
-// with one thread per node, now 14), and not at all once some node has asked for the re-layout (2^20 new
-// keys of 2^22: 528 us on average over epochs of both kinds, now 107).  The block that
+// with one thread per node, now 11), and not at all once some node has asked for the re-layout (2^20 new
+// keys of 2^22: 528 us on average over epochs of both kinds, now 47).  The block that
 // finishes last writes the summary and the smallest and largest key to `host` (mapped pinned memory:
 // words 0..4 and the two u64 at word 8), in place of two more launches.
-constexpr uint32_t kPlanList = 256;  // nodes that a block lists in LDS
-__global__ __launch_bounds__(256) void plan_runs_kernel(const Leaf* __restrict__ leaves, uint32_t n_leaves, int F,
+constexpr uint32_t kPlanList = 1024;  // nodes that a block lists in LDS
+__global__ __launch_bounds__(1024) void plan_runs_kernel(const Leaf* __restrict__ leaves, uint32_t n_leaves, int F,
                                  const uint32_t* __restrict__ leaf, const uint32_t* __restrict__ slot,
                                  const uint8_t* __restrict__ found, const uint64_t* __restrict__ uk, size_t n_max,
                                  const uint32_t* __restrict__ dm, uint32_t* __restrict__ summary,
@@ -696,9 +696,12 @@ hipError_t plan_runs(const Leaf* leaves, uint32_t n_leaves, int F, const uint32_
                      uint32_t* nlist, uint32_t* host, hipStream_t s) {
   if (!n) return hipSuccess;
   ProfScope prof("update", s);
-  // at most 1024 blocks: each ends in an atomic on one word (~10 ns, one after the other)
-  hipLaunchKernelGGL(plan_runs_kernel, dim3(std::min(grid_for(n, 256), 1024)), dim3(256), 0, s, leaves, n_leaves, F, leaf, slot,
-                     found, uk, n, dm, summary, nlist, host);
+  // Few blocks, each ends in an atomic on one word (~10 ns, one after the other): 2^20 entries take 22 us with
+  // 1024 blocks of 256 threads, 16 with 512 of 512, 12 with 256 of 1024; 2^16 7.1 with 256 of 256, 5.4 with 64 of
+  // 1024.  Small batches are spread (4001: 4.2 with 16 blocks for 4.6 with 4).
+  const int threads = n >= (1u << 15) ? 1024 : 256;
+  hipLaunchKernelGGL(plan_runs_kernel, dim3(std::min(grid_for(n, threads), 256)), dim3(threads), 0, s, leaves,
+                     n_leaves, F, leaf, slot, found, uk, n, dm, summary, nlist, host);
   return hipGetLastError();
 }
 
