@@ -31,6 +31,13 @@ constexpr int kWaves = kThreads / 64;
 // instead of eight), above it eight, whose descents share the wave: 2^13 ranges of 16..256 pairs on
 // 2^26 keys 23 against 31 us, 2^14 32.4 against 34.7; 8192 waves are resident, so the gain ends there.
 constexpr uint32_t kOneMax = 16384;
+// Closed intervals may end anywhere before their capacity: a wave that lays eight ranges' leaves end to end
+// reads many for nothing, so above R = 1 they keep a group of 8 lanes each, which stops at the interval's end
+// (2^18 and 2^26 keys: 20000 of up to 256 pairs 24.8 and 28.2 us for 29.5 and 30.2, 200000 of up to 40 37 and 68
+// for 45 and 62, 10^6 of up to 256 1011 and 1297 for 971 and 1356).  R = 1 reaches further for long ones: 30000
+// of up to 256 25 and 39 us for 30 and 40, 60000 45 and 81 to 86 for 49 and 76 to 83; of up to 40 24 and 28 for 17
+// and 24.
+constexpr uint32_t kOneMaxShort = 12288, kOneMaxLong = 49152, kLongInterval = 64;
 constexpr int kWalk = 4;   // loads (8 leaves each) in flight per step, R = 1
 constexpr int kWalk8 = 3;  // the same, R = 8 (2 and 4 were slower, or even)
 
@@ -97,17 +104,15 @@ __device__ __forceinline__ uint32_t walk_range(const TreeView& tv, uint32_t leaf
   return got < L ? got : L;
 }
 
-// Pairs of a wave's eight ranges, range g held by lanes 8 g .. 8 g + 7 (s, h, L, off, the leaf of s; L = 0:
+// Pairs of a wave's eight ranges, range g held by lanes 8 g .. 8 g + 7 (s, L, off, the leaf of s; L = 0:
 // none).  The leaves that the ranges still need are laid end to end and each load takes the next eight of
 // them, whatever ranges they belong to, so short ranges fill the wave as well as long ones.  Returns the
 // lane's range's count.
-__device__ __forceinline__ uint32_t walk_ranges8(const TreeView& tv, uint32_t leaf, uint64_t s, uint64_t h,
-                                                 bool bounded, uint32_t L, uint64_t off,
-                                                 uint64_t* __restrict__ out_keys, uint64_t* __restrict__ out_vals,
-                                                 uint64_t capacity) {
-  // leaves of one range per round: a closed interval may end anywhere before its capacity, so it goes on
-  // in small steps; otherwise nearly every range is done in one round (leaves with free slots leave some)
-  const uint32_t most = bounded ? 8u : 1u << 16;
+__device__ __forceinline__ uint32_t walk_ranges8(const TreeView& tv, uint32_t leaf, uint64_t s, uint32_t L,
+                                                 uint64_t off, uint64_t* __restrict__ out_keys,
+                                                 uint64_t* __restrict__ out_vals, uint64_t capacity) {
+  // leaves of one range per round: nearly every range is done in one (leaves with free slots leave some)
+  constexpr uint32_t most = 1u << 16;
   const int lane = threadIdx.x & 63;
   const int kl = (lane & ~7) | (lane & 3);  // the lane that holds this lane's two keys
   const uint64_t below = (1ull << kl) - 1ull;
@@ -131,7 +136,6 @@ __device__ __forceinline__ uint32_t walk_ranges8(const TreeView& tv, uint32_t le
       T += lane_u32(need, 8 * r);
     }
     if (T == 0) break;
-    bool past_end = false;
     for (uint32_t t0 = 0; t0 < T; t0 += 8 * kWalk8) {  // wave-uniform
       ulonglong2 x[kWalk8];
       int src[kWalk8];
@@ -154,11 +158,11 @@ __device__ __forceinline__ uint32_t walk_ranges8(const TreeView& tv, uint32_t le
       for (int u = 0; u < kWalk8; ++u) {
         const uint32_t tb = t0 + 8 * u;
         if (tb >= T) break;  // wave-uniform
-        const uint64_t rs = __shfl(s, src[u]), rh = bounded ? __shfl(h, src[u]) : KEY_MAX;
+        const uint64_t rs = __shfl(s, src[u]);
         const uint64_t ro = __shfl(off, src[u]);
         const uint32_t rL = __shfl(L, src[u]), rg = __shfl(got, src[u]);
-        const bool t0k = is_key && x[u].x != KEY_MAX && x[u].x >= rs && x[u].x <= rh;
-        const bool t1k = is_key && x[u].y != KEY_MAX && x[u].y >= rs && x[u].y <= rh;
+        const bool t0k = is_key && x[u].x != KEY_MAX && x[u].x >= rs;
+        const bool t1k = is_key && x[u].y != KEY_MAX && x[u].y >= rs;
         const uint64_t m0 = __ballot(t0k), m1 = __ballot(t1k);
         // rank among the range's keys: those counted before plus the ones below in this load
         const uint32_t f = first[u] > tb ? first[u] - tb : 0u;  // the range's first slot here, 0..7
@@ -179,14 +183,10 @@ __device__ __forceinline__ uint32_t walk_ranges8(const TreeView& tv, uint32_t le
         const uint32_t e = mine + need > tb ? (mine + need - tb < 8 ? mine + need - tb : 8) : 0u;
         const uint64_t own = e > a ? (~0ull >> (64 - 8 * (e - a))) << (8 * a) : 0ull;
         got += (uint32_t)__popcll(m0 & own) + (uint32_t)__popcll(m1 & own);
-        if (bounded) {
-          const bool over = is_key && ((x[u].x != KEY_MAX && x[u].x > rh) || (x[u].y != KEY_MAX && x[u].y > rh));
-          past_end |= (__ballot(over) & own) != 0;
-        }
       }
     }
     leaf += need;
-    done = done || got >= L || past_end || leaf >= tv.n_leaves;
+    done = done || got >= L || leaf >= tv.n_leaves;
   }
   return got < L ? got : L;
 }
@@ -243,8 +243,77 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
       count = walk_range(tv, lane_u32(leaf, 0), lane_u64(s, 0), lane_u64(h, 0), lane_u32(want, 0), lane_u64(off, 0),
                          out_keys, out_vals, capacity);
     else
-      count = walk_ranges8(tv, leaf, s, h, hi != nullptr, want, off, out_keys, out_vals, capacity);
+      count = walk_ranges8(tv, leaf, s, want, off, out_keys, out_vals, capacity);
     if (valid && lane % (64 / R) == 0) out_counts[ri] = count;
+  }
+}
+
+// Closed intervals of large calls: 8 lanes per interval, up to eight of its leaves on their way at a time
+// (LDS-direct loads, a group's 8 lanes bring a whole leaf), consumed in order until one key lies past the end.
+constexpr int kWalkInterval = 8;
+template <int F>
+__global__ __launch_bounds__(kThreads) void interval_kernel(TreeView tv, const uint64_t* __restrict__ start,
+                                                            const uint64_t* __restrict__ hi, uint32_t L, uint32_t n,
+                                                            uint64_t offset_stride, uint64_t* __restrict__ out_keys,
+                                                            uint64_t* __restrict__ out_vals,
+                                                            uint32_t* __restrict__ out_counts, uint64_t capacity) {
+  constexpr int G = 8;
+  constexpr uint32_t gpb = kThreads / G;
+  typedef __attribute__((address_space(1))) void global_void_t;
+  typedef __attribute__((address_space(3))) void lds_void_t;
+  // the wave's leaves of one step: step u holds its 8 groups' leaves, lane l's 16-byte piece at byte 16 l
+  __shared__ __align__(16) uint64_t lbuf[kWaves][kWalkInterval][128];
+  uint64_t* wb = &lbuf[threadIdx.x >> 6][0][0];
+  const int lane = threadIdx.x & 63, gl = lane % G, gbase = lane - gl;
+  const uint64_t lanes_below = (1ull << gl) - 1ull;
+  for (uint32_t rb = blockIdx.x * gpb; rb < n; rb += gridDim.x * gpb) {  // uniform across the block
+    const uint32_t ri = rb + threadIdx.x / G;
+    const bool valid = ri < n;
+    const uint64_t s = valid ? start[ri] : 0ull, h = valid ? hi[ri] : 0ull;
+    const uint64_t off = (uint64_t)ri * offset_stride;
+    uint32_t leaf = descend<F, G>(tv, 0, nullptr, s == KEY_MAX ? KEY_MAX - 1 : s, gl, gbase);
+    uint32_t got = 0;
+    bool done = !valid || L == 0 || s > h || s == KEY_MAX;
+    while (!done) {  // uniform inside the group
+      uint64_t k[kWalkInterval], v[kWalkInterval];
+      const uint64_t need = ((uint64_t)(L - got) + LEAF_KEYS - 1) / LEAF_KEYS + 1;  // got < L here
+      const uint32_t step = need < (uint64_t)kWalkInterval ? (uint32_t)need : (uint32_t)kWalkInterval;
+#pragma unroll
+      for (int u = 0; u < kWalkInterval; ++u)
+        if ((uint32_t)u < step) {  // group-uniform; the load writes LDS only
+          const uint32_t lf = leaf + u < tv.n_leaves ? leaf + u : tv.n_leaves - 1;
+          __builtin_amdgcn_global_load_lds(
+              (const global_void_t*)(reinterpret_cast<const ulonglong2*>(tv.leaves + lf) + gl),
+              (lds_void_t*)(wb + u * 128), 16, 0, 0);
+        }
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's leaves are in LDS
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int u = 0; u < kWalkInterval; ++u) {
+        const bool in = (uint32_t)u < step && leaf + u < tv.n_leaves;
+        const uint64_t* lp = wb + u * 128 + gbase * 2;  // this group's leaf
+        k[u] = in ? lp[gl] : KEY_MAX;
+        v[u] = in ? lp[8 + gl] : 0ull;
+      }
+      __builtin_amdgcn_wave_barrier();  // the next step's loads overwrite the buffer after these reads
+#pragma unroll
+      for (int u = 0; u < kWalkInterval; ++u)
+        if (!done && (uint32_t)u < step) {  // group-uniform
+          const bool take = k[u] != KEY_MAX && k[u] >= s && k[u] <= h;
+          const uint64_t m = (__ballot(take) >> gbase) & 0xFFull;
+          const uint64_t beyond = (__ballot(k[u] != KEY_MAX && k[u] > h) >> gbase) & 0xFFull;
+          const uint32_t rank = got + (uint32_t)__popcll(m & lanes_below);
+          const uint64_t o = off + rank;
+          if (take && rank < L && o < capacity) {
+            out_keys[o] = k[u];
+            out_vals[o] = v[u];
+          }
+          got += (uint32_t)__popcll(m);
+          done = got >= L || beyond != 0 || leaf + u + 1 >= tv.n_leaves;
+        }
+      leaf += step;
+    }
+    if (valid && gl == 0) out_counts[ri] = got < L ? got : L;
   }
 }
 
@@ -258,7 +327,8 @@ void launch_range_f(const TreeView& tv, const uint64_t* start, const uint64_t* h
                     uint64_t* out_keys, uint64_t* out_vals, uint32_t* out_counts, uint64_t capacity, hipStream_t s) {
   const size_t cus = (size_t)launch_cfg().num_cus;
   const size_t max_nb = cus * 8;
-  if (n <= kOneMax) {
+  const uint32_t one = !hi ? kOneMax : cap_const < kLongInterval ? kOneMaxShort : kOneMaxLong;
+  if (n <= one) {
     const size_t nb = std::min<size_t>((n + kWaves - 1) / kWaves, max_nb);
     if (scan)
       hipLaunchKernelGGL((range_kernel<F, 1, true>), dim3((unsigned)nb), dim3(kThreads), 0, s, tv, start, hi, len,
@@ -266,8 +336,12 @@ void launch_range_f(const TreeView& tv, const uint64_t* start, const uint64_t* h
     else
       hipLaunchKernelGGL((range_kernel<F, 1, false>), dim3((unsigned)nb), dim3(kThreads), 0, s, tv, start, hi, len,
                          cap_const, n, offsets, offset_stride, out_keys, out_vals, out_counts, capacity);
+  } else if (hi) {
+    const size_t nb = std::min<size_t>((n + kWaves * 8 - 1) / (kWaves * 8), max_nb);
+    hipLaunchKernelGGL(interval_kernel<F>, dim3((unsigned)nb), dim3(kThreads), 0, s, tv, start, hi, cap_const, n,
+                       offset_stride, out_keys, out_vals, out_counts, capacity);
   } else {
-    size_t nb = std::min<size_t>((n + kWaves * 8 - 1) / (kWaves * 8), max_nb);
+    const size_t nb = std::min<size_t>((n + kWaves * 8 - 1) / (kWaves * 8), max_nb);
     hipLaunchKernelGGL((range_kernel<F, 8, false>), dim3((unsigned)nb), dim3(kThreads), 0, s, tv, start, hi, len,
                        cap_const, n, offsets, offset_stride, out_keys, out_vals, out_counts, capacity);
   }
@@ -282,6 +356,7 @@ hipError_t launch_range(const TreeView& tv, const uint64_t* start, const uint64_
                         hipStream_t s) {
   if (n == 0) return hipSuccess;
   if (scan && (n > kRangeScanMax || !len || !offsets)) return hipErrorInvalidValue;
+  if (hi && (len || offsets)) return hipErrorInvalidValue;  // closed intervals: cap_const each, evenly spaced
   ProfScope prof("range", s);
   switch (tv.fanout) {
     case 32:
