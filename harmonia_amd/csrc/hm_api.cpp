@@ -1049,7 +1049,7 @@ struct UpdBufs {
   uint32_t *leaf, *slot;
   uint32_t* nlist;  // nodes to re-spread: (node, first batch entry) pairs
   uint8_t* found;
-  uint32_t* summary;  // [0] overflow, [2] unique count, [4] nodes listed, [6] new keys, [7] plan blocks done
+  uint32_t* summary;  // [2] unique count, the rest plan_runs' (hm_update.hip)
 };
 // Words of hm_tree::upd_host: the plan summary in 0..4, its edge keys as two u64 at 8, the staging flag.
 constexpr int kHostEdge = 8, kHostFlag = 16;

@@ -271,12 +271,13 @@ hipError_t bucket_sort_fill(const uint64_t* keys, const uint64_t* vals, size_t n
                             int fill, Leaf* leaves, uint64_t* mins, uint32_t* flags, uint32_t skip, uint64_t* edge,
                             hipStream_t s);
 // Over the m located unique keys (sorted, so each leaf's keys form one run and each last-level
-// node's keys one range): counts the new keys; summary[0] |= 1 if some leaf would exceed
-// 8 keys.  Such a node goes on the re-spread list (nlist: pairs of node index within the last level and
-// first batch entry; summary[4] = their count) when its leaves can hold all its keys, else
-// summary[0] |= 2 (a full re-layout is needed).  n sizes the grid; nlist holds 2 n entries; summary (8
-// words, zeroed) counts new keys in [6] and finished blocks in [7].  host (mapped pinned memory) receives
-// summary[0], the new keys, summary[2..4] and, as two u64 at word 8, the smallest and largest of the *dm sorted unique keys (KEY_MAX, 0 if none).
+// node's keys one range): counts the new keys and finds the leaves that would exceed 8 keys.  The node of
+// such a leaf goes on the re-spread list (nlist: pairs of node index within the last level and first batch
+// entry; summary[4] = their count) when its leaves can hold all its keys, else a full re-layout is needed.
+// n sizes the grid; nlist holds 2 n entries; summary (8 words, zeroed) is the kernel's.  host (mapped pinned
+// memory) receives in word 0 bit 0 if some leaf overflows and bit 1 if a re-layout is needed (the list is
+// then incomplete), the new keys, summary[2..4] and, as two u64 at word 8, the smallest and largest of the
+// *dm sorted unique keys (KEY_MAX, 0 if none).
 hipError_t plan_runs(const Leaf* leaves, uint32_t n_leaves, int F, const uint32_t* leaf, const uint32_t* slot,
                      const uint8_t* found, const uint64_t* uk, size_t n, const uint32_t* dm, uint32_t* summary,
                      uint32_t* nlist, uint32_t* host, hipStream_t s);

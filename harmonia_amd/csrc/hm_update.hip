@@ -342,10 +342,12 @@ __device__ __forceinline__ bool run_overflows(const uint32_t* __restrict__ leaf,
 // Plan an epoch, one thread per leaf the batch touches (its first batch entry: the batch is sorted, so a
 // leaf's and a node's entries are contiguous).  Last-level node j holds leaves
 // [j F, min((j + 1) F, n_leaves)): the bulk build and re-layouts fill every node but the last, and
-// an in-node re-spread keeps each node's leaf count.  summary[1] += new keys; if a leaf of the node
-// would overflow, summary[0] |= 1 and the node either goes on the re-spread list (nlist: node, first
-// batch entry; count in summary[4]) when its leaves can hold all its keys, or summary[0] |= 2 (the
-// epoch needs a full re-layout).
+// an in-node re-spread keeps each node's leaf count.  If a leaf of a node would overflow, the node goes
+// on the re-spread list (nlist: node, first batch entry; count in summary[4]) when its leaves can hold all
+// its keys, or else the epoch needs a full re-layout (summary[0] tells the other waves early: a hint).
+// What a block has found (new keys, a node listed, a full node) travels in the one addition to summary[6..7]
+// that also counts the block as finished: the block that finishes last has it all from the value returned,
+// and no order among separate words matters (a barrier waits for no atomic whose result is unused).
 // The locate step left each entry's leaf's free slots beside its slot, so the plan reads leaves only for
 // nodes that overflow, and a thread walks one leaf's entries, not a node's: 2^20 entries took 61 us with
 // one thread per node reading its leaves, now 12.  A node that overflows is planned by the wave that holds
@@ -355,6 +357,10 @@ __device__ __forceinline__ bool run_overflows(const uint32_t* __restrict__ leaf,
 // finishes last writes the summary and the smallest and largest key to `host` (mapped pinned memory:
 // words 0..4 and the two u64 at word 8), in place of two more launches.
 constexpr uint32_t kPlanList = 1024;  // nodes that a block lists in LDS
+// The word of that addition: new keys (fewer than 2^31 entries), then three counts of blocks, ten bits each.
+constexpr int kPlanBlocks = 256;
+constexpr int kPlanDone = 32, kPlanListed = 42, kPlanFull = 52;
+static_assert(kPlanBlocks < 1024, "a count of blocks fits ten bits");
 __global__ __launch_bounds__(1024) void plan_runs_kernel(const Leaf* __restrict__ leaves, uint32_t n_leaves, int F,
                                  const uint32_t* __restrict__ leaf, const uint32_t* __restrict__ slot,
                                  const uint8_t* __restrict__ found, const uint64_t* __restrict__ uk, size_t n_max,
@@ -362,7 +368,7 @@ __global__ __launch_bounds__(1024) void plan_runs_kernel(const Leaf* __restrict_
                                  uint32_t* __restrict__ nlist, uint32_t* __restrict__ host) {
   __shared__ uint32_t block_new, block_full, block_nodes, block_at;
   __shared__ uint32_t list[2 * kPlanList];
-  __shared__ bool last_block;
+  __shared__ uint64_t all_found;
   if (threadIdx.x == 0) block_new = block_full = block_nodes = 0;
   __syncthreads();
   const uint32_t m = dm ? *dm : (uint32_t)n_max;
@@ -418,7 +424,7 @@ __global__ __launch_bounds__(1024) void plan_runs_kernel(const Leaf* __restrict_
       total += node_new;
       if (lane == 0) {
         if (total > cap) {
-          if (!atomicExch(&block_full, 1u)) atomicOr(&summary[0], 3u);  // at once: the others need not go on
+          if (!atomicExch(&block_full, 1u)) atomicOr(&summary[0], 2u);  // at once: the others need not go on
         } else {
           const uint32_t k = atomicAdd(&block_nodes, 1u);
           uint32_t* to = k < kPlanList ? list + 2 * k : nlist + 2 * atomicAdd(&summary[4], 1u);
@@ -436,28 +442,25 @@ __global__ __launch_bounds__(1024) void plan_runs_kernel(const Leaf* __restrict_
   // the block's nodes: one addition for their places (each takes about 10 ns, one after the other)
   const uint32_t nodes = block_nodes < kPlanList ? block_nodes : kPlanList;
   if (nodes > 0) {  // block-uniform
-    if (threadIdx.x == 0) {
-      atomicOr(&summary[0], 1u);
-      block_at = atomicAdd(&summary[4], nodes);
-    }
+    if (threadIdx.x == 0) block_at = atomicAdd(&summary[4], nodes);
     __syncthreads();
     for (uint32_t x = threadIdx.x; x < 2 * nodes; x += blockDim.x) nlist[2 * block_at + x] = list[x];
   }
-  __syncthreads();  // waits for every thread's summary atomics, so they come before the block's count
+  __syncthreads();  // every wave has the results of its additions to summary[4], its list places
   if (threadIdx.x == 0) {
-    // new keys in the low word, finished blocks in the high one: one atomic per block.  (A device-scope
-    // fence instead of the barrier above would write the L2 back, in every block: 0.25 ms for 2^20 entries.)
-    const uint64_t mine = (1ull << 32) | block_new;
-    const uint64_t old = atomicAdd(reinterpret_cast<unsigned long long*>(summary + 6), (unsigned long long)mine);
-    last_block = (uint32_t)(old >> 32) == gridDim.x - 1;
-    block_new += (uint32_t)old;  // in the last block: every new key
+    // (A device-scope fence in every block would write the L2 back: 0.25 ms for 2^20 entries.)
+    const uint64_t mine = (uint64_t)block_new | 1ull << kPlanDone | (nodes ? 1ull << kPlanListed : 0ull) |
+                          (block_full ? 1ull << kPlanFull : 0ull);
+    all_found = mine + atomicAdd(reinterpret_cast<unsigned long long*>(summary + 6), (unsigned long long)mine);
   }
   __syncthreads();
-  if (!last_block) return;  // every block's atomics are done
+  const uint64_t all = all_found;
+  if (((all >> kPlanDone) & 1023u) != gridDim.x) return;  // not the last block
   if (threadIdx.x < 5)
-    host[threadIdx.x] = threadIdx.x == 1 ? block_new
-                                         : __hip_atomic_load(&summary[threadIdx.x], __ATOMIC_RELAXED,
-                                                             __HIP_MEMORY_SCOPE_AGENT);
+    host[threadIdx.x] = threadIdx.x == 0   ? (all >> kPlanFull ? 3u : (all >> kPlanListed) & 1023u ? 1u : 0u)
+                        : threadIdx.x == 1 ? (uint32_t)all
+                                           : __hip_atomic_load(&summary[threadIdx.x], __ATOMIC_RELAXED,
+                                                               __HIP_MEMORY_SCOPE_AGENT);
   if (threadIdx.x == 64) {
     uint64_t* edge = reinterpret_cast<uint64_t*>(host + 8);
     edge[0] = m ? uk[0] : KEY_MAX;
@@ -700,7 +703,7 @@ hipError_t plan_runs(const Leaf* leaves, uint32_t n_leaves, int F, const uint32_
   // 1024 blocks of 256 threads, 16 with 512 of 512, 12 with 256 of 1024; 2^16 7.1 with 256 of 256, 5.4 with 64 of
   // 1024.  Small batches are spread (4001: 4.2 with 16 blocks for 4.6 with 4).
   const int threads = n >= (1u << 15) ? 1024 : 256;
-  hipLaunchKernelGGL(plan_runs_kernel, dim3(std::min(grid_for(n, threads), 256)), dim3(threads), 0, s, leaves,
+  hipLaunchKernelGGL(plan_runs_kernel, dim3(std::min(grid_for(n, threads), kPlanBlocks)), dim3(threads), 0, s, leaves,
                      n_leaves, F, leaf, slot, found, uk, n, dm, summary, nlist, host);
   return hipGetLastError();
 }
