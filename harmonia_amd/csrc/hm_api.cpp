@@ -441,28 +441,28 @@ int rebuild_inner(hm_tree* t, const Levels& lv, bool mins_ready, hipStream_t s) 
 
 void free_tree(hm_tree* t) {
   if (!t) return;
-  if (t->own) (void)hipStreamSynchronize(t->own);
+  const bool own_idle = t->own && hipStreamSynchronize(t->own) == hipSuccess;
   for (hipStream_t h : t->hs)
     if (h) (void)hipStreamSynchronize(h);
-  (void)hipDeviceSynchronize();  // work on any stream may still use the arrays
+  const bool idle = dev_wait() == hipSuccess;  // work on any stream may still use the arrays
   for (auto& kv : t->ws) {
-    (void)dev_free(kv.second.buf, true);
+    (void)dev_free(kv.second.buf, idle);
     if (kv.second.last_use) (void)hipEventDestroy(kv.second.last_use);
   }
-  (void)dev_free(t->d_inner, true);
-  (void)dev_free(t->d_prefix, true);
-  (void)dev_free(t->d_leaves, true);
-  (void)dev_free(t->pend_k, true);
-  (void)dev_free(t->pend_v, true);
-  (void)dev_free(t->upd_buf, true);
+  (void)dev_free(t->d_inner, idle);
+  (void)dev_free(t->d_prefix, idle);
+  (void)dev_free(t->d_leaves, idle);
+  (void)dev_free(t->pend_k, idle);
+  (void)dev_free(t->pend_v, idle);
+  (void)dev_free(t->upd_buf, idle);
   if (t->upd_host) (void)hipHostFree(t->upd_host);
   if (t->pin_stage) (void)hipHostFree(t->pin_stage);
   if (t->stage_ev) (void)hipEventDestroy(t->stage_ev);
-  (void)dev_free(t->sb_leaves, true);
-  (void)dev_free(t->sb_inner, true);
-  (void)dev_free(t->sb_prefix, true);
-  (void)dev_free(t->rl_buf, true);
-  (void)dev_free(t->bl_child, true);
+  (void)dev_free(t->sb_leaves, idle);
+  (void)dev_free(t->sb_inner, idle);
+  (void)dev_free(t->sb_prefix, idle);
+  (void)dev_free(t->rl_buf, idle);
+  (void)dev_free(t->bl_child, idle);
   for (int k = 0; k < 2; ++k) {
     if (t->hs_stage[k]) (void)hipHostFree(t->hs_stage[k]);
     if (t->hs_ev[k]) (void)hipEventDestroy(t->hs_ev[k]);
@@ -470,7 +470,10 @@ void free_tree(hm_tree* t) {
   }
   if (t->publish_ev) (void)hipEventDestroy(t->publish_ev);
   if (t->na_ev) (void)hipEventDestroy(t->na_ev);
-  if (t->own) stream_give(t->own, t->device);
+  if (own_idle)
+    stream_give(t->own, t->device);
+  else if (t->own)
+    (void)hipStreamDestroy(t->own);
   delete t;
 }
 
@@ -575,8 +578,7 @@ int hm_tree_build(const uint64_t* keys, const uint64_t* vals, uint64_t n, const 
   const bool fits = t->leaf_cap * sizeof(Leaf) >= 2 * nb;  // (a tree of one or two leaves may be smaller)
   char* scratch = nullptr;
   auto cleanup = [&]() {
-    (void)hipStreamSynchronize(s);
-    (void)dev_free(scratch, true);
+    (void)dev_free(scratch, hipStreamSynchronize(s) == hipSuccess);
   };
 #define BUILD_TRY(expr)            \
   do {                             \
@@ -1736,8 +1738,7 @@ int hm_psa_sort(const uint64_t* keys, uint64_t n, int begin_bit, int end_bit, ui
     hipStream_t s = nullptr;
     ~Scratch() {
       if (p) {
-        (void)hipStreamSynchronize(s);
-        (void)dev_free(p, true);
+        (void)dev_free(p, hipStreamSynchronize(s) == hipSuccess);
       }
     }
   } scratch;

@@ -3,12 +3,14 @@
 // A build allocates its scratch and the tree's arrays, a destroyed tree gives them back.  The driver unmaps
 // freed memory and clears it before it is used again: building 4 million keys, searching them and closing
 // the tree took 3 to 10 ms, of which the kernels were 0.7 (the higher figure when the freed memory is still
-// being cleared); with blocks and streams kept 0.66 ms.  Blocks are kept instead, at most kPoolKeep bytes per device and none above kPoolBlock,
-// and handed out again to requests of at least half their size.  They go back to the driver when an
-// allocation fails and at hm_device_synchronize.
+// being cleared); with blocks and streams kept 0.66 ms.  Blocks are kept instead, at most kPoolKeep bytes per
+// device and none above kPoolBlock, and handed out again to requests of at least half their size.  They go back
+// to the driver when an allocation here finds no memory and at hm_device_synchronize.
 //
-// A block is given to the pool only when no work that may use it is in flight: dev_free waits for the
-// device, as hipFree does; callers that have waited themselves say so.
+// A block is given to the pool only when no work that may use it is in flight (dev_free's `idle`, after a wait
+// that succeeded); others go to hipFree, which waits itself.  The wait for the whole device is hipFree's own:
+// hipDeviceSynchronize fails while any stream of the process captures, another thread's too, and ends that
+// capture.  The allocation and its hipFree take 1.3 us on an idle device.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -77,12 +79,12 @@ hipError_t dev_malloc_bytes(void** out, size_t bytes) {
     }
   }
   e = hipMalloc(out, bytes);
-  if (e != hipSuccess) {  // give back what is kept and try once more
+  if (e == hipErrorOutOfMemory) {  // give back what is kept and try once more
     (void)hipGetLastError();
     dev_pool_trim();
     e = hipMalloc(out, bytes);
-    if (e != hipSuccess) return e;
   }
+  if (e != hipSuccess) return e;
   if (bytes <= kPoolBlock) {
     try {
       std::lock_guard<std::mutex> g(p.mu);
@@ -106,15 +108,7 @@ hipError_t dev_free(void* ptr, bool idle) {
     }
   }
   int dev = -1;
-  if (!b.bytes || hipGetDevice(&dev) != hipSuccess || dev != b.device) return hipFree(ptr);
-  if (!idle) {
-    hipError_t e = hipDeviceSynchronize();
-    if (e != hipSuccess) {
-      (void)hipFree(ptr);
-      return e;
-    }
-  }
-  hipError_t e = hipSuccess;
+  if (!idle || !b.bytes || hipGetDevice(&dev) != hipSuccess || dev != b.device) return hipFree(ptr);
   while (true) {  // the oldest blocks make room
     void* oldest = nullptr;
     {
@@ -136,13 +130,16 @@ hipError_t dev_free(void* ptr, bool idle) {
       oldest = p.idle[first].p;
       p.idle.erase(p.idle.begin() + (long)first);
     }
-    const hipError_t x = hipFree(oldest);
-    if (x != hipSuccess) e = x;
+    (void)hipFree(oldest);
   }
-  if (ptr) {
-    const hipError_t x = hipFree(ptr);
-    if (x != hipSuccess) e = x;
-  }
+  return ptr ? hipFree(ptr) : hipSuccess;
+}
+
+hipError_t dev_wait() {
+  void* p = nullptr;
+  hipError_t e = hipMalloc(&p, 256);
+  if (e == hipSuccess) e = hipFree(p);
+  if (e != hipSuccess) (void)hipGetLastError();  // the caller does without the pool
   return e;
 }
 

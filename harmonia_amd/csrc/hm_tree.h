@@ -29,13 +29,15 @@ int host_alloc_mapped(void** p, size_t bytes);
   } while (0)
 
 // Device memory of trees and builds (hm_pool.cpp): freed blocks are kept, bounded, for later requests.
-// dev_free waits for the device unless `idle` says that nothing in flight can use the block.
+// dev_free is hipFree, which waits for the device, unless `idle` says that nothing in flight can use the block.
 hipError_t dev_malloc_bytes(void** out, size_t bytes);
 template <typename T>
 hipError_t dev_malloc(T** out, size_t bytes) {
   return dev_malloc_bytes(reinterpret_cast<void**>(out), bytes);
 }
 hipError_t dev_free(void* p, bool idle = false);
+// Waits for everything on the current device; captures in progress elsewhere stay intact.
+hipError_t dev_wait();
 void dev_pool_trim();  // gives every kept block of the current device back to the driver
 // A non-blocking stream of the current device; a stream given back is idle.
 hipError_t stream_take(hipStream_t* s);
