@@ -287,9 +287,10 @@ int enqueue_pipeline(const TreeView& tv, const SearchLaunch& sl, int psa_bits, i
   const int top = out_mode == HM_OUT_PSA_ORDER ? 64 : std::max(std::min((int)tv.psa_top, 64), psa_bits);
   if (out_mode == HM_OUT_UNPERMUTE && partitions(sl, psa_bits)) {
     const int bits = partition_bits(n);
+    const int ptop = std::max(top, bits);  // keys below 2^10 and few psa_bits: the digit reaches above them
     const Clash clash{(uint32_t*)b.ft, (uint8_t*)b.vt};
-    HM_TRY(partition_keys(dq, n, top, b.k0, b.replay, clash, s, dn));
-    HM_TRY(launch_search_chunks(tv, b.k0, b.rv, b.rf, n, top, bits, kMissMark, clash, s, dn));
+    HM_TRY(partition_keys(dq, n, ptop, b.k0, b.replay, clash, s, dn));
+    HM_TRY(launch_search_chunks(tv, b.k0, b.rv, b.rf, n, ptop, bits, kMissMark, clash, s, dn));
     HM_TRY(unpartition_results(b.rv, b.rf, n, b.replay, clash, dvals, dfound, s, dn));
     return HM_OK;
   }
