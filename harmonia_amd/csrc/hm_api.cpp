@@ -218,6 +218,8 @@ int resolve_search(const hm_tree* t, uint64_t n, const hm_search_opts* o, Search
   if (sk > HM_SORTED_WINDOW) return set_err(HM_EINVAL, "sorted_kernel %u not in 0..2", sk);
   // leaf window: only when asked for (measured slower than one descent per query on the 2^26-key tree)
   sl->window = psa && mode != HM_OUT_SCATTER && sk == HM_SORTED_WINDOW;
+  sl->named = sk == HM_SORTED_QUERY || (o && (o->group_size || o->queries_per_group || o->blocks_per_cu ||
+                                              o->lds_levels >= 0));
   sl->window_blocks_per_cu = (o && o->blocks_per_cu && sk == HM_SORTED_WINDOW) ? (int)o->blocks_per_cu : 2;
   *psa_bits = psa ? bits : 0;
   *out_mode = psa ? mode : 0;
@@ -256,12 +258,12 @@ PipeBufs carve_pipe(char*& cur, size_t n, int psa_bits, int out_mode) {
 }
 
 // Searches that return results in input order split the batch once and order it further inside each
-// block.  The rule: the launch shape is the default one, which that kernel replaces (other shapes are asked
-// for by name or by the tuner), and two sort passes would be made, whose records' memory then holds the
-// partition's.  Over 2^18..2^26 keys, fanouts 32..128, 2^20..2^24 queries in every order it takes 0.45 to
+// block.  The rule: the launch shape is the default one, which that kernel replaces, and the caller has not
+// named it (a call that names a shape or one descent per query gets the kernel that it means), and two sort
+// passes would be made, whose records' memory then holds the partition's.  Over 2^18..2^26 keys, fanouts 32..128, 2^20..2^24 queries in every order it takes 0.45 to
 // 0.92 of the time of the two passes and search_span_kernel, and nowhere more.
 static bool partitions(const SearchLaunch& sl, int psa_bits) {
-  return sl.group == 2 && sl.queries_per_group == 4 && !sl.window && psa_bits > 8 && psa_bits <= 16;
+  return sl.group == 2 && sl.queries_per_group == 4 && !sl.window && !sl.named && psa_bits > 8 && psa_bits <= 16;
 }
 
 // PSA-order results need both passes, and the same kernel may search what they sorted: if the window orders

@@ -189,6 +189,7 @@ struct SearchLaunch {
   int queries_per_group = 2;  // independent descents interleaved per group
   bool sorted = false;        // queries are PSA-sorted: waves share node reads (group 1, or group 2 x 4)
   bool window = false;        // with sorted, OUT_DIRECT: the leaf-window kernel (dense batches)
+  bool named = false;         // the caller named the shape, or one descent per query: no other kernel's place
   int window_blocks_per_cu = 2;
   // unsorted OUT_DIRECT searches with 1..8 lanes per query: read the queries from these segments
   // (blocks take whole segments) instead of the packed array

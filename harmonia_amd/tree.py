@@ -144,9 +144,10 @@ class BPlusTree:
                      out_pos=None, sorted_kernel=0):
         """Batched search; returns (values, found) in input order (or PSA order with out_pos).
 
-        output_mode: 0 tree default, 1 input order via the replayed sort passes, 2 input order via direct
-        scatter, 3 (or sorted_output=True) PSA order with the permutation in out_pos.
-        sorted_kernel (PSA batches): 0 automatic, 1 one descent per query, 2 leaf window."""
+        output_mode: 0 tree default, 1 input order via the replayed sort or partition, 2 input order via
+        direct scatter, 3 (or sorted_output=True) PSA order with the permutation in out_pos.
+        sorted_kernel (PSA batches): 0 automatic, 1 one descent per query, 2 leaf window; naming group_size,
+        lds_levels, blocks_per_cu or queries_per_group means 1."""
         if sorted_output:
             output_mode = _lib.HM_OUT_PSA_ORDER
         q = _u64(q)

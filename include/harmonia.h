@@ -73,19 +73,23 @@ typedef struct hm_stats {
                             * place (a leaf overflowed, the node had room) */
   uint64_t key_min;        /* smallest stored key (HM_KEY_MAX for an empty tree) */
   uint64_t key_max;        /* largest stored key (0 for an empty tree) */
-  uint32_t psa_window_top; /* input-order PSA searches sort by bits [top - psa_bits, top): one past the
-                            * highest bit in which key_min and key_max differ (64 for fewer than two
-                            * keys); PSA-order results (HM_OUT_PSA_ORDER) always use [64 - psa_bits, 64) */
+  uint32_t psa_window_top; /* input-order PSA searches order by bits below top: one past the highest bit
+                            * in which key_min and key_max differ (64 for fewer than two keys).  Sort
+                            * passes take [top - psa_bits, top); the tree's choice for 9 to 16 bits
+                            * (HM_SORTED_AUTO) splits the batch by 8 to 11 of them and orders each part
+                            * on the chip.  PSA-order results (HM_OUT_PSA_ORDER) always use
+                            * [64 - psa_bits, 64) */
   uint32_t reserved;
 } hm_stats;
 
 /* hm_search_opts.output_mode (with PSA on; without PSA results are always in input order) */
 #define HM_OUT_DEFAULT 0 /* the tree's choice */
-#define HM_OUT_UNPERMUTE 1 /* input order: the sort passes replayed backwards over the results (coalesced) */
+#define HM_OUT_UNPERMUTE 1 /* input order: the sort or partition replayed backwards over the results (coalesced) */
 #define HM_OUT_SCATTER 2 /* input order: each result written straight to its position */
 #define HM_OUT_PSA_ORDER 3 /* PSA order plus out_pos, as the reference returns them (H/regular_bpt/prefix-sort.cu:296-297) */
 
-/* Per-call overrides for batched search (used by the autotuner); 0 / -1 = tree default. */
+/* Per-call overrides for batched search; 0 / -1 = tree default.  A call that names any of group_size,
+ * lds_levels, blocks_per_cu and queries_per_group runs the kernel they shape: one descent per query. */
 typedef struct hm_search_opts {
   uint32_t group_size;     /* lanes per query: 1, 2, 4, 8, 16, 32, 64 (at most the fanout) */
   int32_t lds_levels;      /* -1 = default */
@@ -99,7 +103,8 @@ typedef struct hm_search_opts {
 } hm_search_opts;
 
 /* hm_search_opts.sorted_kernel */
-#define HM_SORTED_AUTO 0    /* the tree's choice (one descent per query) */
+#define HM_SORTED_AUTO 0    /* the tree's choice: blocks that each order and search a part of the batch, or
+                             * one descent per query */
 #define HM_SORTED_QUERY 1   /* one descent per query (each wave shares its upper-level node reads and
                              * loads the run of last-level nodes its queries reach) */
 #define HM_SORTED_WINDOW 2  /* leaf window: each wave streams the leaves its chunk of sorted queries
