@@ -262,7 +262,7 @@ PipeBufs carve_pipe(char*& cur, size_t n, int psa_bits, int out_mode) {
 // named it (a call that names a shape or one descent per query gets the kernel that it means), and two sort
 // passes would be made, whose records' memory then holds the partition's.  Over 2^18..2^26 keys, fanouts 32..128, 2^20..2^24 queries in every order it takes 0.45 to
 // 0.92 of the time of the two passes and search_span_kernel, and nowhere more.
-static bool partitions(const SearchLaunch& sl, int psa_bits) {
+bool partitions(const SearchLaunch& sl, int psa_bits) {
   return sl.group == 2 && sl.queries_per_group == 4 && !sl.window && !sl.named && psa_bits > 8 && psa_bits <= 16;
 }
 

@@ -50,6 +50,10 @@ struct SearchCfg {
   int blocks_per_cu;
   int output_mode;
 };
+// PSA-ordered batches: neighbours share nodes.  10 blocks per CU = two full rounds of the five
+// blocks of this shape that fit on a CU (96 VGPRs): a partial last round of the persistent grid
+// (8 per CU: 5 + 3) measured 3% slower.
+constexpr SearchCfg kPsaCfg{2, 4, 10, HM_OUT_UNPERMUTE};
 
 struct Workspace {
   void* buf = nullptr;
@@ -75,10 +79,7 @@ struct hm_tree {
   uint64_t layout_version = 0;  // bumped whenever a device array of the layout is reallocated
   bool tuned = false;  // the tuner has set cfg_direct and cfg_psa
   hm::SearchCfg cfg_direct{4, 4, 4, HM_OUT_UNPERMUTE};  // unsorted batches: memory-transaction bound
-  // PSA-ordered batches: neighbours share nodes.  10 blocks per CU = two full rounds of the five
-  // blocks of this shape that fit on a CU (96 VGPRs): a partial last round of the persistent grid
-  // (8 per CU: 5 + 3) measured 3% slower.
-  hm::SearchCfg cfg_psa{2, 4, 10, HM_OUT_UNPERMUTE};
+  hm::SearchCfg cfg_psa = hm::kPsaCfg;
   std::mutex mu;
   std::unordered_map<hipStream_t, hm::Workspace> ws;
   hipStream_t own = nullptr;
@@ -213,6 +214,9 @@ struct PipeBufs {
   uint8_t *rf, *ft;   // PSA-order found flags and their ping-pong buffer
 };
 size_t pipe_bytes(size_t n, int psa_bits, int out_mode);
+// Whether an input-order search of this shape partitions its batch (its kernel has no width and no blocks per
+// CU of its own).
+bool partitions(const SearchLaunch& sl, int psa_bits);
 PipeBufs carve_pipe(char*& cur, size_t n, int psa_bits, int out_mode);
 // Enqueue sort -> search -> un-sort on s.  n sizes every launch; dn (device) may hold a smaller
 // actual count, so the same enqueue can be captured once into a graph and replayed.  The PSA-order

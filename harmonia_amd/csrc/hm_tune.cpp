@@ -134,6 +134,9 @@ int tune_tree(hm_tree* t, const uint64_t* sample, uint64_t n, uint32_t flags, hm
             sl.group = g;
             sl.queries_per_group = q;
             sl.blocks_per_cu = bpc;
+            // one pipeline whatever its bits and blocks per CU: timed once, kept with the defaults for both
+            if (mode == HM_OUT_UNPERMUTE && partitions(sl, bits) && (bits != 16 || bpc != kPsaCfg.blocks_per_cu))
+              continue;
             float ms = 0;
             if ((rc = time_pipeline(t, sl, bits, mode, b, n, s, reps, &ms))) return rc;
             ++trials;
