@@ -116,7 +116,7 @@ void free_batcher(hm_batcher* b) {
     b->g_direct[k].reset();
   }
   for (void* p : {(void*)b->d_q, (void*)b->d_vals, (void*)b->d_found, (void*)b->d_n, b->scratch})
-    if (p) (void)hipFree(p);
+    (void)dev_free(p);
   for (void* p : {(void*)b->h_stage, (void*)b->h_items[0], (void*)b->h_items[1], (void*)b->h_hdr, (void*)b->h_gran[0],
                   (void*)b->h_gran[1]})
     if (p) (void)hipHostFree(p);
@@ -199,9 +199,9 @@ int hm_batcher_create(hm_tree* t, uint64_t capacity, const hm_search_opts* opts,
   if (t->p.mem_budget && t->device_bytes() + need + capacity * 17 > t->p.mem_budget)
     return fail(set_err(HM_EBUDGET, "batcher of %llu queries exceeds the device-memory budget",
                         (unsigned long long)capacity));
-  if (hipMalloc(&b->d_q, capacity * 8) != hipSuccess || hipMalloc(&b->d_vals, capacity * 8) != hipSuccess ||
-      hipMalloc(&b->d_found, capacity) != hipSuccess || hipMalloc(&b->d_n, 256) != hipSuccess ||
-      hipMalloc(&b->scratch, need) != hipSuccess)
+  if (dev_malloc(&b->d_q, capacity * 8) != hipSuccess || dev_malloc(&b->d_vals, capacity * 8) != hipSuccess ||
+      dev_malloc(&b->d_found, capacity) != hipSuccess || dev_malloc(&b->d_n, 256) != hipSuccess ||
+      dev_malloc(&b->scratch, need) != hipSuccess)
     return fail(set_err(HM_ENOMEM, "batcher allocation failed"));
   if (int rc = host_alloc_mapped((void**)&b->h_hdr, 2 * sizeof(GatherHdr))) return fail(rc);
   for (int k = 0; k < 2; ++k)

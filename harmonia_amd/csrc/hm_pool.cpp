@@ -84,7 +84,10 @@ hipError_t dev_malloc_bytes(void** out, size_t bytes) {
     dev_pool_trim();
     e = hipMalloc(out, bytes);
   }
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // reported here, not by the next launch
+    return e;
+  }
   if (bytes <= kPoolBlock) {
     try {
       std::lock_guard<std::mutex> g(p.mu);

@@ -81,13 +81,13 @@ struct Buf {
       const int rc = host_alloc_mapped(&p, want);
       if (rc) return rc;
     } else {
-      HM_TRY(hipMalloc(&p, want));
+      HM_TRY(dev_malloc(&p, want));
     }
     bytes = want;
     return HM_OK;
   }
   void release() {
-    if (p) (void)(pinned ? hipHostFree(p) : hipFree(p));
+    if (p) (void)(pinned ? hipHostFree(p) : dev_free(p));
     p = nullptr;
     bytes = 0;
   }

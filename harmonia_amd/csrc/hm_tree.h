@@ -28,7 +28,7 @@ int host_alloc_mapped(void** p, size_t bytes);
     }                                                                                                      \
   } while (0)
 
-// Device memory of trees and builds (hm_pool.cpp): freed blocks are kept, bounded, for later requests.
+// All device memory of the library (hm_pool.cpp): blocks of closed trees are kept, bounded, for later requests.
 // dev_free is hipFree, which waits for the device, unless `idle` says that nothing in flight can use the block.
 hipError_t dev_malloc_bytes(void** out, size_t bytes);
 template <typename T>
