@@ -604,7 +604,7 @@ int hm_tree_build(const uint64_t* keys, const uint64_t* vals, uint64_t n, const 
       unsorted ? std::max(align256(radix_tmp_bytes(n)), bbits ? align256(partition_pairs_bytes(n)) : 0) : 0;
   const size_t need =
       256 + (hk ? nb : 0) + (hv ? nb : 0) + (unsorted ? 2 * nb + (fits ? 0 : 2 * nb) + tmp_bytes : 0);
-  BUILD_TRY(dev_malloc(&scratch, need));
+  BUILD_TRY(dev_scratch(&scratch, need));
   BUILD_TRY(dev_malloc(&t->d_leaves, t->leaf_cap * sizeof(Leaf)));
   Levels lv;
   if ((rc = prepare_inner(t, &lv, s))) {
@@ -1746,7 +1746,7 @@ int hm_psa_sort(const uint64_t* keys, uint64_t n, int begin_bit, int end_bit, ui
     }
   } scratch;
   scratch.s = s;
-  HM_TRY(dev_malloc(&scratch.p, 3 * kq + 2 * kp + align256(radix_tmp_bytes(n))));
+  HM_TRY(dev_scratch(&scratch.p, 3 * kq + 2 * kp + align256(radix_tmp_bytes(n))));
   char* cur = scratch.p;
   const uint64_t* dk = keys;
   if (!is_device_ptr(keys)) {

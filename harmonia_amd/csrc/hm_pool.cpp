@@ -4,8 +4,10 @@
 // freed memory and clears it before it is used again: building 4 million keys, searching them and closing
 // the tree took 3 to 10 ms, of which the kernels were 0.7 (the higher figure when the freed memory is still
 // being cleared); with blocks and streams kept 0.66 ms.  Blocks are kept instead, at most kPoolKeep bytes per
-// device and none above kPoolBlock, and handed out again to requests of at least half their size.  They go back
-// to the driver when an allocation here finds no memory and at hm_device_synchronize.
+// device and none above kPoolBlock, and handed out again: to requests of exactly their size, since what a tree
+// holds is counted against its budget by the bytes it asked for, or for a call's own scratch to requests of at
+// least half their size.  They go back to the driver when an allocation here finds no memory and at
+// hm_device_synchronize.
 //
 // A block is given to the pool only when no work that may use it is in flight (dev_free's `idle`, after a wait
 // that succeeded); others go to hipFree, which waits itself.  The wait for the whole device is hipFree's own:
@@ -53,7 +55,7 @@ Pool& pool() {
 
 }  // namespace
 
-hipError_t dev_malloc_bytes(void** out, size_t bytes) {
+hipError_t dev_malloc_bytes(void** out, size_t bytes, bool scratch) {
   *out = nullptr;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -64,7 +66,7 @@ hipError_t dev_malloc_bytes(void** out, size_t bytes) {
     size_t best = p.idle.size();
     for (size_t i = 0; i < p.idle.size(); ++i) {
       const auto& f = p.idle[i];
-      if (f.device == dev && f.bytes >= bytes && f.bytes / 2 <= bytes &&
+      if (f.device == dev && (scratch ? f.bytes >= bytes && f.bytes / 2 <= bytes : f.bytes == bytes) &&
           (best == p.idle.size() || f.bytes < p.idle[best].bytes))
         best = i;
     }

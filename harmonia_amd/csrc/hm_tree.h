@@ -30,10 +30,16 @@ int host_alloc_mapped(void** p, size_t bytes);
 
 // All device memory of the library (hm_pool.cpp): blocks of closed trees are kept, bounded, for later requests.
 // dev_free is hipFree, which waits for the device, unless `idle` says that nothing in flight can use the block.
-hipError_t dev_malloc_bytes(void** out, size_t bytes);
+// dev_malloc gives a block of the requested size; dev_scratch, for memory that the same call frees, up to twice
+// that.
+hipError_t dev_malloc_bytes(void** out, size_t bytes, bool scratch);
 template <typename T>
 hipError_t dev_malloc(T** out, size_t bytes) {
-  return dev_malloc_bytes(reinterpret_cast<void**>(out), bytes);
+  return dev_malloc_bytes(reinterpret_cast<void**>(out), bytes, false);
+}
+template <typename T>
+hipError_t dev_scratch(T** out, size_t bytes) {
+  return dev_malloc_bytes(reinterpret_cast<void**>(out), bytes, true);
 }
 hipError_t dev_free(void* p, bool idle = false);
 // Waits for everything on the current device; captures in progress elsewhere stay intact.

@@ -68,10 +68,10 @@ struct Best {
 int tune_tree(hm_tree* t, const uint64_t* sample, uint64_t n, uint32_t flags, hm_tune_result* res) {
   hipStream_t s = t->own;
   Bufs b;
-  HM_TRY(dev_malloc(&b.q, n * 8));
-  HM_TRY(dev_malloc(&b.vals, n * 8));
-  HM_TRY(dev_malloc(&b.found, n));
-  HM_TRY(dev_malloc(&b.scratch, pipe_bytes(n, 32, HM_OUT_UNPERMUTE)));
+  HM_TRY(dev_scratch(&b.q, n * 8));
+  HM_TRY(dev_scratch(&b.vals, n * 8));
+  HM_TRY(dev_scratch(&b.found, n));
+  HM_TRY(dev_scratch(&b.scratch, pipe_bytes(n, 32, HM_OUT_UNPERMUTE)));
   HM_TRY(hipMemcpyAsync(b.q, sample, n * 8, is_device_ptr(sample) ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
                         s));
   const int reps = (flags & HM_TUNE_QUICK) ? 2 : 4;
