@@ -306,6 +306,12 @@ def read_ranges_text(path):
     return a[:n.value], b[:n.value]
 
 
+def device_synchronize():
+    """Wait for the current GPU and give back to the driver the device memory that closed trees left for reuse
+    (at most 512 MiB)."""
+    check(_lib.load().hm_device_synchronize())
+
+
 def psa_sort(keys, begin_bit=48, end_bit=64, stream=None):
     """Stable radix sort of (key, position) over key bits [begin_bit, end_bit) on the GPU."""
     lib = _lib.load()
