@@ -983,8 +983,10 @@ static int range_common(hm_tree* t, const uint64_t* start, const uint64_t* hi, c
     dl = b;
   }
   uint64_t* doff = nullptr;
-  // lengths in mapped host memory are read once, by the scan kernel, not by every range
-  const bool scan = out_offsets && !mapped && n <= kRangeScanMax;
+  // The one-launch form has every wave add up the lengths before its range: not for lengths in mapped host
+  // memory (the scan kernel reads them once), nor where the counts, written meanwhile, take the lengths' place.
+  const bool counts_apart = !dl || out_counts + n <= dl || dl + n <= out_counts;
+  const bool scan = out_offsets && !mapped && n <= kRangeScanMax && counts_apart;
   if (out_offsets) doff = ho ? (uint64_t*)take(k8p) : out_offsets;
   if (out_offsets && !scan) {
     void* scan_tmp = take(align256(scan_tmp_bytes(n + 1)));
