@@ -768,12 +768,12 @@ int search_host_stream_body(hm_tree* t, const uint64_t* q, uint64_t n, uint64_t*
   Workspace* w[2] = {nullptr, nullptr};
   for (int k = 0; k < 2; ++k)
     if ((rc = ensure_ws(t, t->hs[k], 2 * kq + kf + pipe_bytes(C, bits, mode), &w[k]))) return rc;
-  // after the caller's earlier work on s and the latest publish
-  Workspace* ws_s = nullptr;
-  if ((rc = ensure_ws(t, s, 0, &ws_s))) return rc;
-  HM_TRY(hipEventRecord(ws_s->last_use, s));
+  // After the caller's earlier work on s and the latest publish.  That work may have written the queries to
+  // pinned memory, which the DMA engine reads: an event with the system-scope fence (every earlier chunk that
+  // hs_ev stood for has been waited for).
+  HM_TRY(hipEventRecord(t->hs_ev[0], s));
   for (int k = 0; k < 2; ++k) {
-    HM_TRY(hipStreamWaitEvent(t->hs[k], ws_s->last_use, 0));
+    HM_TRY(hipStreamWaitEvent(t->hs[k], t->hs_ev[0], 0));
     if (t->publish_valid) HM_TRY(hipStreamWaitEvent(t->hs[k], t->publish_ev, 0));
   }
   const TreeView tv = t->view();
