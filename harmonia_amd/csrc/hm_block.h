@@ -5,6 +5,13 @@
 
 namespace hm {
 
+// Blocks are dispatched round-robin over the 8 XCDs: block b's share of m pieces of work if each XCD is to take a
+// contiguous eighth of them (m or more: none).  m is the work there is, not the grid, which may be sized for more.
+__device__ __forceinline__ uint32_t xcd_share(uint32_t b, uint32_t m) {
+  const uint32_t per = (m + 7) >> 3;
+  return (b >> 3) < per ? (b & 7u) * per + (b >> 3) : m;
+}
+
 // Make this wave's LDS writes visible to its own later LDS reads (and keep the compiler from moving
 // LDS accesses across): the LDS executes one wave's operations in order, so no block barrier is
 // needed for a wave-private buffer.

@@ -32,22 +32,22 @@ constexpr int kDPer = kDigits / kThreads;  // digits per thread
 static_assert(kDPer == 4, "a thread's digits are one 16-byte load");
 static_assert(kTile <= 65536, "staging indices are 16-bit");
 
-// As the radix sort: XCD x takes the tiles [x grid / 8, (x + 1) grid / 8), so partial cache lines at the
-// ends of neighbouring tiles' runs meet in one L2.
-__device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t grid) { return (b & 7u) * (grid >> 3) + (b >> 3); }
+// As the radix sort: XCD x takes a contiguous eighth of the tiles, so partial cache lines at the ends of
+// neighbouring tiles' runs meet in one L2.
+__device__ __forceinline__ uint32_t tiles_of(size_t n) { return (uint32_t)((n + kTile - 1) / kTile); }
 unsigned grid_for(size_t nb) { return (unsigned)((nb + 7) / 8 * 8); }
 
 // counts[tile][digit], one block per tile.  VEC: keys 16-byte aligned.
 template <bool VEC>
 __global__ __launch_bounds__(kThreads) void part_hist_kernel(const uint64_t* __restrict__ keys, size_t n, int shift,
-                                                             uint32_t nd, uint32_t* __restrict__ counts, uint32_t nb,
+                                                             uint32_t nd, uint32_t* __restrict__ counts,
                                                              uint32_t* __restrict__ clash,
                                                              const uint32_t* __restrict__ dn) {
   __shared__ uint32_t h[kDigits];
-  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
-  if (tile >= nb) return;  // block-uniform
+  if (dn) n = *dn;
+  const uint32_t tile = xcd_share(blockIdx.x, tiles_of(n));
+  if (tile >= tiles_of(n)) return;  // block-uniform
   if (clash && tile == 0 && threadIdx.x == 0) *clash = 0;
-  if (dn) n = *dn;         // tiles past n count nothing
   const uint32_t mask = nd - 1;
   for (uint32_t d = threadIdx.x; d < nd; d += kThreads) h[d] = 0;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -70,7 +70,7 @@ __global__ __launch_bounds__(kThreads) void part_hist_kernel(const uint64_t* __r
       }
     }
   } else {
-    const size_t last = n ? n - 1 : 0;
+    const size_t last = n - 1;
     uint64_t kk[kItems];
 #pragma unroll
     for (int r = 0; r < kItems; ++r) {
@@ -86,20 +86,22 @@ __global__ __launch_bounds__(kThreads) void part_hist_kernel(const uint64_t* __r
   for (uint32_t d = threadIdx.x; d < nd; d += kThreads) counts[(size_t)tile * nd + d] = h[d];
 }
 
-// Per digit: exclusive scan of its counts along the tiles, in place; the digit's total to row nb.  A block
-// takes 16 digits (64-byte pieces of the rows), 64 segments of tiles side by side.
+// Per digit: exclusive scan of its counts along the tiles (of the *dn keys there are, if dn), in place; the
+// digit's total to row nb.  A block takes 16 digits (64-byte pieces of the rows), 64 segments of tiles side by side.
 constexpr int kScanThreads = 1024;
 constexpr int kScanDigits = 16;
 constexpr int kScanSegs = kScanThreads / kScanDigits;
 constexpr int kScanBatch = 8;
 __global__ __launch_bounds__(kScanThreads) void part_scan_kernel(uint32_t* __restrict__ counts, uint32_t nd,
                                                                  uint32_t nb, uint32_t limit,
-                                                                 uint32_t* __restrict__ flags, uint32_t flag) {
+                                                                 uint32_t* __restrict__ flags, uint32_t flag,
+                                                                 const uint32_t* __restrict__ dn) {
   __shared__ uint32_t sums[kScanSegs][kScanDigits];
+  const uint32_t live = dn ? tiles_of(*dn) : nb;
   const uint32_t j = threadIdx.x % kScanDigits, seg = threadIdx.x / kScanDigits;
   uint32_t* col = counts + blockIdx.x * kScanDigits + j;
-  const uint32_t per = (nb + kScanSegs - 1) / kScanSegs;
-  const uint32_t t0 = seg * per < nb ? seg * per : nb, t1 = t0 + per < nb ? t0 + per : nb;
+  const uint32_t per = (live + kScanSegs - 1) / kScanSegs;
+  const uint32_t t0 = seg * per < live ? seg * per : live, t1 = t0 + per < live ? t0 + per : live;
   uint32_t s = 0;
   for (uint32_t t = t0; t < t1; t += kScanBatch) {
     uint32_t v[kScanBatch];
@@ -160,9 +162,9 @@ __global__ __launch_bounds__(kThreads) void part_scatter_kernel(const uint64_t* 
   __shared__ uint64_t skeys[kTile];
   __shared__ __align__(16) uint32_t dig[kDigits];  // counts, then tile offsets, then output minus tile offsets
   __shared__ uint32_t scan_sh[kThreads / 64 + 1];
-  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
   if (dn) n = *dn;
-  if (tile >= nb || (size_t)tile * kTile >= n) return;  // block-uniform
+  const uint32_t tile = xcd_share(blockIdx.x, tiles_of(n));
+  if (tile >= tiles_of(n)) return;  // block-uniform
   const uint32_t mask = nd - 1, d0 = threadIdx.x * kDPer;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const size_t tile0 = (size_t)tile * kTile, base = tile0 + (size_t)w * 64 * kItems;
@@ -239,9 +241,9 @@ __global__ __launch_bounds__(kThreads) void part_unscatter_kernel(const uint64_t
   static_assert(sizeof(adj) >= kTile, "the found flags fit");
   uint8_t* sf = reinterpret_cast<uint8_t*>(adj);
   uint16_t* dg = reinterpret_cast<uint16_t*>(sv);
-  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
   if (dn) n = *dn;
-  if (tile >= nb || (size_t)tile * kTile >= n) return;  // block-uniform
+  const uint32_t live = tiles_of(n), tile = xcd_share(blockIdx.x, live);
+  if (tile >= live) return;  // block-uniform
   const bool flags = *clash.any != 0;  // uniform
   const uint32_t d0 = threadIdx.x * kDPer;
   const size_t tile0 = (size_t)tile * kTile;
@@ -249,7 +251,7 @@ __global__ __launch_bounds__(kThreads) void part_unscatter_kernel(const uint64_t
   uint32_t g[kDPer], nx[kDPer], tot[kDPer], c[kDPer];
   load_digits(offsets + (size_t)nb * nd, d0, nd, tot);
   load_digits(offsets + (size_t)tile * nd, d0, nd, g);
-  load_digits(offsets + (size_t)(tile + 1) * nd, d0, nd, nx);  // row nb: the totals
+  load_digits(offsets + (size_t)(tile + 1 < live ? tile + 1 : nb) * nd, d0, nd, nx);  // row nb: the totals
   uint2 pw[VEC ? kItems / 4 : 1];
   if constexpr (VEC) {
 #pragma unroll
@@ -385,7 +387,7 @@ __global__ __launch_bounds__(kPairThreads) void part_pairs_kernel(const uint64_t
   __shared__ uint64_t skeys[kTile], svals[kTile];
   __shared__ __align__(16) uint32_t dig[kDigits];
   __shared__ uint32_t scan_sh[kPairThreads / 64 + 1];
-  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  const uint32_t tile = xcd_share(blockIdx.x, nb);
   if (tile >= nb || (*flags & skip)) return;  // block-uniform
   const uint32_t mask = nd - 1, d0 = threadIdx.x * kPairDPer;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -462,16 +464,16 @@ hipError_t partition_keys(const uint64_t* q, size_t n, int top, uint64_t* out, v
   {
     ProfScope prof("psa_hist", s);
     if ((reinterpret_cast<uintptr_t>(q) & 15) == 0)
-      hipLaunchKernelGGL(part_hist_kernel<true>, dim3(grid_for(nb)), dim3(kThreads), 0, s, q, n, shift, nd, offsets, nb,
+      hipLaunchKernelGGL(part_hist_kernel<true>, dim3(grid_for(nb)), dim3(kThreads), 0, s, q, n, shift, nd, offsets,
                          clash.any, dn);
     else
       hipLaunchKernelGGL(part_hist_kernel<false>, dim3(grid_for(nb)), dim3(kThreads), 0, s, q, n, shift, nd, offsets,
-                         nb, clash.any, dn);
+                         clash.any, dn);
   }
   {
     ProfScope prof("scan", s);
     hipLaunchKernelGGL(part_scan_kernel, dim3(nd / kScanDigits), dim3(kScanThreads), 0, s, offsets, nd, nb, 0u,
-                       (uint32_t*)nullptr, 0u);
+                       (uint32_t*)nullptr, 0u, dn);
   }
   ProfScope prof("psa_scatter", s);
   hipLaunchKernelGGL(part_scatter_kernel, dim3(grid_for(nb)), dim3(kThreads), 0, s, q, out, place, n, shift, nd,
@@ -497,13 +499,13 @@ hipError_t partition_pairs(const uint64_t* keys, const uint64_t* vals, size_t n,
   uint32_t* offsets = reinterpret_cast<uint32_t*>(tmp);
   ProfScope prof("build", s);
   if ((reinterpret_cast<uintptr_t>(keys) & 15) == 0)
-    hipLaunchKernelGGL(part_hist_kernel<true>, dim3(grid_for(nb)), dim3(kThreads), 0, s, keys, n, shift, nd, offsets, nb,
+    hipLaunchKernelGGL(part_hist_kernel<true>, dim3(grid_for(nb)), dim3(kThreads), 0, s, keys, n, shift, nd, offsets,
                        (uint32_t*)nullptr, (const uint32_t*)nullptr);
   else
     hipLaunchKernelGGL(part_hist_kernel<false>, dim3(grid_for(nb)), dim3(kThreads), 0, s, keys, n, shift, nd, offsets,
-                       nb, (uint32_t*)nullptr, (const uint32_t*)nullptr);
+                       (uint32_t*)nullptr, (const uint32_t*)nullptr);
   hipLaunchKernelGGL(part_scan_kernel, dim3(nd / kScanDigits), dim3(kScanThreads), 0, s, offsets, nd, nb,
-                     kBucketSortMax, flags, flag);
+                     kBucketSortMax, flags, flag, (const uint32_t*)nullptr);
   hipLaunchKernelGGL(part_pairs_kernel, dim3(grid_for(nb)), dim3(kPairThreads), 0, s, keys, vals, kout, vout, n, shift,
                      nd, (const uint32_t*)offsets, nb, (const uint32_t*)flags, flag);
   *totals = offsets + (size_t)nb * nd;

@@ -832,8 +832,9 @@ __global__ __launch_bounds__(kChunkThreads) void search_chunk_kernel(TreeView tv
   uint32_t* cnt = reinterpret_cast<uint32_t*>(nbufs);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if (dn) n = *dn;
-  const uint32_t c0 = xcd_block(blockIdx.x, gridDim.x) * kChunk;
-  if (c0 >= n) return;  // block-uniform
+  const uint32_t chunks = (uint32_t)(((uint64_t)n + kChunk - 1) / kChunk), chunk = xcd_share(blockIdx.x, chunks);
+  if (chunk >= chunks) return;  // block-uniform
+  const uint32_t c0 = chunk * kChunk;
   const uint32_t m = n - c0 < kChunk ? n - c0 : kChunk;
   uint64_t k[I];
 #pragma unroll
