@@ -6,10 +6,11 @@
 // The reference emits at most Range_Size = 8 records per range (H/src/range.cu:32); here a range
 // emits up to its own length, or every key of a closed interval [lo, hi] as
 // find_range(start, end) does (H/regular_bpt/regular_bpt.cpp:320-338).
-// A wave takes R ranges.  Their descents run together (R = 8: one 8-lane group per range; R = 1: the
-// whole wave ranks a node in one step), then all 64 lanes walk the leaves: one 16-byte load per lane brings
-// 8 leaves (1 KiB), lanes 0-3 of a leaf's 8 holding its keys and 4-7 its values, two ballots rank the
-// qualifying keys, and one 16-byte store per lane writes the pairs, keys and values as contiguous runs.
+// A wave takes R ranges (calls in between give 8 lanes to each, group_kernel).  Their descents run together (R = 8:
+// one 8-lane group per range; R = 1: the whole wave ranks a node in one step), then all 64 lanes walk the leaves:
+// one 16-byte load per lane brings 8 leaves (1 KiB), lanes 0-3 of a leaf's 8 holding its keys and 4-7 its values,
+// two ballots rank the qualifying keys, and one 16-byte store per lane writes the pairs, keys and values as
+// contiguous runs.
 //
 // Large calls are bound by memory traffic: 2^20 ranges of 16..256 pairs on 2^26 keys (fanout 128) move
 // 5.4 GB in 0.99-1.09 ms, the rate of a plain copy here (4.8-5.1 TB/s).  Walking each range with a group
@@ -27,17 +28,19 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
-// Up to this many ranges a wave takes one (R = 1, whole-node ranks: four dependent reads per descent
-// instead of eight), above it eight, whose descents share the wave: 2^13 ranges of 16..256 pairs on
-// 2^26 keys 23 against 31 us, 2^14 32.4 against 34.7; 8192 waves are resident, so the gain ends there.
-constexpr uint32_t kOneMax = 16384;
-// Closed intervals may end anywhere before their capacity: a wave that lays eight ranges' leaves end to end
-// reads many for nothing, so above R = 1 they keep a group of 8 lanes each, which stops at the interval's end
-// (2^18 and 2^26 keys: 20000 of up to 256 pairs 24.8 and 28.2 us for 29.5 and 30.2, 200000 of up to 40 37 and 68
-// for 45 and 62, 10^6 of up to 256 1011 and 1297 for 971 and 1356).  R = 1 reaches further for long ones: 30000
-// of up to 256 25 and 39 us for 30 and 40, 60000 45 and 81 to 86 for 49 and 76 to 83; of up to 40 24 and 28 for 17
-// and 24.
-constexpr uint32_t kOneMaxShort = 12288, kOneMaxLong = 49152, kLongInterval = 64;
+// Which kernel takes how many ranges; device times in us of a wave per range (R = 1), 8 lanes each and eight laid
+// end to end (R = 8), trees of 2^20 to 2^25 keys, 1 to 8 keys to a leaf.
+// R = 1 while waves are free: its descents have four dependent reads instead of eight.  4096 ranges of 1..3 pairs
+// 10.5, 10.3, 11.2 (6 in the scan launches), of 16..256 13 to 41, 18 to 73, 22 to 123.  Above, for long ranges (by
+// the capacity for them): 8192 of 16..256 25 to 68, 28 to 83, 34 to 140; 16384 47 to 123, 49 to 123, 51 to 165; of
+// 1..40 38 to 64, 34 to 50, 36 to 58.
+// R = 8 once there are enough of them that each of its loads is wanted: 24576 of 16..256 35 to 153, 38 to 160, 37 to
+// 175, of 1..40 24 to 62, 18 to 35, 20 to 45; 65536 of 16..256 67 to 367, 67 to 376, 66 to 318, of 1..40 41 to 129, 29
+// to 65, 28 to 71; 100000 of 16..256 98 to 526, 105 to 559, 104 to 477, of 1..40 54 to 195, 36 to 101, 34 to 102.
+// Closed intervals may end anywhere before their capacity, which tells nothing then, and R = 8 would read many
+// leaves for nothing: 4096 of 1..3 pairs 4 and 4 (R = 1, 8 lanes), of 1..40 5 to 7 and 5 to 14, of 16..256 7 to 32
+// and 14 to 76; 8192 of 1..40 8 to 12 and 5 to 16; 24576 of 1..40 20 to 27 and 9 to 24.
+constexpr uint32_t kOneMax = 4096, kOneMaxLong = 16384, kLongRange = 64, kGroupMax = 65536;
 constexpr int kWalk = 4;   // loads (8 leaves each) in flight per step, R = 1
 constexpr int kWalk8 = 3;  // the same, R = 8 (2 and 4 were slower, or even)
 
@@ -248,15 +251,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
   }
 }
 
-// Closed intervals of large calls: 8 lanes per interval, up to eight of its leaves on their way at a time
-// (LDS-direct loads, a group's 8 lanes bring a whole leaf), consumed in order until one key lies past the end.
+// 8 lanes per range or closed interval (HI), up to eight of its leaves on their way at a time (LDS-direct loads, a
+// group's 8 lanes bring a whole leaf), consumed in order until the length is reached or one key lies past the end.
 constexpr int kWalkInterval = 8;
-template <int F>
-__global__ __launch_bounds__(kThreads) void interval_kernel(TreeView tv, const uint64_t* __restrict__ start,
-                                                            const uint64_t* __restrict__ hi, uint32_t L, uint32_t n,
-                                                            uint64_t offset_stride, uint64_t* __restrict__ out_keys,
-                                                            uint64_t* __restrict__ out_vals,
-                                                            uint32_t* __restrict__ out_counts, uint64_t capacity) {
+template <int F, bool HI>
+__global__ __launch_bounds__(kThreads) void group_kernel(TreeView tv, const uint64_t* __restrict__ start,
+                                                         const uint64_t* __restrict__ hi,
+                                                         const uint32_t* __restrict__ len, uint32_t cap_const,
+                                                         uint32_t n, const uint64_t* __restrict__ offsets,
+                                                         uint64_t offset_stride, uint64_t* __restrict__ out_keys,
+                                                         uint64_t* __restrict__ out_vals,
+                                                         uint32_t* __restrict__ out_counts, uint64_t capacity) {
   constexpr int G = 8;
   constexpr uint32_t gpb = kThreads / G;
   typedef __attribute__((address_space(1))) void global_void_t;
@@ -269,8 +274,9 @@ __global__ __launch_bounds__(kThreads) void interval_kernel(TreeView tv, const u
   for (uint32_t rb = blockIdx.x * gpb; rb < n; rb += gridDim.x * gpb) {  // uniform across the block
     const uint32_t ri = rb + threadIdx.x / G;
     const bool valid = ri < n;
-    const uint64_t s = valid ? start[ri] : 0ull, h = valid ? hi[ri] : 0ull;
-    const uint64_t off = (uint64_t)ri * offset_stride;
+    const uint64_t s = valid ? start[ri] : 0ull, h = !HI ? KEY_MAX : valid ? hi[ri] : 0ull;
+    const uint32_t L = HI ? cap_const : valid ? len[ri] : 0u;
+    const uint64_t off = HI ? (uint64_t)ri * offset_stride : valid ? offsets[ri] : 0ull;
     uint32_t leaf = descend<F, G>(tv, 0, nullptr, s == KEY_MAX ? KEY_MAX - 1 : s, gl, gbase);
     uint32_t got = 0;
     bool done = !valid || L == 0 || s > h || s == KEY_MAX;
@@ -327,7 +333,7 @@ void launch_range_f(const TreeView& tv, const uint64_t* start, const uint64_t* h
                     uint64_t* out_keys, uint64_t* out_vals, uint32_t* out_counts, uint64_t capacity, hipStream_t s) {
   const size_t cus = (size_t)launch_cfg().num_cus;
   const size_t max_nb = cus * 8;
-  const uint32_t one = !hi ? kOneMax : cap_const < kLongInterval ? kOneMaxShort : kOneMaxLong;
+  const uint32_t one = !hi && capacity / n >= kLongRange ? kOneMaxLong : kOneMax;
   if (n <= one) {
     const size_t nb = std::min<size_t>((n + kWaves - 1) / kWaves, max_nb);
     if (scan)
@@ -336,10 +342,14 @@ void launch_range_f(const TreeView& tv, const uint64_t* start, const uint64_t* h
     else
       hipLaunchKernelGGL((range_kernel<F, 1, false>), dim3((unsigned)nb), dim3(kThreads), 0, s, tv, start, hi, len,
                          cap_const, n, offsets, offset_stride, out_keys, out_vals, out_counts, capacity);
-  } else if (hi) {
+  } else if (hi || n <= kGroupMax) {
     const size_t nb = std::min<size_t>((n + kWaves * 8 - 1) / (kWaves * 8), max_nb);
-    hipLaunchKernelGGL(interval_kernel<F>, dim3((unsigned)nb), dim3(kThreads), 0, s, tv, start, hi, cap_const, n,
-                       offset_stride, out_keys, out_vals, out_counts, capacity);
+    if (hi)
+      hipLaunchKernelGGL((group_kernel<F, true>), dim3((unsigned)nb), dim3(kThreads), 0, s, tv, start, hi, len, cap_const,
+                         n, offsets, offset_stride, out_keys, out_vals, out_counts, capacity);
+    else
+      hipLaunchKernelGGL((group_kernel<F, false>), dim3((unsigned)nb), dim3(kThreads), 0, s, tv, start, hi, len,
+                         cap_const, n, offsets, offset_stride, out_keys, out_vals, out_counts, capacity);
   } else {
     const size_t nb = std::min<size_t>((n + kWaves * 8 - 1) / (kWaves * 8), max_nb);
     hipLaunchKernelGGL((range_kernel<F, 8, false>), dim3((unsigned)nb), dim3(kThreads), 0, s, tv, start, hi, len,
