@@ -202,11 +202,14 @@ int resolve_search(const hm_tree* t, uint64_t n, const hm_search_opts* o, Search
   sl->queries_per_group = (o && o->queries_per_group) ? (int)o->queries_per_group : base.queries_per_group;
   // An unsorted batch that one round of resident blocks holds with one query per group takes one: nothing is
   // gained by more in flight, and a query's chain is shorter (kernel, 20011 queries on 2^25 keys: 4.4-5.2 us
-  // against 6.0-6.2 with four; 2^16: 6.2-6.4 against 7.0-7.2; 2^18, four rounds: 18.0-19.6 against 18.9).  Tuned
-  // trees and explicit shapes keep theirs.
-  if (!psa && !t->tuned && !(o && (o->group_size || o->queries_per_group || o->blocks_per_cu)) &&
-      n * (uint64_t)sl->group <= (uint64_t)launch_cfg().num_cus * (uint64_t)sl->blocks_per_cu * 256)
-    sl->queries_per_group = 1;
+  // against 6.0-6.2 with four; 2^16: 6.2-6.4 against 7.0-7.2; 2^18, four rounds: 18.0-19.6 against 18.9).  Staged
+  // levels above 40 KiB leave room for fewer blocks than blocks_per_cu (2^16 queries, fanout 32, 2^25 keys, three
+  // of four resident: 10.4 us against 7.6).  Tuned trees and explicit shapes keep theirs.
+  if (!psa && !t->tuned && !(o && (o->group_size || o->queries_per_group || o->blocks_per_cu))) {
+    const size_t lds = lds_bytes_for(t->view(), sl->lds_levels);
+    const uint64_t resident = std::min<uint64_t>(sl->blocks_per_cu, lds ? 160 * 1024 / lds : 64);
+    if (n * (uint64_t)sl->group <= (uint64_t)launch_cfg().num_cus * resident * 256) sl->queries_per_group = 1;
+  }
   if (sl->queries_per_group != 1 && sl->queries_per_group != 2 && sl->queries_per_group != 4)
     return set_err(HM_EINVAL, "queries_per_group %d not in {1,2,4}", sl->queries_per_group);
   int mode = (o && o->output_mode) ? (int)o->output_mode : base.output_mode;
