@@ -15,7 +15,7 @@ namespace {
 
 // Both reductions below end in atomics on one address, which the memory system serializes (~10 ns
 // each): every block reduces in LDS first and the grid is capped (kReduceBlocks), so a launch issues
-// at most a thousand of them (4096 blocks: 99 us for 4 million keys, now 15).
+// at most a thousand of them (the key summary over 4 million keys: 99 us with 4096 blocks, 12.9 with 512).
 constexpr int kReduceBlocks = 512;
 constexpr int kUnroll = 4;  // independent loads in flight per thread
 

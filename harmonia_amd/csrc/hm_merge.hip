@@ -392,7 +392,7 @@ __global__ __launch_bounds__(kTileThreads) void compact_last_kernel(const uint64
 // its leaves: sorted pair g goes to slot g % fill of leaf g / fill.  The values are read from the bucket's own
 // 40 KiB, which its block has just brought to L2.  4 million pairs: partition 45 us and this kernel 66 (132
 // with nine merges in place of the digit), where eight radix passes, the validation, the leaf fill and the
-// minima took 388; the build with one search of its keys went 656 -> 318 us.
+// minima took 388; the build with one search of its keys went 656 -> 312 us.
 constexpr int kBucketThreads = (int)kBucketSortMax / kPer;
 __global__ __launch_bounds__(kBucketThreads) void bucket_sort_fill_kernel(
     const uint64_t* __restrict__ keys, const uint64_t* __restrict__ vals, size_t n, int shift,

@@ -3,7 +3,7 @@
 //
 // Measured, 2^24 queries: histogram 33 us, scan 17, scatter 72, un-scatter 92, where the two 8-bit passes
 // took 58, 10, 132 and 159; 2^20 queries: 4.0, 4.7, 8.9 and 9.8 against 8.7, 8.5, 25 and 20.  The whole
-// search went 699 -> 564 us at 2^24 on 2^26 keys and 82 -> 46 us at 2^20 on 2^20.  What bounds it: memory at
+// search went 699 -> 565 us at 2^24 on 2^26 keys and 82 -> 48 us at 2^20 on 2^20.  What bounds it: memory at
 // the copy rate (the histogram reads 134 MB, the scatter moves 318 MB); the un-scatter's 2048 short runs per
 // tile (nine or ten bits instead of eleven: 81 and 96 us for then 120, but the search reads more leaves
 // twice, 455 and 423 us for 404; 1024 threads per tile: 124).  It gathered the found flags too, a second
