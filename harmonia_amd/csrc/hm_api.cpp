@@ -207,7 +207,7 @@ int resolve_search(const hm_tree* t, uint64_t n, const hm_search_opts* o, Search
   // levels above 40 KiB leave room for fewer blocks than blocks_per_cu (2^16 queries, fanout 32, 2^25 keys, three
   // of four resident: 10.4 us against 7.6).  Tuned trees and explicit shapes keep theirs.
   if (!psa && !t->tuned && !(o && (o->group_size || o->queries_per_group || o->blocks_per_cu))) {
-    const size_t lds = lds_bytes_for(t->view(), sl->lds_levels);
+    const size_t lds = sl->lds_levels > 0 ? (size_t)t->level_start[sl->lds_levels] * t->NS * 8 : 0;
     const uint64_t resident = std::min<uint64_t>(sl->blocks_per_cu, lds ? 160 * 1024 / lds : 64);
     if (n * (uint64_t)sl->group <= (uint64_t)launch_cfg().num_cus * resident * 256) sl->queries_per_group = 1;
   }
